@@ -801,7 +801,7 @@ struct GridBarrier {
   // the flat, two-level and XCD kinds honour it
   uint32_t poll_sleep;
 
-  __device__ void init(const ArenaView &arena, int kind, uint32_t ngroups, uint32_t nx) {
+  __device__ __forceinline__ void init(const ArenaView &arena, int kind, uint32_t ngroups, uint32_t nx) {
     a = arena;
     nwg = gridDim.x;
     wg = blockIdx.x;
@@ -827,7 +827,7 @@ struct GridBarrier {
   // the episode (it only publishes, e.g. a partial result, and then exits), so
   // the XCD barriers skip its L1/L2 invalidate; other kinds ignore the flag.
   template <int KIND>
-  __device__ int sync(bool acquire = true) {
+  __device__ __forceinline__ int sync(bool acquire = true) {
     __shared__ int rc_sh;
     ++e;
     if constexpr (KIND == 6 /*HS_BAR_COOP*/) {

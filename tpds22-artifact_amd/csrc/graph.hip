@@ -1016,94 +1016,625 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 }
 
 // ===========================================================================
+// Rounds by a team: high-diameter graphs (meshes, roads) run thousands of rounds
+// of a few thousand vertices each, and such a round costs one grid barrier (5-7
+// us, most of it words bouncing between the XCDs' L2s) and a chain of loads that
+// miss an L2 the barrier's acquire has just emptied.  While the rounds are small
+// they are run by the workgroups b with b % nxcd == 0 alone, which dispatch puts
+// on one XCD: there an atomic or a coherent load of the device takes 0.12 us (a
+// miss 0.5 us).  What bounds a round is that chain, so it is kept short:
+//  - every workgroup appends to an output segment of its own, counted in LDS (an
+//    atomic on one queue counter serializes for ~11 ns and is waited for), and a
+//    segment entry carries the vertex's first edge, so its edges, key and end are
+//    loaded together;
+//  - the team's barrier is one word per workgroup, its episode and its segment's
+//    count, which every workgroup reads with one load, so that the barrier also
+//    says what the next round's input is;
+//  - on meshes (degree <= 4) four lanes share a vertex: one edge per lane and a
+//    single pass of short code.
+// Correctness does not depend on the placement: everything the rounds write is
+// written and read with agent-scope operations, and every wave's stores have
+// completed before its workgroup arrives.  The other workgroups wait in the grid
+// barrier meanwhile; a stretch is at most kTeamRounds rounds, so that wait stays
+// short.
+constexpr int kTeamWg = 1024;               // threads per workgroup of the kernels that run team rounds
+constexpr uint32_t kTeamMax = 32;           // workgroups of a team
+constexpr uint32_t kTeamRounds = 256;
+constexpr uint64_t kTeamEdges = 1ull << 17;  // edges of a round up to which the team runs it
+constexpr uint32_t kTeamIdleSleep = 32;     // s_sleep units between the idle workgroups' polls
+constexpr uint32_t kSegCap = 2048;          // entries of a workgroup's output segment; the rest goes to the queue
+constexpr uint32_t kSegBlock = 16;          // entries a wave takes at once: 4 lanes each
+
+__device__ __forceinline__ void st_u64(uint64_t *p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Who works on a round: wave `wave` of `waves`, the waves of a workgroup far apart
+// so that a small round is spread over the compute units.
+struct Crew {
+  uint32_t wave, waves;
+  __device__ Crew(uint32_t rank, uint32_t size) {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * size + rank;
+    waves = size * (kTeamWg / 64);
+  }
+};
+
+// The segments' share of a round's input: lane l holds segment l's entries and the
+// blocks of segments 0..l; the same in every wave.
+struct Segments {
+  uint32_t cnt, upto, blocks, total;
+  bool queued;  // some workgroup also appended to the queues
+
+  __device__ void none() { cnt = upto = blocks = total = 0; queued = true; }
+  // word: lane l's segment count, bit 31 = "appended to the queues"
+  __device__ __forceinline__ void take(uint32_t word) {
+    queued = ballot(word >> 31) != 0;
+    cnt = word & 0x7FFFFFFFu;
+    upto = wave_incl_scan((cnt + kSegBlock - 1) / kSegBlock);
+    blocks = __builtin_amdgcn_readlane(upto, 63);
+    total = wave_sum(cnt);
+  }
+  // entry index (of all segments, kSegCap apart) of this lane in block b, or ~0
+  __device__ __forceinline__ uint32_t entry(uint32_t b) const {
+    const uint32_t s = (uint32_t)__builtin_popcountll(ballot(upto <= b));
+    const uint32_t n = __builtin_amdgcn_readlane(cnt, s);
+    const uint32_t first = __builtin_amdgcn_readlane(upto, s) - (n + kSegBlock - 1) / kSegBlock;
+    const uint32_t i = (b - first) * kSegBlock + (lane_id() >> 2);
+    return i < n ? s * kSegCap + i : 0xFFFFFFFFu;
+  }
+};
+
+struct Team {
+  uint64_t *word;       // [2][kTeamMax] episode << 32 | segment word, zero before the first grid barrier
+  uint32_t size, rank;  // rank: position in the team (workgroups outside it: any value)
+  bool in, usable;
+  uint32_t episode;
+
+  __device__ void init(uint64_t *w, uint32_t nxcd) {
+    const uint32_t x = nxcd < gridDim.x ? nxcd : gridDim.x;
+    word = w;
+    size = (gridDim.x + x - 1) / x;
+    rank = blockIdx.x / x;
+    in = blockIdx.x % x == 0;
+    usable = size < gridDim.x && size <= kTeamMax;
+    episode = 0;
+  }
+  // Barrier of the team; `mine` (thread 0): this workgroup's segment word, `seg`:
+  // everyone's.  Words alternate by parity: a workgroup writes the same word again
+  // two episodes on, when all have read it.  A status uniform across the workgroup.
+  __device__ __forceinline__ int sync(const ArenaView &a, uint32_t mine, Segments &seg) {
+    __shared__ int rc_sh;
+    __shared__ uint32_t seg_sh[64];
+    ++episode;
+    wait_stores();
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      uint64_t *w = word + (episode & 1) * kTeamMax;
+      const uint32_t want = episode, lane = lane_id();
+      // an exchange: it reaches the readers in 0.22 us, a store in 0.32
+      if (lane == 0)
+        (void)__hip_atomic_exchange(w + rank, ((uint64_t)want << 32) | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      uint64_t got = 0;
+      const int rc = spin_until(a, [&] {
+        got = lane < size ? ld_u64(w + lane) : (uint64_t)want << 32;
+        return ballot((uint32_t)(got >> 32) != want) == 0;
+      }, 1);
+      seg_sh[lane] = (uint32_t)got;
+      if (lane == 0) rc_sh = rc;
+    }
+    __syncthreads();
+    seg.take(seg_sh[lane_id()]);
+    return rc_sh;
+  }
+};
+
+// hs_worklist.hpp's wave_push_batch and wave_push_chunks_batch for readers that no
+// acquire precedes: agent-scope stores.
+template <int B>
+__device__ __forceinline__ void team_push(uint32_t *q, uint32_t *cnt, const bool (&want)[B], const uint32_t (&v)[B]) {
+  uint64_t mask[B];
+  uint32_t total = 0;
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    mask[x] = ballot(want[x]);
+    total += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+  if (total == 0) return;
+  uint32_t base = 0;
+  if (lane_id() == 0) base = add_relaxed(cnt, total);
+  base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    if (mask[x] >> lane_id() & 1) st_relaxed(q + base + lanes_below(mask[x]), v[x]);
+    base += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+}
+
+template <int B>
+__device__ __forceinline__ bool team_push_chunks(uint64_t *hq, uint32_t *hcnt, const uint32_t (&nc)[B],
+                                                 const uint32_t (&v)[B]) {
+  uint32_t ncl = 0;
+#pragma unroll
+  for (int x = 0; x < B; ++x) ncl += nc[x];
+  if (!ballot(ncl != 0)) return false;
+  const uint32_t incl = wave_incl_scan(ncl);
+  const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+  uint32_t base = 0;
+  if (lane_id() == 63) base = add_relaxed(hcnt, total);
+  base = __builtin_amdgcn_readlane(base, 63) + incl - ncl;
+#pragma unroll
+  for (int x = 0; x < B; ++x)
+    for (uint32_t c = 0; c < nc[x]; ++c) st_u64(hq + base++, v[x] | ((uint64_t)c << 32));
+  return true;
+}
+
+// A wave's appends to one queue, staged in LDS: every atomic on a queue's counter
+// serializes for ~11 ns over the whole device, and with one per batch of 256 edges
+// those atomics were most of a large round (R-MAT 22, one source: 7.7 -> 2.9 ms).
+// The count is the same in every lane.
+template <class T, uint32_t CAP>
+struct WaveList {
+  T *buf;         // [CAP] LDS of this wave
+  uint32_t n;
+  T *q;           // the queue and its counter
+  uint32_t *cnt;
+
+  __device__ __forceinline__ void flush() {
+    if (n == 0) return;
+    uint32_t base = 0;
+    if (lane_id() == 0) base = add_relaxed(cnt, n);
+    base = __builtin_amdgcn_readfirstlane(base);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (uint32_t i = lane_id(); i < n; i += 64) put(q + base + i, buf[i]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    n = 0;
+  }
+  // room for `total` more entries, in LDS (returns true) or not at all
+  __device__ __forceinline__ bool room(uint32_t total) {
+    if (n + total > CAP) flush();
+    return total <= CAP;
+  }
+  static __device__ __forceinline__ void put(uint32_t *p, uint32_t v) { st_relaxed(p, v); }
+  static __device__ __forceinline__ void put(uint64_t *p, uint64_t v) { st_u64(p, v); }
+};
+
+constexpr uint32_t kWaveNear = 512, kWaveFar = 256, kWaveChunks = 128;
+struct WaveBuffers {
+  uint64_t chunks[kTeamWg / 64][kWaveChunks];
+  uint32_t near[kTeamWg / 64][kWaveNear];
+  uint32_t far[kTeamWg / 64][kWaveFar];
+};
+
+template <int B, uint32_t CAP>
+__device__ __forceinline__ void wave_list_push(WaveList<uint32_t, CAP> &l, const bool (&want)[B], const uint32_t (&v)[B]) {
+  static_assert(B * 64 <= CAP, "a batch fits");
+  uint64_t mask[B];
+  uint32_t total = 0;
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    mask[x] = ballot(want[x]);
+    total += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+  if (total == 0) return;
+  l.room(total);
+  uint32_t at = l.n;
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    if (mask[x] >> lane_id() & 1) l.buf[at + lanes_below(mask[x])] = v[x];
+    at += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+  l.n = at;
+}
+
+// chunk entries v | c << 32 (c < nc[x])
+template <int B, uint32_t CAP>
+__device__ __forceinline__ void wave_list_push_chunks(WaveList<uint64_t, CAP> &l, const uint32_t (&nc)[B],
+                                                      const uint32_t (&v)[B]) {
+  uint32_t ncl = 0;
+#pragma unroll
+  for (int x = 0; x < B; ++x) ncl += nc[x];
+  if (!ballot(ncl != 0)) return;
+  const uint32_t incl = wave_incl_scan(ncl);
+  const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+  if (l.room(total)) {
+    uint32_t at = l.n + incl - ncl;
+#pragma unroll
+    for (int x = 0; x < B; ++x)
+      for (uint32_t c = 0; c < nc[x]; ++c) l.buf[at++] = v[x] | ((uint64_t)c << 32);
+    l.n += total;
+  } else {
+    team_push_chunks<B>(l.q, l.cnt, nc, v);
+  }
+}
+
+// A workgroup's outputs of a team round: its segment's count, whether it appended
+// to the queues, and a list kept in LDS until it is asked for (the SSSP far list).
+constexpr uint32_t kStage = 4096;
+struct Output {
+  uint32_t cnt[2], queued[2];  // by round parity
+  uint32_t kept, fill;         // slots handed out of `keep`, end of the filled ones
+  uint32_t keep[kStage];
+
+  __device__ void clear(uint32_t par) { cnt[par] = queued[par] = 0; }  // one thread
+  __device__ uint32_t segment_word(uint32_t par) const {
+    return min(cnt[par], kSegCap) | (queued[par] ? 0x80000000u : 0u);
+  }
+};
+
+// Appends vertices (with their first edges) to the workgroup's segment, those
+// that do not fit to the queue.
+template <int B>
+__device__ __forceinline__ void segment_push(Output &out, uint32_t par, uint64_t *seg, uint32_t *q, uint32_t *cnt,
+                                             const bool (&want)[B], const uint32_t (&v)[B], const uint32_t (&eb)[B]) {
+  uint64_t mask[B];
+  uint32_t total = 0;
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    mask[x] = ballot(want[x]);
+    total += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+  if (total == 0) return;
+  uint32_t base = 0;
+  if (lane_id() == 0) base = atomicAdd(&out.cnt[par], total);
+  base = __builtin_amdgcn_readfirstlane(base);
+  const bool over = base + total > kSegCap;
+  bool rest[B];
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    const uint32_t at = base + lanes_below(mask[x]);
+    const bool mine = mask[x] >> lane_id() & 1;
+    if (mine && at < kSegCap) st_u64(seg + at, v[x] | ((uint64_t)eb[x] << 32));
+    rest[x] = mine && at >= kSegCap;
+    base += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+  if (over) {
+    team_push<B>(q, cnt, rest, v);
+    if (lane_id() == 0) out.queued[par] = 1;
+  }
+}
+
+// Appends to the kept list, what does not fit to its queue.
+template <int B>
+__device__ __forceinline__ void kept_push(Output &out, uint32_t *q, uint32_t *cnt, const bool (&want)[B],
+                                          const uint32_t (&v)[B]) {
+  uint64_t mask[B];
+  uint32_t total = 0;
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    mask[x] = ballot(want[x]);
+    total += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+  if (total == 0) return;
+  uint32_t base = 0;
+  if (lane_id() == 0) {
+    base = atomicAdd(&out.kept, total);
+    if (base + total <= kStage) atomicMax(&out.fill, base + total);  // slots in order: those that fit form a prefix
+  }
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (base + total > kStage) {
+    team_push<B>(q, cnt, want, v);
+    return;
+  }
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    if (mask[x] >> lane_id() & 1) out.keep[base + lanes_below(mask[x])] = v[x];
+    base += (uint32_t)__builtin_popcountll(mask[x]);
+  }
+}
+
+// Moves the kept list to its queue (every thread of the workgroup calls it).
+__device__ __forceinline__ void kept_flush(Output &out, uint32_t *q, uint32_t *cnt) {
+  __shared__ uint32_t base_sh;
+  __syncthreads();
+  const uint32_t n = out.fill;
+  if (threadIdx.x == 0) base_sh = n ? add_relaxed(cnt, n) : 0u;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < n; i += kTeamWg) st_relaxed(q + base_sh + i, out.keep[i]);
+  __syncthreads();
+  if (threadIdx.x == 0) out.kept = out.fill = 0;
+  __syncthreads();
+}
+
+// Vertices a wave takes at once from a queue of nin: 64, fewer (at least 8) while
+// that still gives no wave a second share
+__device__ __forceinline__ uint32_t queue_share(uint32_t nin, uint32_t waves) {
+  uint32_t s = 64;
+  while (s > 8 && (uint64_t)nin * 2 <= (uint64_t)waves * s) s >>= 1;
+  return s;
+}
+
+// ===========================================================================
 // SSSP, near/far buckets (LONESTAR/apps/sssp/kernel_gsrb.cu:459-687).
 struct SsspArgs {
-  uint32_t n;
+  uint32_t n, m;
   const uint32_t *row, *col, *w;
   int32_t src, delta;
-  int32_t *dist;
+  int32_t *dist;     // output
+  uint64_t *key;     // [n] distance (sign flipped: order of unsigned) << 32 | stamp of its last change
   uint32_t *nq;      // [2][n] near queues (light vertices)
   uint64_t *hq;      // [2][hcap] near chunk lists (heavy vertices, chunks of kBfsChunk edges)
   uint64_t hcap;
   uint32_t *fq;      // [3][n] far lists
-  uint32_t *nstamp;  // [n] round stamp of the near list holding v
-  uint32_t *fstamp;  // [n] epoch stamp of the far list holding v
-  uint32_t *ctr;     // near counts [3] (0..2), steal [3] (3..5), far counts [3] (6..8),
-                     // near chunk counts [3] (9..11)
+  uint64_t *seg;     // [2][kTeamMax][kSegCap] near segments of a team: v | first edge << 32
+  uint32_t *ctr;     // near counts [3] (0..2), grab [3] (3..5), far counts [3] (6..8),
+                     // near chunk counts [3] (9..11), the state a team stretch ends in (12),
+                     // the team's words (13..14)
   uint32_t *stats;
+  uint32_t mean_degree;  // rounded up, for the size of a round
   uint32_t ng, nx;
 };
+constexpr int kSsCounters = 15;
+static_assert(2 * kTeamMax * sizeof(uint64_t) <= 2 * kCtr * sizeof(uint32_t), "the team's words fit slots 13 and 14");
 
 constexpr int kSsBatch = 4;
 
-// Entries of the next near input: light vertices to the queue, heavy ones as
-// chunks to the chunk list (every wave of the grid shares them next round).
-__device__ __forceinline__ void sssp_push_near(const SsspArgs &p, const bool (&near)[kSsBatch],
-                                               const uint32_t (&v)[kSsBatch], uint32_t *qnear,
-                                               uint32_t *cnear, uint64_t *hnear, uint32_t *hcnear) {
-  uint32_t nc[kSsBatch];
-#pragma unroll
-  for (int x = 0; x < kSsBatch; ++x) nc[x] = near[x] ? bfs_chunks(p.row[v[x] + 1] - p.row[v[x]]) : 0u;
-  bool light[kSsBatch];
-#pragma unroll
-  for (int x = 0; x < kSsBatch; ++x) light[x] = near[x] && nc[x] == 0;
-  wave_push_batch<kSsBatch>(qnear, cnear, light, v);
-  wave_push_chunks_batch<kSsBatch>(hnear, hcnear, nc, v);
+__device__ __forceinline__ uint64_t ss_key(int32_t d, uint32_t stamp) {
+  return ((uint64_t)((uint32_t)d ^ 0x80000000u) << 32) | stamp;
+}
+__device__ __forceinline__ int32_t ss_dist(uint64_t key) { return (int32_t)((uint32_t)(key >> 32) ^ 0x80000000u); }
+
+// where a round stands: r counts rounds and bucket steps; stamp r + 1 marks the
+// changes made in it.  far_since: stamps of the changes since the bucket was opened.
+struct SsState {
+  uint32_t r, epoch, relax, far_since;
+};
+
+// the input of a step
+struct SsInput {
+  Segments seg;
+  uint32_t nin, nh, nfar;
+  __device__ bool near() const { return (seg.total | nin | nh) != 0; }
+};
+
+__device__ __forceinline__ int32_t ss_bound(const SsspArgs &p, uint32_t epoch) {
+  return (int32_t)min((int64_t)(epoch + 1) * p.delta, (int64_t)kInf - 1);
+}
+__device__ __forceinline__ uint32_t *ss_near_q(const SsspArgs &p, uint32_t r) { return p.nq + (size_t)(r & 1) * p.n; }
+__device__ __forceinline__ uint32_t *ss_near_cnt(const SsspArgs &p, uint32_t r) { return p.ctr + (r % 3) * kCtr; }
+__device__ __forceinline__ uint32_t *ss_heavy_cnt(const SsspArgs &p, uint32_t r) { return p.ctr + (9 + r % 3) * kCtr; }
+__device__ __forceinline__ uint32_t *ss_far_q(const SsspArgs &p, uint32_t e) { return p.fq + (size_t)(e % 3) * p.n; }
+__device__ __forceinline__ uint32_t *ss_far_cnt(const SsspArgs &p, uint32_t e) { return p.ctr + (6 + e % 3) * kCtr; }
+__device__ __forceinline__ uint64_t *ss_seg(const SsspArgs &p, uint32_t r, uint32_t rank) {
+  return p.seg + ((size_t)(r & 1) * kTeamMax + rank) * kSegCap;
 }
 
-// relaxation (kernel_gsrb.cu:415): atomicMin(dist[dst], dist[n] + w); the
-// improved vertex joins the near list when within the current bucket bound,
-// else the far list; the stamps keep each list free of duplicates.  A batch of
-// kSsBatch candidates per lane (v == ~0 for none): their loads and atomics are
-// each in flight together.
-__device__ __forceinline__ void sssp_relax_batch(const SsspArgs &p, const uint32_t (&v)[kSsBatch],
-                                                 const int32_t (&nd)[kSsBatch], int32_t bound,
-                                                 uint32_t round_stamp, uint32_t *qnear, uint32_t *cnear,
-                                                 uint64_t *hnear, uint32_t *hcnear, uint32_t epoch_stamp,
-                                                 uint32_t *qfar, uint32_t *cfar) {
-  int32_t cur[kSsBatch];
+// Entries of the next near input (light vertices, heavy ones as chunks that every
+// wave shares) and of the far list of bucket `epoch`; out: a team's, else null.
+// What a wave needs of its surroundings in a step
+struct SsStep {
+  const SsspArgs &p;
+  SsState st;
+  int32_t bound;
+  uint32_t far_epoch;  // bucket whose far list is appended to
+  Output *out;         // of a team, else null, and the wave's lists instead
+  uint32_t rank;
+  WaveList<uint32_t, kWaveNear> near;
+  WaveList<uint32_t, kWaveFar> far;
+  WaveList<uint64_t, kWaveChunks> chunks;
+};
+
+template <bool TEAM, int B>
+__device__ __forceinline__ void sssp_push(SsStep &s, const bool (&near)[B], const bool (&far)[B], const uint32_t (&v)[B],
+                                          const uint32_t (&eb)[B], const uint32_t (&deg)[B]) {
+  const SsspArgs &p = s.p;
+  const uint32_t r = s.st.r;
+  uint32_t nc[B];
+  bool light[B];
 #pragma unroll
-  for (int x = 0; x < kSsBatch; ++x) cur[x] = v[x] != 0xFFFFFFFFu ? ld_i32(p.dist + v[x]) : 0;
-  bool better[kSsBatch];
-#pragma unroll
-  for (int x = 0; x < kSsBatch; ++x) {
-    better[x] = false;
-    if (v[x] != 0xFFFFFFFFu && nd[x] < cur[x]) {
-      const int32_t old = __hip_atomic_fetch_min(p.dist + v[x], nd[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      better[x] = nd[x] < old;
-    }
+  for (int x = 0; x < B; ++x) {
+    nc[x] = near[x] ? bfs_chunks(deg[x]) : 0u;
+    light[x] = near[x] && nc[x] == 0;
   }
-  bool near[kSsBatch], far[kSsBatch];
+  if constexpr (TEAM) {
+    segment_push<B>(*s.out, r & 1, ss_seg(p, r + 1, s.rank), ss_near_q(p, r + 1), ss_near_cnt(p, r + 1), light, v, eb);
+    kept_push<B>(*s.out, ss_far_q(p, s.far_epoch), ss_far_cnt(p, s.far_epoch), far, v);
+    if (team_push_chunks<B>(p.hq + (size_t)((r + 1) & 1) * p.hcap, ss_heavy_cnt(p, r + 1), nc, v) && lane_id() == 0)
+      s.out->queued[r & 1] = 1;
+  } else {
+    wave_list_push<B>(s.near, light, v);
+    wave_list_push<B>(s.far, far, v);
+    wave_list_push_chunks<B>(s.chunks, nc, v);
+  }
+}
+
+// Relaxation (kernel_gsrb.cu:415) of B candidates per lane (v == ~0 for none),
+// their loads and atomics each in flight together.  One 64-bit atomic minimum on
+// (distance, stamp of the change) does the update and says whether the vertex is
+// in the list already: it joins the near list when within the bucket bound, unless
+// an earlier change of this round put it there (stamp r + 1 and within the bound),
+// else the far list, unless a change since the bucket was opened did (beyond the
+// bound).  A later stamp never lowers a key of equal distance.  Where the atomics
+// would contend the present distance is looked at first; the one-edge-per-lane
+// rounds of a team do not (each step of their chain of loads is 0.4-0.9 us: 16.2
+// -> 11.4 ms on a mesh of 1.1M vertices), and a team loads the degree beside the
+// atomic.
+template <bool TEAM, int B>
+__device__ __forceinline__ void sssp_relax_batch(SsStep &s, const uint32_t (&v)[B], const int32_t (&nd)[B]) {
+  constexpr bool kBlind = TEAM && B == 1;
+  const SsspArgs &p = s.p;
+  const uint32_t stamp = s.st.r + 1;
+  uint32_t eb[B], deg[B];
+  bool better[B];
+  uint64_t old[B];
+  int32_t cur[B];
 #pragma unroll
-  for (int x = 0; x < kSsBatch; ++x) {
-    near[x] = far[x] = false;
+  for (int x = 0; x < B; ++x) {
+    cur[x] = kInf;
+    if (!kBlind && v[x] != 0xFFFFFFFFu) cur[x] = ss_dist(ld_u64(p.key + v[x]));
+  }
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    better[x] = v[x] != 0xFFFFFFFFu && (kBlind || nd[x] < cur[x]);
+    old[x] = 0;
+    eb[x] = deg[x] = 0;
     if (better[x]) {
-      if (nd[x] <= bound)
-        near[x] = __hip_atomic_exchange(p.nstamp + v[x], round_stamp, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT) != round_stamp;
-      else
-        far[x] = __hip_atomic_exchange(p.fstamp + v[x], epoch_stamp, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT) != epoch_stamp;
+      old[x] = __hip_atomic_fetch_min(p.key + v[x], ss_key(nd[x], stamp), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (TEAM) { eb[x] = p.row[v[x]]; deg[x] = p.row[v[x] + 1] - eb[x]; }
     }
   }
-  sssp_push_near(p, near, v, qnear, cnear, hnear, hcnear);
-  wave_push_batch<kSsBatch>(qfar, cfar, far, v);
+  bool near[B], far[B];
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    const int32_t od = ss_dist(old[x]);
+    const uint32_t os = (uint32_t)old[x];
+    better[x] = better[x] && nd[x] < od;
+    near[x] = better[x] && nd[x] <= s.bound && !(od <= s.bound && os == stamp);
+    far[x] = better[x] && nd[x] > s.bound && (od == kInf || os < s.st.far_since);
+    if (!TEAM) deg[x] = near[x] ? p.row[v[x] + 1] - p.row[v[x]] : 0u;
+  }
+  sssp_push<TEAM, B>(s, near, far, v, eb, deg);
 }
 
-// Edge destinations and weights are read with streaming loads: each edge is
-// read once per relaxation of its vertex, and cached they evict distances and
-// stamps (R-MAT 22: 8.5 -> 8.0 ms per source; the same change slowed the
-// 64-source SSSP by 2% and left BFS and PageRank unchanged, so only here).
+// Edge destinations and weights are read with streaming loads in the rounds of
+// the whole grid: each edge is read once per relaxation of its vertex, and cached
+// they evict distances (R-MAT 22: 8.5 -> 8.0 ms per source; the same change slowed
+// the 64-source SSSP by 2% and left BFS and PageRank unchanged, so only here).
+template <bool TEAM>
+__device__ __forceinline__ uint32_t ss_edge(const uint32_t *q) {
+  return TEAM ? *q : __builtin_nontemporal_load(q);
+}
+
+// the edges of up to 64 vertices, one per lane (edges [eb, eb + deg), distance du)
+template <bool TEAM>
+__device__ __forceinline__ void sssp_expand(SsStep &s, uint32_t eb, uint32_t deg, int32_t du) {
+  wave_expand<kSsBatch>(eb, deg, [&](const uint32_t (&e)[kSsBatch], const bool (&ev)[kSsBatch],
+                                     const uint32_t (&own)[kSsBatch]) {
+    uint32_t vb[kSsBatch];
+    int32_t nd[kSsBatch];
+#pragma unroll
+    for (int x = 0; x < kSsBatch; ++x) {
+      const int32_t odu = __shfl(du, (int)own[x]);
+      vb[x] = ev[x] ? ss_edge<TEAM>(s.p.col + e[x]) : 0xFFFFFFFFu;
+      nd[x] = ev[x] ? odu + (int32_t)ss_edge<TEAM>(s.p.w + e[x]) : 0;
+    }
+    sssp_relax_batch<TEAM, kSsBatch>(s, vb, nd);
+  });
+}
+
+// One round, or with an empty near input one bucket step, by the given crew.
+// `first`: the thread that clears the counters.
+template <bool TEAM>
+__device__ __forceinline__ void sssp_step(const SsspArgs &p, SsState &st, const SsInput &in, const Crew &crew, bool first,
+                                          Output *out, uint32_t rank, WaveBuffers *wb) {
+  const uint32_t r = st.r, lane = lane_id();
+  if (TEAM && threadIdx.x == 0) out->clear((r + 1) & 1);
+  if (first) {  // counters last used two rounds ago
+    st_relaxed(ss_near_cnt(p, r + 2), 0u);
+    st_relaxed(ss_heavy_cnt(p, r + 2), 0u);
+    st_relaxed(p.ctr + (3 + (r + 1) % 3) * kCtr, 0u);
+  }
+  const uint32_t far_epoch = in.near() ? st.epoch : st.epoch + 1;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  SsStep s{p, st, ss_bound(p, st.epoch), far_epoch, out, rank,
+           {TEAM ? nullptr : wb->near[wv], 0, ss_near_q(p, r + 1), ss_near_cnt(p, r + 1)},
+           {TEAM ? nullptr : wb->far[wv], 0, ss_far_q(p, far_epoch), ss_far_cnt(p, far_epoch)},
+           {TEAM ? nullptr : wb->chunks[wv], 0, p.hq + (size_t)((r + 1) & 1) * p.hcap, ss_heavy_cnt(p, r + 1)}};
+  if (in.near()) {
+    // segments of a team's round
+    for (uint32_t b = crew.wave; b < in.seg.blocks; b += crew.waves) {
+      const uint32_t i = in.seg.entry(b), x = lane & 3;
+      const uint64_t ent = i != 0xFFFFFFFFu ? ld_u64(ss_seg(p, r, 0) + i) : 0ull;
+      const uint32_t u = (uint32_t)ent, eb = (uint32_t)(ent >> 32);
+      uint32_t end = eb, c = 0, w = 0;
+      int32_t du = 0;
+      if (i != 0xFFFFFFFFu) {
+        end = p.row[u + 1];
+        du = ss_dist(ld_u64(p.key + u));
+        if (eb + x < p.m) { c = p.col[eb + x]; w = p.w[eb + x]; }
+      }
+      const uint32_t deg = end - eb;
+      if (TEAM && !ballot(deg > 4)) {
+        const uint32_t vb[1] = {x < deg ? c : 0xFFFFFFFFu};
+        const int32_t nd[1] = {du + (int32_t)w};
+        sssp_relax_batch<TEAM, 1>(s, vb, nd);
+      } else {
+        sssp_expand<TEAM>(s, eb, x == 0 ? deg : 0u, du);
+      }
+    }
+    // heavy chunks of the near input, spread over the crew
+    const uint64_t *hin = p.hq + (size_t)(r & 1) * p.hcap;
+    for (uint32_t i = crew.wave; i < in.nh; i += crew.waves) {
+      const uint64_t ent = ld_u64(hin + i);
+      const uint32_t u = (uint32_t)ent, c = (uint32_t)(ent >> 32);
+      const uint32_t eb = p.row[u] + c * kBfsChunk, ee = min(p.row[u + 1], eb + kBfsChunk);
+      const int32_t du = ss_dist(ld_u64(p.key + u));
+      for (uint32_t e0 = eb; e0 < ee; e0 += kSsBatch * 64) {
+        uint32_t vb[kSsBatch];
+        int32_t nd[kSsBatch];
+#pragma unroll
+        for (int x = 0; x < kSsBatch; ++x) {
+          const uint32_t e = e0 + 64 * x + lane;
+          vb[x] = e < ee ? ss_edge<TEAM>(p.col + e) : 0xFFFFFFFFu;
+          nd[x] = e < ee ? du + (int32_t)ss_edge<TEAM>(p.w + e) : 0;
+        }
+        sssp_relax_batch<TEAM, kSsBatch>(s, vb, nd);
+      }
+    }
+    // light near queue: the first share of each wave is dealt, further ones are
+    // taken from the round's grab counter
+    const uint32_t *qin = ss_near_q(p, r);
+    uint32_t *grab = p.ctr + (3 + r % 3) * kCtr;
+    const uint32_t share = queue_share(in.nin, crew.waves);
+    for (uint32_t b = crew.wave; (uint64_t)b * share < in.nin;) {
+      const uint32_t i = b * share + lane;
+      const bool valid = lane < share && i < in.nin;
+      const uint32_t u = valid ? ld_relaxed(qin + i) : 0u;
+      uint32_t eb = 0, deg = 0;
+      int32_t du = 0;
+      if (valid) { eb = p.row[u]; deg = p.row[u + 1] - eb; du = ss_dist(ld_u64(p.key + u)); }
+      sssp_expand<TEAM>(s, eb, deg, du);
+      if ((uint64_t)crew.waves * share >= in.nin) break;
+      uint32_t g = 0;
+      if (lane == 0) g = add_relaxed(grab, 1u);
+      b = crew.waves + __builtin_amdgcn_readfirstlane(g);
+    }
+    ++st.relax;
+  } else {
+    // near input empty: advance the bucket and split the far list
+    // (remove_dups_dev + curdelta += DELTA, kernel_gsrb.cu:310-348,669-677).
+    // Entries that a shorter path brought below the old bound are done already.
+    const uint32_t *fin = ss_far_q(p, st.epoch);
+    if (first) st_relaxed(ss_far_cnt(p, st.epoch + 2), 0u);
+    const int32_t nbound = ss_bound(p, st.epoch + 1);
+    for (uint64_t b = (uint64_t)crew.wave * 64; b < in.nfar; b += (uint64_t)crew.waves * 64) {
+      const uint64_t i = b + lane;
+      uint32_t v[1] = {0}, eb[1] = {0}, deg[1] = {0};
+      bool to_near[1] = {false}, to_far[1] = {false};
+      if (i < in.nfar) {
+        v[0] = ld_relaxed(fin + i);
+        const int32_t d = ss_dist(ld_u64(p.key + v[0]));
+        to_near[0] = d > s.bound && d <= nbound;
+        to_far[0] = d > nbound;
+        if (to_near[0]) { eb[0] = p.row[v[0]]; deg[0] = p.row[v[0] + 1] - eb[0]; }
+        if (to_far[0]) st_u64(p.key + v[0], ss_key(d, r + 1));  // in the new bucket's far list
+      }
+      sssp_push<TEAM, 1>(s, to_near, to_far, v, eb, deg);
+    }
+    ++st.epoch;
+    st.far_since = r + 1;
+  }
+  if (!TEAM) {
+    s.near.flush();
+    s.far.flush();
+    s.chunks.flush();
+  }
+  ++st.r;
+}
+
 template <int KIND>
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k_sssp(ArenaView a, SsspArgs p) {
+__global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4))) k_sssp(ArenaView a, SsspArgs p) {
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
-  for (uint32_t v = gtid(); v < p.n; v += gthreads()) {
-    p.dist[v] = (v == (uint32_t)p.src) ? 0 : kInf;
-    p.nstamp[v] = 0;
-    p.fstamp[v] = 0;
-  }
-  if (gtid() == 0) {
+  Team team;
+  team.init(reinterpret_cast<uint64_t *>(p.ctr + 13 * kCtr), p.nx);
+  uint32_t *ctl = p.ctr + 12 * kCtr;
+  __shared__ Output out;
+  __shared__ WaveBuffers wb;
+  const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
+  for (uint64_t v = t0; v < p.n; v += nt) p.key[v] = ss_key(v == (uint32_t)p.src ? 0 : kInf, 0);
+  if (threadIdx.x == 0) { out.clear(0); out.clear(1); out.kept = out.fill = 0; }
+  if (t0 < 2 * kTeamMax) team.word[t0] = 0;
+  if (t0 == 0) {
     for (int i = 0; i < 12; ++i) p.ctr[i * kCtr] = 0;
     const uint32_t nc = bfs_chunks(p.row[p.src + 1] - p.row[p.src]);
     if (nc) {
@@ -1115,108 +1646,69 @@ __global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k
     }
   }
   if (gb.sync<KIND>()) return;
-  __shared__ uint32_t s_base;
-  uint32_t r = 0, epoch = 0, relax_rounds = 0;
-  for (;; ++r) {
-    const uint32_t nin = ld_relaxed(p.ctr + (r % 3) * kCtr);
-    const uint32_t nh = ld_relaxed(p.ctr + (9 + r % 3) * kCtr);
-    uint32_t *qnear = p.nq + (size_t)((r + 1) & 1) * p.n;
-    uint32_t *cnear = p.ctr + ((r + 1) % 3) * kCtr;
-    uint64_t *hnear = p.hq + (size_t)((r + 1) & 1) * p.hcap;
-    uint32_t *hcnear = p.ctr + (9 + (r + 1) % 3) * kCtr;
-    if (gtid() == 0) {  // counters last used two rounds ago
-      st_relaxed(p.ctr + ((r + 2) % 3) * kCtr, 0u);
-      st_relaxed(p.ctr + (9 + (r + 2) % 3) * kCtr, 0u);
-      st_relaxed(p.ctr + (3 + (r + 1) % 3) * kCtr, 0u);
-    }
-    const int32_t bound = (int32_t)min((int64_t)(epoch + 1) * p.delta, (int64_t)kInf - 1);
-    if (nin > 0 || nh > 0) {
-      uint32_t *qfar = p.fq + (size_t)(epoch % 3) * p.n;
-      uint32_t *cfar = p.ctr + (6 + epoch % 3) * kCtr;
-      // heavy chunks of the near input, spread over every wave of the grid
-      const uint64_t *hin = p.hq + (size_t)(r & 1) * p.hcap;
-      for (uint32_t i = gwave(); i < nh; i += gwaves()) {
-        const uint64_t ent = hin[i];
-        const uint32_t u = (uint32_t)ent, c = (uint32_t)(ent >> 32);
-        const uint32_t eb = p.row[u] + c * kBfsChunk, ee = min(p.row[u + 1], eb + kBfsChunk);
-        const int32_t du = ld_i32(p.dist + u);
-        for (uint32_t e0 = eb; e0 < ee; e0 += kSsBatch * 64) {
-          uint32_t vb[kSsBatch];
-          int32_t nd[kSsBatch];
-#pragma unroll
-          for (int x = 0; x < kSsBatch; ++x) {
-            const uint32_t e = e0 + 64 * x + lane_id();
-            vb[x] = e < ee ? __builtin_nontemporal_load(p.col + e) : 0xFFFFFFFFu;
-            nd[x] = e < ee ? du + (int32_t)__builtin_nontemporal_load(p.w + e) : 0;
-          }
-          sssp_relax_batch(p, vb, nd, bound, r + 2, qnear, cnear, hnear, hcnear, epoch + 1, qfar, cfar);
+  const Crew all(blockIdx.x, gridDim.x), few(team.rank, team.size);
+  SsState st{0, 0, 0, 0};
+  SsInput in;
+  in.seg.none();
+  // the queues' part of the next step's input
+  auto look = [&]() {
+    in.nin = ld_relaxed(ss_near_cnt(p, st.r));
+    in.nh = ld_relaxed(ss_heavy_cnt(p, st.r));
+    in.nfar = ld_relaxed(ss_far_cnt(p, st.epoch));
+  };
+  auto small = [&]() {
+    if (!team.usable) return false;
+    if (!in.near()) return in.nfar <= kTeamEdges / 4;
+    return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk <= kTeamEdges;
+  };
+  for (;;) {
+    look();
+    if (!in.near() && in.nfar == 0) break;
+    const bool by_team = small();
+    if (!by_team) {
+      sssp_step<false>(p, st, in, all, t0 == 0, nullptr, 0, &wb);
+    } else if (team.in) {
+      for (uint32_t k = 0; k < kTeamRounds; ++k) {
+        const uint32_t par = st.r & 1;
+        sssp_step<true>(p, st, in, few, t0 == 0, &out, team.rank, nullptr);
+        __syncthreads();
+        if (team.sync(a, out.segment_word(par), in.seg)) return;
+        in.nin = in.nh = 0;
+        in.nfar = 1;  // not looked at while there are near vertices
+        if (in.seg.queued) look();
+        if (!in.near()) {
+          // the kept far entries join the bucket's list
+          kept_flush(out, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
+          if (team.sync(a, 0, in.seg)) return;
+          look();
+          if (in.nfar == 0) break;
         }
+        if (!small()) break;
       }
-      // light near queue: 256 vertices per workgroup grab, wave64 fine-grained
-      const uint32_t *qin = p.nq + (size_t)(r & 1) * p.n;
-      uint32_t *wsc = p.ctr + (3 + r % 3) * kCtr;
-      for (;;) {
-        if (threadIdx.x == 0) s_base = add_relaxed(wsc, (uint32_t)kWg);
-        __syncthreads();
-        const uint32_t base = s_base;
-        __syncthreads();
-        if (base >= nin) break;
-        const uint32_t i = base + threadIdx.x;
-        const bool valid = i < nin;
-        const uint32_t u = valid ? qin[i] : 0u;
-        uint32_t b = 0, deg = 0;
-        int32_t du = 0;
-        if (valid) { b = p.row[u]; deg = p.row[u + 1] - b; du = ld_i32(p.dist + u); }
-        wave_expand<kSsBatch>(b, deg, [&](const uint32_t (&e)[kSsBatch], const bool (&ev)[kSsBatch],
-                                          const uint32_t (&own)[kSsBatch]) {
-          uint32_t vb[kSsBatch];
-          int32_t nd[kSsBatch];
-#pragma unroll
-          for (int x = 0; x < kSsBatch; ++x) {
-            const int32_t odu = __shfl(du, (int)own[x]);
-            vb[x] = ev[x] ? __builtin_nontemporal_load(p.col + e[x]) : 0xFFFFFFFFu;
-            nd[x] = ev[x] ? odu + (int32_t)__builtin_nontemporal_load(p.w + e[x]) : 0;
-          }
-          sssp_relax_batch(p, vb, nd, bound, r + 2, qnear, cnear, hnear, hcnear, epoch + 1, qfar, cfar);
-        });
+      kept_flush(out, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
+      if (t0 == 0) {
+        st_relaxed(ctl, st.r);
+        st_relaxed(ctl + 1, st.epoch);
+        st_relaxed(ctl + 2, st.relax);
+        st_relaxed(ctl + 3, st.far_since);
+        st_relaxed(ctl + 4, team.episode);
       }
-      ++relax_rounds;
     } else {
-      // near input empty: advance the bucket and split the far list
-      // (remove_dups_dev + curdelta += DELTA, kernel_gsrb.cu:310-348,669-677)
-      const uint32_t nfar = ld_relaxed(p.ctr + (6 + epoch % 3) * kCtr);
-      if (nfar == 0) break;
-      const uint32_t *fin = p.fq + (size_t)(epoch % 3) * p.n;
-      uint32_t *fout = p.fq + (size_t)((epoch + 1) % 3) * p.n;
-      uint32_t *cfout = p.ctr + (6 + (epoch + 1) % 3) * kCtr;
-      if (gtid() == 0) st_relaxed(p.ctr + (6 + (epoch + 2) % 3) * kCtr, 0u);
-      const int32_t nbound = (int32_t)min((int64_t)(epoch + 2) * p.delta, (int64_t)kInf - 1);
-      const uint32_t span = (nfar + kWg * kSsBatch - 1) / (kWg * kSsBatch) * (kWg * kSsBatch);
-      for (uint32_t i0 = blockIdx.x * kWg * kSsBatch + threadIdx.x; i0 < span; i0 += gthreads() * kSsBatch) {
-        uint32_t vb[kSsBatch];
-        bool to_near[kSsBatch], to_far[kSsBatch];
-#pragma unroll
-        for (int x = 0; x < kSsBatch; ++x) {
-          const uint32_t i = i0 + x * kWg;
-          vb[x] = i < nfar ? fin[i] : 0u;
-          to_near[x] = to_far[x] = false;
-          if (i < nfar) {
-            if (ld_i32(p.dist + vb[x]) <= nbound)
-              to_near[x] = __hip_atomic_exchange(p.nstamp + vb[x], r + 2, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT) != r + 2;
-            else
-              to_far[x] = __hip_atomic_exchange(p.fstamp + vb[x], epoch + 2, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT) != epoch + 2;
-          }
-        }
-        sssp_push_near(p, to_near, vb, qnear, cnear, hnear, hcnear);
-        wave_push_batch<kSsBatch>(fout, cfout, to_far, vb);
-      }
-      ++epoch;
+      gb.poll_sleep = kTeamIdleSleep;
     }
     if (gb.sync<KIND>()) return;
+    gb.poll_sleep = 0;
+    if (!by_team) {
+      in.seg.none();
+      continue;
+    }
+    st = SsState{ld_relaxed(ctl), ld_relaxed(ctl + 1), ld_relaxed(ctl + 2), ld_relaxed(ctl + 3)};
+    team.episode = ld_relaxed(ctl + 4);
+    // the segments of the last team round are still there
+    in.seg.take(lane_id() < team.size ? (uint32_t)ld_u64(team.word + (team.episode & 1) * kTeamMax + lane_id()) : 0u);
   }
-  if (gtid() == 0 && p.stats) { p.stats[0] = relax_rounds; p.stats[1] = epoch; }
+  for (uint64_t v = t0; v < p.n; v += nt) p.dist[v] = ss_dist(p.key[v]);
+  if (t0 == 0 && p.stats) { p.stats[0] = st.relax; p.stats[1] = st.epoch; }
 }
 
 // ===========================================================================
@@ -1581,6 +2073,19 @@ __global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k
 
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
+// Grid of a kernel of kTeamWg-thread workgroups for a request of num_wgs
+// workgroups of kWg threads (0: one workgroup per CU), at most one per CU.
+// Requests that kWg-thread workgroups could not serve (8 per CU) are refused as
+// they would be there.
+int team_grid_for(const void *k, hs_arena *ar, int num_wgs) {
+  constexpr int kPer = kTeamWg / kWg;
+  const int cus = hs_host::device_cus();
+  if (num_wgs > 8 * cus || num_wgs > ar->view.max_blocks) return -1;
+  int g = num_wgs > 0 ? (num_wgs + kPer - 1) / kPer : cus;
+  g = std::min({g, cus, ar->view.max_blocks});
+  return hs_host::check_residency(k, g, kTeamWg, 0) == HS_OK ? g : -1;
+}
+
 int grid_for(const void *k, hs_arena *ar, int num_wgs, int per_cu = 2) {
   if (num_wgs <= 0) {  // the default grid, within the arena's barrier slots
     num_wgs = hs_host::default_grid(k, kWg, per_cu);
@@ -1712,7 +2217,8 @@ int hs_msbfs(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const 
 int hs_sssp_work_size(uint32_t n, uint64_t m, uint64_t *bytes) {
   if (!bytes) return HS_ERR_INVALID;
   *bytes = align256(sizeof(uint32_t) * 2ull * n) + align256(sizeof(uint32_t) * 3ull * n) +
-           2 * align256(sizeof(uint32_t) * (uint64_t)n) + align256(sizeof(uint32_t) * 12 * kCtr) +
+           align256(sizeof(uint64_t) * (uint64_t)n) + align256(sizeof(uint32_t) * kSsCounters * kCtr) +
+           align256(sizeof(uint64_t) * 2 * kTeamMax * kSegCap) +
            align256(sizeof(uint64_t) * 2 * bfs_hcap(m));
   return HS_OK;
 }
@@ -1725,29 +2231,30 @@ int hs_sssp(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const u
     return HS_ERR_INVALID;
   const void *k = HS_KIND_SWITCH(k_sssp, kind);
   if (!k) return HS_ERR_INVALID;
-  const int g = grid_for(k, ar, num_wgs);
+  const int g = team_grid_for(k, ar, num_wgs);
   if (g < 0) return HS_ERR_RESIDENCY;
   hipStream_t s = (hipStream_t)stream;
   int rc = hs_host::prepare_barrier(ar, kind, s);
   if (rc) return rc;
   SsspArgs p{};
-  p.n = n; p.row = d_row; p.col = d_col; p.w = d_w; p.src = src;
+  p.n = n; p.m = (uint32_t)m; p.row = d_row; p.col = d_col; p.w = d_w; p.src = src;
   p.delta = delta > 0 ? delta : 10000;  // DELTA default, LONESTAR/apps/sssp/support.cu:10
   p.dist = d_dist;
   char *w = (char *)d_work;
   p.nq = (uint32_t *)w; w += align256(sizeof(uint32_t) * 2ull * n);
   p.fq = (uint32_t *)w; w += align256(sizeof(uint32_t) * 3ull * n);
-  p.nstamp = (uint32_t *)w; w += align256(sizeof(uint32_t) * (uint64_t)n);
-  p.fstamp = (uint32_t *)w; w += align256(sizeof(uint32_t) * (uint64_t)n);
-  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * 12 * kCtr);
+  p.key = (uint64_t *)w; w += align256(sizeof(uint64_t) * (uint64_t)n);
+  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * kSsCounters * kCtr);
+  p.seg = (uint64_t *)w; w += align256(sizeof(uint64_t) * 2 * kTeamMax * kSegCap);
   p.hq = (uint64_t *)w;
   p.hcap = bfs_hcap(m);
   p.stats = d_stats;
+  p.mean_degree = (uint32_t)((m + n - 1) / n);
   p.ng = (uint32_t)ar->view.num_groups;
   p.nx = (uint32_t)hs_host::xcd_groups(g);
   hs::ArenaView v = ar->view;
   void *args[] = {(void *)&v, (void *)&p};
-  return hs_host::launch_persistent(k, args, kind, g, kWg, 0, s);
+  return hs_host::launch_persistent(k, args, kind, g, kTeamWg, 0, s);
 }
 
 // ---------------------------------------------------------------- PageRank
