@@ -26,6 +26,13 @@ int hs_bfs(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uint32_t *d_
            const uint32_t *d_col, int32_t src, int32_t *d_level, void *d_work, int barrier_kind,
            int num_wgs, uint32_t *d_stats, void *stream);
 
+/* hs_bfs with the transposed graph as well (d_rrow, d_rcol: the in-edges): levels
+   whose frontier has a large part of the remaining edges are pulled.  Same
+   levels, d_stats and d_work size. */
+int hs_bfs_dir(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uint32_t *d_row,
+               const uint32_t *d_col, const uint32_t *d_rrow, const uint32_t *d_rcol, int32_t src,
+               int32_t *d_level, void *d_work, int barrier_kind, int num_wgs, uint32_t *d_stats,
+               void *stream);
 /* the same BFS with the reference's load balancer on (bfs -l: the inspector, the
    prefix sum over the degrees of the frontier vertices of out-degree >=
    DEGREE_LIMIT and the kernel that gives every thread an equal share of their

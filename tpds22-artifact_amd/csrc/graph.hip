@@ -62,13 +62,14 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t v, uint32_t lane) {
 }
 
 // ===========================================================================
-// single-source BFS (LONESTAR/apps/bfs/kernel_gsrb.cu:400-626)
-// Level-synchronous push.  A vertex reached at level L goes to one of two
+// single-source BFS with load balancing (LONESTAR/apps/bfs/kernel_gsrb.cu:400-626)
+// Level-synchronous push.  A vertex reached at level L goes to one of the
 // inputs of level L: the light queue (out-degree < kHeavy), expanded 256
 // vertices per workgroup grab with the wave64 fine-grained scheme, or, when
 // heavy, as chunks of kBfsChunk out-edges to the chunk list that every wave of
 // the grid shares (so one hub does not serialize a level on one workgroup).
 constexpr uint32_t kBfsChunk = 1024;
+constexpr int kBfsCounters = 15;
 
 struct BfsArgs {
   uint32_t n;
@@ -98,36 +99,7 @@ __device__ __forceinline__ uint32_t bfs_chunks(uint32_t d) {
   return d >= kHeavy ? (d + kBfsChunk - 1) / kBfsChunk : 0u;
 }
 
-// visit (kernel_gsrb.cu:473-479): the reference writes level[dst]=LEVEL when it
-// reads INF and may push duplicates; a CAS makes the push exactly-once.
-// kBfsBatch candidates per lane at once: their level loads, CASes and degree
-// loads are each in flight together before the wave-aggregated pushes.
 constexpr int kBfsBatch = 8;
-__device__ __forceinline__ void bfs_visit_batch(const BfsArgs &p, const uint32_t (&v)[kBfsBatch], int32_t L,
-                                                uint32_t *qout, uint32_t *cout, uint64_t *hout,
-                                                uint32_t *hcout) {
-  int32_t lv[kBfsBatch];
-#pragma unroll
-  for (int x = 0; x < kBfsBatch; ++x) lv[x] = v[x] != 0xFFFFFFFFu ? ld_i32(p.level + v[x]) : 0;
-  bool won[kBfsBatch];
-#pragma unroll
-  for (int x = 0; x < kBfsBatch; ++x) {
-    won[x] = false;
-    if (v[x] != 0xFFFFFFFFu && lv[x] == kInf) {
-      int32_t expected = kInf;
-      won[x] = __hip_atomic_compare_exchange_strong(p.level + v[x], &expected, L, __ATOMIC_RELAXED,
-                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  uint32_t nc[kBfsBatch];
-#pragma unroll
-  for (int x = 0; x < kBfsBatch; ++x) nc[x] = won[x] ? bfs_chunks(p.row[v[x] + 1] - p.row[v[x]]) : 0u;
-  bool light[kBfsBatch];
-#pragma unroll
-  for (int x = 0; x < kBfsBatch; ++x) light[x] = won[x] && nc[x] == 0;
-  wave_push_batch<kBfsBatch>(qout, cout, light, v);
-  wave_push_chunks_batch<kBfsBatch>(hout, hcout, nc, v);
-}
 
 // Load-balanced mode (the -l path of the reference: the inspector that moves
 // vertices of out-degree >= DEGREE_LIMIT to a work list with their degrees, the
@@ -197,16 +169,8 @@ __device__ __forceinline__ uint32_t bfs_lb_owner(const uint64_t *lin, uint32_t n
   return lo;
 }
 
-template <bool LB>
-__device__ __forceinline__ void bfs_visit(const BfsArgs &p, const uint32_t (&v)[kBfsBatch], int32_t L,
-                                          uint32_t *qout, uint32_t *cout, uint64_t *hout, uint32_t *hcout,
-                                          uint64_t *lout, uint64_t *lcout) {
-  if constexpr (LB) bfs_visit_batch_lb(p, v, L, qout, cout, hout, hcout, lout, lcout);
-  else bfs_visit_batch(p, v, L, qout, cout, hout, hcout);
-}
-
-template <int KIND, bool LB>
-__device__ __forceinline__ void bfs_run(ArenaView a, const BfsArgs &p) {
+template <int KIND>
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k_bfs_lb(ArenaView a, BfsArgs p) {
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   for (uint32_t v = gtid(); v < p.n; v += gthreads()) p.level[v] = (v == (uint32_t)p.src) ? 0 : kInf;
@@ -215,11 +179,11 @@ __device__ __forceinline__ void bfs_run(ArenaView a, const BfsArgs &p) {
       *cnt_at(p.ctr, i) = 0;
       *steal_at(p.ctr, i) = 0;
       *hcnt_at(p.ctr, i) = 0;
-      if (LB) *lbcnt_at(p.ctr, i) = 0;
+      *lbcnt_at(p.ctr, i) = 0;
     }
     const uint32_t d = p.row[p.src + 1] - p.row[p.src];
     const uint32_t nc = bfs_chunks(d);
-    if (LB && d >= p.lb_limit) {
+    if (d >= p.lb_limit) {
       p.lq[0] = (uint32_t)p.src;
       *lbcnt_at(p.ctr, 0) = (1ull << 32) | d;
     } else if (nc) {
@@ -236,29 +200,25 @@ __device__ __forceinline__ void bfs_run(ArenaView a, const BfsArgs &p) {
     const Frontier fr{p.q, p.ctr, p.ctr + 3 * kCtr, p.n, (uint32_t)kCtr};
     const uint32_t nin = fr.in_count(k);
     const uint32_t nh = ld_relaxed(hcnt_at(p.ctr, k % 3));
-    uint32_t nl = 0, el = 0;  // load-balanced mode: balanced entries and their edges
-    if constexpr (LB) {
-      const uint64_t lc = __hip_atomic_load(lbcnt_at(p.ctr, k % 3), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      nl = (uint32_t)(lc >> 32);
-      el = (uint32_t)lc;
-    }
+    const uint64_t lc = __hip_atomic_load(lbcnt_at(p.ctr, k % 3), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t nl = (uint32_t)(lc >> 32), el = (uint32_t)lc;  // balanced entries and their edges
     if (nin == 0 && nh == 0 && nl == 0) break;
     const uint32_t *qin = fr.in(k);
     uint32_t *qout = fr.out(k);
     const uint64_t *hin = p.hq + (size_t)(k & 1) * p.hcap;
     uint64_t *hout = p.hq + (size_t)((k + 1) & 1) * p.hcap;
-    const uint64_t *lin = LB ? p.lq + (size_t)(k & 1) * p.hcap : nullptr;
-    uint64_t *lout = LB ? p.lq + (size_t)((k + 1) & 1) * p.hcap : nullptr;
+    const uint64_t *lin = p.lq + (size_t)(k & 1) * p.hcap;
+    uint64_t *lout = p.lq + (size_t)((k + 1) & 1) * p.hcap;
     uint32_t *cout = fr.out_count(k);
     uint32_t *hcout = hcnt_at(p.ctr, (k + 1) % 3);
     uint64_t *lcout = lbcnt_at(p.ctr, (k + 1) % 3);
     if (gtid() == 0) {  // counters last used two levels ago
       fr.clear_for_next(k);
       st_relaxed(hcnt_at(p.ctr, (k + 2) % 3), 0u);
-      if (LB) __hip_atomic_store(lbcnt_at(p.ctr, (k + 2) % 3), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(lbcnt_at(p.ctr, (k + 2) % 3), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const int32_t L = (int32_t)k + 1;
-    if constexpr (LB) {
+    {
       // the balanced vertices' edges [0, el), an equal share per wave of the
       // grid; a lane's owner entry only moves forward as its edge does (an
       // entry holds >= kHeavy edges, a step of a lane 64 apart)
@@ -285,7 +245,7 @@ __device__ __forceinline__ void bfs_run(ArenaView a, const BfsArgs &p) {
               vb[x] = p.col[rb + (q - (uint32_t)(ent >> 32))];
             }
           }
-          bfs_visit<LB>(p, vb, L, qout, cout, hout, hcout, lout, lcout);
+          bfs_visit_batch_lb(p, vb, L, qout, cout, hout, hcout, lout, lcout);
         }
       }
     }
@@ -301,7 +261,7 @@ __device__ __forceinline__ void bfs_run(ArenaView a, const BfsArgs &p) {
           const uint32_t e = e0 + 64 * x + lane_id();
           vb[x] = e < ee ? p.col[e] : 0xFFFFFFFFu;
         }
-        bfs_visit<LB>(p, vb, L, qout, cout, hout, hcout, lout, lcout);
+        bfs_visit_batch_lb(p, vb, L, qout, cout, hout, hcout, lout, lcout);
       }
     }
     // light queue: 256 vertices per workgroup grab, wave64 fine-grained expansion
@@ -322,22 +282,12 @@ __device__ __forceinline__ void bfs_run(ArenaView a, const BfsArgs &p) {
         uint32_t vb[kBfsBatch];
 #pragma unroll
         for (int x = 0; x < kBfsBatch; ++x) vb[x] = ev[x] ? p.col[e[x]] : 0xFFFFFFFFu;
-        bfs_visit<LB>(p, vb, L, qout, cout, hout, hcout, lout, lcout);
+        bfs_visit_batch_lb(p, vb, L, qout, cout, hout, hcout, lout, lcout);
       });
     }
     if (gb.sync<KIND>()) return;
   }
   if (gtid() == 0 && p.stats) p.stats[0] = k;
-}
-
-template <int KIND>
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k_bfs(ArenaView a, BfsArgs p) {
-  bfs_run<KIND, false>(a, p);
-}
-
-template <int KIND>
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k_bfs_lb(ArenaView a, BfsArgs p) {
-  bfs_run<KIND, true>(a, p);
 }
 
 // ===========================================================================
@@ -1344,6 +1294,422 @@ __device__ __forceinline__ uint32_t queue_share(uint32_t nin, uint32_t waves) {
 }
 
 // ===========================================================================
+// single-source BFS (LONESTAR/apps/bfs/kernel_gsrb.cu:400-626)
+// Level-synchronous, pushing or (with the transposed graph) pulling.  A vertex
+// reached at level L joins the light queue of level L (out-degree < kHeavy) or,
+// when heavy, as chunks of kBfsChunk out-edges the chunk list that every wave of
+// the grid shares (so one hub does not serialize a level on one workgroup).
+// Small levels are pushed by a team (above).  A level whose frontier has a large
+// part of the edges not yet behind it is pulled (Beamer, Asanovic & Patterson,
+// "Direction-optimizing breadth-first search", 2012): the vertices not yet reached
+// look for an in-neighbour in the frontier's bitmap (512 KiB at R-MAT 22, kept in
+// L2) and stop at the first; no atomics, and the new bitmap is written a word per
+// wave.  R-MAT 22: 0.96 ms pushed only (2.0 ms with one queue atomic per 512
+// edges), 0.37 ms; a mesh of 720k vertices 15.9 -> 4.0 ms with the team.
+struct BfsArgs1 {
+  uint32_t n, m;
+  const uint32_t *row, *col, *rrow, *rcol;  // rrow, rcol null: push only
+  int32_t src;
+  int32_t *level;
+  uint32_t *q;    // [2][n] light frontier queues
+  uint64_t *hq;   // [2][hcap] heavy chunk entries v | chunk << 32
+  uint64_t hcap;
+  uint64_t *seg;  // [2][kTeamMax][kSegCap] segments of a team: v | first edge << 32
+  uint64_t *fbm[2];  // frontier bitmaps
+  uint32_t *ctr;  // light counts [3] (0..2), grab [3] (3..5), chunk counts [3] (6..8), pull chunks
+                  // [3] (9..11), the state a team stretch ends in (12), the team's words (13..14)
+  uint32_t *stats;
+  uint32_t mean_degree;
+  uint32_t ng, nx;
+};
+
+struct BfInput {
+  Segments seg;
+  uint32_t nin, nh;
+  __device__ bool any() const { return (seg.total | nin | nh) != 0; }
+};
+
+__device__ __forceinline__ uint32_t *bf_q(const BfsArgs1 &p, uint32_t r) { return p.q + (size_t)(r & 1) * p.n; }
+__device__ __forceinline__ uint64_t *bf_hq(const BfsArgs1 &p, uint32_t r) { return p.hq + (size_t)(r & 1) * p.hcap; }
+__device__ __forceinline__ uint32_t *bf_cnt(const BfsArgs1 &p, uint32_t r) { return p.ctr + (r % 3) * kCtr; }
+__device__ __forceinline__ uint32_t *bf_grab(const BfsArgs1 &p, uint32_t r) { return p.ctr + (3 + r % 3) * kCtr; }
+__device__ __forceinline__ uint32_t *bf_hcnt(const BfsArgs1 &p, uint32_t r) { return p.ctr + (6 + r % 3) * kCtr; }
+__device__ __forceinline__ uint32_t *bf_pcnt(const BfsArgs1 &p, uint32_t r) { return p.ctr + (9 + r % 3) * kCtr; }
+__device__ __forceinline__ uint64_t *bf_seg(const BfsArgs1 &p, uint32_t r, uint32_t rank) {
+  return p.seg + ((size_t)(r & 1) * kTeamMax + rank) * kSegCap;
+}
+
+struct BfStep {
+  const BfsArgs1 &p;
+  uint32_t r;
+  Output *out;  // of a team, else null, and the wave's lists instead
+  uint32_t rank;
+  WaveList<uint32_t, kWaveNear> light;
+  WaveList<uint64_t, kWaveChunks> chunks;
+
+  __device__ __forceinline__ void flush() { light.flush(); chunks.flush(); }
+};
+
+__device__ __forceinline__ BfStep bf_step(const BfsArgs1 &p, uint32_t r, Output *out, uint32_t rank, WaveBuffers *wb) {
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  return BfStep{p, r, out, rank,
+                {wb ? wb->near[wv] : nullptr, 0, bf_q(p, r + 1), bf_cnt(p, r + 1)},
+                {wb ? wb->chunks[wv] : nullptr, 0, bf_hq(p, r + 1), bf_hcnt(p, r + 1)}};
+}
+
+// new vertices of level r + 1 to its input
+template <bool TEAM, int B>
+__device__ __forceinline__ void bf_push(BfStep &s, const bool (&won)[B], const uint32_t (&v)[B], const uint32_t (&eb)[B],
+                                        const uint32_t (&deg)[B]) {
+  uint32_t nc[B];
+  bool light[B];
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    nc[x] = won[x] ? bfs_chunks(deg[x]) : 0u;
+    light[x] = won[x] && nc[x] == 0;
+  }
+  if constexpr (TEAM) {
+    segment_push<B>(*s.out, s.r & 1, bf_seg(s.p, s.r + 1, s.rank), s.light.q, s.light.cnt, light, v, eb);
+    if (team_push_chunks<B>(s.chunks.q, s.chunks.cnt, nc, v) && lane_id() == 0) s.out->queued[s.r & 1] = 1;
+  } else {
+    wave_list_push<B>(s.light, light, v);
+    wave_list_push_chunks<B>(s.chunks, nc, v);
+  }
+}
+
+// visit (kernel_gsrb.cu:473-479) of B candidates per lane (~0: none): the minimum
+// with the level says whether this visit is the vertex's first
+template <bool TEAM, int B>
+__device__ __forceinline__ void bf_visit(BfStep &s, const uint32_t (&v)[B]) {
+  constexpr bool kBlind = TEAM && B == 1;  // as in the SSSP's relaxation
+  const BfsArgs1 &p = s.p;
+  const int32_t L = (int32_t)s.r + 1;
+  int32_t lv[B];
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    lv[x] = 0;
+    if (v[x] != 0xFFFFFFFFu) lv[x] = kBlind ? kInf : ld_i32(p.level + v[x]);
+  }
+  bool won[B];
+  uint32_t eb[B], deg[B];
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    eb[x] = deg[x] = 0;
+    if (lv[x] == kInf) {
+      lv[x] = __hip_atomic_fetch_min(p.level + v[x], L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (TEAM) { eb[x] = p.row[v[x]]; deg[x] = p.row[v[x] + 1] - eb[x]; }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < B; ++x) {
+    won[x] = v[x] != 0xFFFFFFFFu && lv[x] == kInf;
+    if (!TEAM) deg[x] = won[x] ? p.row[v[x] + 1] - p.row[v[x]] : 0u;
+  }
+  bf_push<TEAM, B>(s, won, v, eb, deg);
+}
+
+template <bool TEAM>
+__device__ __forceinline__ void bf_expand(BfStep &s, uint32_t eb, uint32_t deg) {
+  constexpr int kB = TEAM ? 4 : kBfsBatch;
+  wave_expand<kB>(eb, deg, [&](const uint32_t (&e)[kB], const bool (&ev)[kB], const uint32_t (&)[kB]) {
+    uint32_t vb[kB];
+#pragma unroll
+    for (int x = 0; x < kB; ++x) vb[x] = ev[x] ? s.p.col[e[x]] : 0xFFFFFFFFu;
+    bf_visit<TEAM, kB>(s, vb);
+  });
+}
+
+template <bool TEAM>
+__device__ __forceinline__ void bf_push_level(const BfsArgs1 &p, uint32_t r, const BfInput &in, const Crew &crew,
+                                              Output *out, uint32_t rank, WaveBuffers *wb) {
+  const uint32_t lane = lane_id();
+  BfStep s = bf_step(p, r, out, rank, wb);
+  for (uint32_t b = crew.wave; b < in.seg.blocks; b += crew.waves) {
+    const uint32_t i = in.seg.entry(b), x = lane & 3;
+    const uint64_t ent = i != 0xFFFFFFFFu ? ld_u64(bf_seg(p, r, 0) + i) : 0ull;
+    const uint32_t u = (uint32_t)ent, eb = (uint32_t)(ent >> 32);
+    uint32_t end = eb, c = 0;
+    if (i != 0xFFFFFFFFu) {
+      end = p.row[u + 1];
+      if (eb + x < p.m) c = p.col[eb + x];
+    }
+    const uint32_t deg = end - eb;
+    if (TEAM && !ballot(deg > 4)) {
+      const uint32_t vb[1] = {x < deg ? c : 0xFFFFFFFFu};
+      bf_visit<TEAM, 1>(s, vb);
+    } else {
+      bf_expand<TEAM>(s, eb, x == 0 ? deg : 0u);
+    }
+  }
+  // heavy chunks, spread over the crew
+  constexpr int kB = TEAM ? 4 : kBfsBatch;
+  const uint64_t *hin = bf_hq(p, r);
+  for (uint32_t i = crew.wave; i < in.nh; i += crew.waves) {
+    const uint64_t ent = ld_u64(hin + i);
+    const uint32_t u = (uint32_t)ent, c = (uint32_t)(ent >> 32);
+    const uint32_t eb = p.row[u] + c * kBfsChunk, ee = min(p.row[u + 1], eb + kBfsChunk);
+    for (uint32_t e0 = eb; e0 < ee; e0 += kB * 64) {
+      uint32_t vb[kB];
+#pragma unroll
+      for (int x = 0; x < kB; ++x) {
+        const uint32_t e = e0 + 64 * x + lane;
+        vb[x] = e < ee ? p.col[e] : 0xFFFFFFFFu;
+      }
+      bf_visit<TEAM, kB>(s, vb);
+    }
+  }
+  // light queue: the first share of each wave is dealt, further ones are grabbed
+  const uint32_t *qin = bf_q(p, r);
+  const uint32_t share = queue_share(in.nin, crew.waves);
+  for (uint32_t b = crew.wave; (uint64_t)b * share < in.nin;) {
+    const uint32_t i = b * share + lane;
+    const bool valid = lane < share && i < in.nin;
+    const uint32_t u = valid ? ld_relaxed(qin + i) : 0u;
+    uint32_t eb = 0, deg = 0;
+    if (valid) { eb = p.row[u]; deg = p.row[u + 1] - eb; }
+    bf_expand<TEAM>(s, eb, deg);
+    if ((uint64_t)crew.waves * share >= in.nin) break;
+    uint32_t g = 0;
+    if (lane == 0) g = add_relaxed(bf_grab(p, r), 1u);
+    b = crew.waves + __builtin_amdgcn_readfirstlane(g);
+  }
+  if (!TEAM) s.flush();
+}
+
+// bitmap of level r's frontier from the levels
+__device__ __forceinline__ void bf_make_bitmap(const BfsArgs1 &p, uint32_t r, const Crew &crew) {
+  const uint32_t nblk = (p.n + 63) / 64;
+  for (uint32_t b = crew.wave; b < nblk; b += crew.waves) {
+    const uint32_t v = b * 64 + lane_id();
+    const uint64_t w = ballot(v < p.n && p.level[v] == (int32_t)r);
+    if (lane_id() == 0) p.fbm[r & 1][b] = w;
+  }
+}
+
+__device__ __forceinline__ bool bf_in_frontier(const uint64_t *fbm, uint32_t u) { return fbm[u >> 6] >> (u & 63u) & 1u; }
+
+// Pull: every vertex not yet reached looks through its in-edges for the frontier,
+// a wave 64 consecutive vertices at a time: the first kPullFirst in-edges by the
+// vertex's own lane, then the rest of the vertices still looking packed over the
+// wave, in rounds of 8, 16, ... 256 edges each, so that a vertex that finds its
+// parent early costs no more.  What is left of a vertex with more than kPullRest
+// in-edges becomes chunks that all waves share after the level's barrier.
+constexpr uint64_t kPullEdges = 8;
+constexpr uint32_t kPullFirst = 4, kPullRest = 8192, kPullChunk = 4096;
+
+__device__ __forceinline__ void bf_pull_found(BfStep &s, bool found, uint32_t v) {
+  const uint32_t row = found ? s.p.row[v] : 0u, end = found ? s.p.row[v + 1] : 0u;
+  const bool won[1] = {found};
+  const uint32_t vs[1] = {v}, eb[1] = {row}, deg[1] = {end - row};
+  bf_push<false, 1>(s, won, vs, eb, deg);
+}
+
+__device__ __forceinline__ void bf_pull_level(const BfsArgs1 &p, uint32_t r, const Crew &crew, WaveBuffers *wb) {
+  __shared__ uint32_t hit_sh[kTeamWg];
+  const uint32_t lane = lane_id();
+  uint32_t *hit = hit_sh + (threadIdx.x & ~63u);
+  BfStep s = bf_step(p, r, nullptr, 0, wb);
+  const uint64_t *fbm = p.fbm[r & 1];
+  uint64_t *nbm = p.fbm[(r + 1) & 1];
+  const uint32_t nblk = (p.n + 63) / 64, kb = log2_ceil(nblk);
+  for (uint32_t j = crew.wave; j < (1u << kb); j += crew.waves) {
+    const uint32_t blk = scatter_block(j, kb);
+    if (blk >= nblk) continue;
+    const uint32_t v = blk * 64 + lane;
+    const bool open = v < p.n && p.level[v] == kInf;
+    uint32_t b = 0, rem = 0;
+    if (open) { b = p.rrow[v]; rem = p.rrow[v + 1] - b; }
+    bool found = false;
+    {
+      uint32_t u[kPullFirst];
+      uint64_t w[kPullFirst];
+#pragma unroll
+      for (uint32_t x = 0; x < kPullFirst; ++x) u[x] = x < rem ? p.rcol[b + x] : 0xFFFFFFFFu;
+#pragma unroll
+      for (uint32_t x = 0; x < kPullFirst; ++x) w[x] = u[x] != 0xFFFFFFFFu ? fbm[u[x] >> 6] : 0ull;
+#pragma unroll
+      for (uint32_t x = 0; x < kPullFirst; ++x) found |= (w[x] >> (u[x] & 63u)) & 1u;
+      const uint32_t took = rem < kPullFirst ? rem : kPullFirst;
+      b += took;
+      rem = found ? 0u : rem - took;
+    }
+    for (uint32_t cap = 2 * kPullFirst; ballot(rem != 0); cap = cap < 256 ? cap * 2 : 256) {
+      if (cap == 256) {
+        const bool rest = rem > kPullRest;
+        if (ballot(rest)) {
+          // the rest of a hub: chunks by first edge, for everyone
+          const uint32_t nc = rest ? (rem + kPullChunk - 1) / kPullChunk : 0u;
+          const uint32_t incl = wave_incl_scan(nc);
+          uint32_t base = 0;
+          if (lane == 63) base = add_relaxed(bf_pcnt(p, r), incl);
+          base = __builtin_amdgcn_readlane(base, 63) + incl - nc;
+          for (uint32_t c = 0; c < nc; ++c) st_u64(bf_hq(p, r) + base + c, v | ((uint64_t)(b + c * kPullChunk) << 32));
+          if (rest) rem = 0;
+        }
+      }
+      hit[lane] = 0;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const uint32_t take = rem < cap ? rem : cap;
+      wave_expand<4>(b, take, [&](const uint32_t (&e)[4], const bool (&ev)[4], const uint32_t (&own)[4]) {
+        uint32_t u[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) u[x] = ev[x] ? p.rcol[e[x]] : 0u;
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          if (ev[x] && bf_in_frontier(fbm, u[x])) hit[own[x]] = 1;
+      });
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const bool got = hit[lane] != 0;
+      found |= got;
+      b += take;
+      rem = got ? 0u : rem - take;
+    }
+    const uint64_t fm = ballot(found);
+    if (lane == 0) nbm[blk] = fm;
+    if (found) p.level[v] = (int32_t)r + 1;
+    if (fm) bf_pull_found(s, found, v);
+  }
+  s.flush();
+}
+
+// the hubs' chunks: the first wave that finds a parent reaches the vertex
+__device__ __forceinline__ void bf_pull_chunks(const BfsArgs1 &p, uint32_t r, uint32_t count, const Crew &crew,
+                                               WaveBuffers *wb) {
+  const uint32_t lane = lane_id();
+  BfStep s = bf_step(p, r, nullptr, 0, wb);
+  const uint64_t *fbm = p.fbm[r & 1];
+  for (uint32_t i = crew.wave; i < count; i += crew.waves) {
+    const uint64_t ent = ld_u64(bf_hq(p, r) + i);
+    const uint32_t v = (uint32_t)ent, eb = (uint32_t)(ent >> 32);
+    const uint32_t ee = min(p.rrow[v + 1], eb + kPullChunk);
+    bool found = false;
+    for (uint32_t e0 = eb; e0 < ee && ld_i32(p.level + v) == kInf; e0 += 4 * 64) {
+      bool h = false;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const uint32_t e = e0 + 64 * x + lane;
+        h |= e < ee && bf_in_frontier(fbm, p.rcol[e]);
+      }
+      if (ballot(h)) { found = true; break; }
+    }
+    bool won = false;
+    if (found && lane == 0)
+      won = __hip_atomic_fetch_min(p.level + v, (int32_t)r + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kInf;
+    if (won) __hip_atomic_fetch_or(p.fbm[(r + 1) & 1] + (v >> 6), 1ull << (v & 63u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (ballot(won)) bf_pull_found(s, won, v);
+  }
+  s.flush();
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4))) k_bfs(ArenaView a, BfsArgs1 p) {
+  GridBarrier gb;
+  gb.init(a, KIND, p.ng, p.nx);
+  Team team;
+  team.init(reinterpret_cast<uint64_t *>(p.ctr + 13 * kCtr), p.nx);
+  uint32_t *ctl = p.ctr + 12 * kCtr;
+  __shared__ Output out;
+  __shared__ WaveBuffers wb;
+  const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
+  for (uint64_t v = t0; v < p.n; v += nt) p.level[v] = v == (uint32_t)p.src ? 0 : kInf;
+  if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
+  if (t0 < 2 * kTeamMax) team.word[t0] = 0;
+  if (t0 == 0) {
+    for (int i = 0; i < 12; ++i) p.ctr[i * kCtr] = 0;
+    const uint32_t nc = bfs_chunks(p.row[p.src + 1] - p.row[p.src]);
+    for (uint32_t c = 0; c < nc; ++c) p.hq[c] = (uint32_t)p.src | ((uint64_t)c << 32);
+    p.ctr[6 * kCtr] = nc;
+    p.q[0] = (uint32_t)p.src;
+    p.ctr[0] = nc ? 0u : 1u;
+  }
+  if (gb.sync<KIND>()) return;
+  const Crew all(blockIdx.x, gridDim.x), few(team.rank, team.size);
+  uint32_t r = 0;
+  uint64_t behind = 0;        // edges of the frontiers so far, by the same estimate as `ahead` below
+  bool have_bitmap = false;   // of the present frontier
+  BfInput in;
+  in.seg.none();
+  auto look = [&]() {
+    in.nin = ld_relaxed(bf_cnt(p, r));
+    in.nh = ld_relaxed(bf_hcnt(p, r));
+  };
+  auto edges = [&]() { return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk; };
+  auto clear_next = [&]() {  // counters last used two levels ago
+    if (t0 != 0) return;
+    st_relaxed(bf_cnt(p, r + 2), 0u);
+    st_relaxed(bf_hcnt(p, r + 2), 0u);
+    st_relaxed(bf_pcnt(p, r + 1), 0u);
+    st_relaxed(bf_grab(p, r + 1), 0u);
+  };
+  for (;;) {
+    look();
+    if (!in.any()) break;
+    const uint64_t ahead = edges();
+    const bool by_team = team.usable && ahead <= kTeamEdges;
+    // Pull once the frontier's edges are 1/kPullEdges of those left (they are
+    // estimated by the mean degree, which a frontier of hubs exceeds).  Any factor
+    // from 4 to 64 gives the same times at R-MAT 12..22; 2 costs 45% at R-MAT 22.
+    const bool pull = p.rrow && !by_team && ahead * kPullEdges > (p.m > behind ? p.m - behind : 0);
+    if (pull && !have_bitmap) {
+      bf_make_bitmap(p, r, all);
+      if (gb.sync<KIND>()) return;
+      have_bitmap = true;
+      continue;
+    }
+    behind += ahead;
+    if (pull) {
+      clear_next();
+      bf_pull_level(p, r, all, &wb);
+    } else if (!by_team) {
+      clear_next();
+      bf_push_level<false>(p, r, in, all, nullptr, 0, &wb);
+    } else if (team.in) {
+      for (uint32_t k = 0; k < kTeamRounds; ++k) {
+        const uint32_t par = r & 1;
+        if (threadIdx.x == 0) out.clear(par ^ 1);
+        clear_next();
+        bf_push_level<true>(p, r, in, few, &out, team.rank, nullptr);
+        ++r;
+        __syncthreads();
+        if (team.sync(a, out.segment_word(par), in.seg)) return;
+        in.nin = in.nh = 0;
+        if (in.seg.queued) look();
+        if (!in.any() || edges() > kTeamEdges) break;
+        behind += edges();
+      }
+      if (t0 == 0) {
+        st_relaxed(ctl, r);
+        st_relaxed(ctl + 1, team.episode);
+        st_u64(reinterpret_cast<uint64_t *>(ctl + 2), behind);
+      }
+    } else {
+      gb.poll_sleep = kTeamIdleSleep;
+    }
+    if (gb.sync<KIND>()) return;
+    gb.poll_sleep = 0;
+    have_bitmap = pull;
+    if (by_team) {
+      r = ld_relaxed(ctl);
+      team.episode = ld_relaxed(ctl + 1);
+      behind = ld_u64(reinterpret_cast<uint64_t *>(ctl + 2));
+      // the segments of the last team level are still there
+      in.seg.take(lane_id() < team.size ? (uint32_t)ld_u64(team.word + (team.episode & 1) * kTeamMax + lane_id()) : 0u);
+      continue;
+    }
+    in.seg.none();
+    if (pull) {
+      const uint32_t hubs = ld_relaxed(bf_pcnt(p, r));
+      if (hubs) {
+        bf_pull_chunks(p, r, hubs, all, &wb);
+        if (gb.sync<KIND>()) return;
+      }
+    }
+    ++r;
+  }
+  if (t0 == 0 && p.stats) p.stats[0] = r;
+}
+
+// ===========================================================================
 // SSSP, near/far buckets (LONESTAR/apps/sssp/kernel_gsrb.cu:459-687).
 struct SsspArgs {
   uint32_t n, m;
@@ -2107,20 +2473,73 @@ extern "C" {
 // d / kHeavy chunks of kBfsChunk, and each vertex is reached once
 static uint64_t bfs_hcap(uint64_t m) { return m / kHeavy + 64; }
 
+// work layouts: queues, counters, chunk lists, then (load-balanced) the balanced
+// lists or (plain) the bitmaps; the team's segments last
+static uint64_t bfs_bitmap_bytes(uint32_t n) { return align256(sizeof(uint64_t) * ((n + 63ull) / 64)); }
+
 int hs_bfs_work_size(uint32_t n, uint64_t m, uint64_t *bytes) {
   if (!bytes) return HS_ERR_INVALID;
-  *bytes = align256(sizeof(uint32_t) * 2ull * n) + align256(sizeof(uint32_t) * 12 * kCtr) +
-           2 * align256(sizeof(uint64_t) * 2 * bfs_hcap(m));
+  *bytes = align256(sizeof(uint32_t) * 2ull * n) + align256(sizeof(uint32_t) * kBfsCounters * kCtr) +
+           2 * align256(sizeof(uint64_t) * 2 * bfs_hcap(m)) + 2 * bfs_bitmap_bytes(n) +
+           align256(sizeof(uint64_t) * 2 * kTeamMax * kSegCap);
   return HS_OK;
 }
 
+static bool bfs_args_ok(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col, int32_t src,
+                        const int32_t *d_level, const void *d_work) {
+  return ar && d_row && (!m || d_col) && d_level && d_work && n != 0 && src >= 0 && (uint32_t)src < n &&
+         m <= 0xFFFFFFFFull;
+}
+
 static int bfs_launch(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
-                      int32_t src, int32_t *d_level, void *d_work, int kind, int num_wgs, bool lb,
-                      int degree_limit, uint32_t *d_stats, void *stream) {
-  if (!ar || !d_row || (m && !d_col) || !d_level || !d_work || n == 0 || src < 0 ||
-      (uint32_t)src >= n || m > 0xFFFFFFFFull || (lb && degree_limit != 0 && degree_limit < (int)kHeavy))
+                      const uint32_t *d_rrow, const uint32_t *d_rcol, int32_t src, int32_t *d_level, void *d_work,
+                      int kind, int num_wgs, uint32_t *d_stats, void *stream) {
+  if (!bfs_args_ok(ar, n, m, d_row, d_col, src, d_level, d_work)) return HS_ERR_INVALID;
+  const void *k = HS_KIND_SWITCH(k_bfs, kind);
+  if (!k) return HS_ERR_INVALID;
+  const int g = team_grid_for(k, ar, num_wgs);
+  if (g < 0) return HS_ERR_RESIDENCY;
+  hipStream_t s = (hipStream_t)stream;
+  int rc = hs_host::prepare_barrier(ar, kind, s);
+  if (rc) return rc;
+  BfsArgs1 p{};
+  p.n = n; p.m = (uint32_t)m; p.row = d_row; p.col = d_col; p.rrow = d_rrow; p.rcol = d_rcol;
+  p.src = src; p.level = d_level;
+  char *w = (char *)d_work;
+  p.q = (uint32_t *)w; w += align256(sizeof(uint32_t) * 2ull * n);
+  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * kBfsCounters * kCtr);
+  p.hq = (uint64_t *)w; w += align256(sizeof(uint64_t) * 2 * bfs_hcap(m));
+  p.hcap = bfs_hcap(m);
+  for (auto &f : p.fbm) { f = (uint64_t *)w; w += bfs_bitmap_bytes(n); }
+  p.seg = (uint64_t *)w;
+  p.stats = d_stats;
+  p.mean_degree = (uint32_t)((m + n - 1) / n);
+  p.ng = (uint32_t)ar->view.num_groups;
+  p.nx = (uint32_t)hs_host::xcd_groups(g);
+  hs::ArenaView v = ar->view;
+  void *args[] = {(void *)&v, (void *)&p};
+  return hs_host::launch_persistent(k, args, kind, g, kTeamWg, 0, s);
+}
+
+int hs_bfs(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
+           int32_t src, int32_t *d_level, void *d_work, int kind, int num_wgs, uint32_t *d_stats,
+           void *stream) {
+  return bfs_launch(ar, n, m, d_row, d_col, nullptr, nullptr, src, d_level, d_work, kind, num_wgs, d_stats, stream);
+}
+
+int hs_bfs_dir(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
+               const uint32_t *d_rrow, const uint32_t *d_rcol, int32_t src, int32_t *d_level, void *d_work, int kind,
+               int num_wgs, uint32_t *d_stats, void *stream) {
+  if (!d_rrow || (m && !d_rcol)) return HS_ERR_INVALID;
+  return bfs_launch(ar, n, m, d_row, d_col, d_rrow, d_rcol, src, d_level, d_work, kind, num_wgs, d_stats, stream);
+}
+
+int hs_bfs_lb(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
+              int32_t src, int32_t *d_level, void *d_work, int kind, int num_wgs, int degree_limit,
+              uint32_t *d_stats, void *stream) {
+  if (!bfs_args_ok(ar, n, m, d_row, d_col, src, d_level, d_work) || (degree_limit != 0 && degree_limit < (int)kHeavy))
     return HS_ERR_INVALID;
-  const void *k = lb ? HS_KIND_SWITCH(k_bfs_lb, kind) : HS_KIND_SWITCH(k_bfs, kind);
+  const void *k = HS_KIND_SWITCH(k_bfs_lb, kind);
   if (!k) return HS_ERR_INVALID;
   const int g = grid_for(k, ar, num_wgs);
   if (g < 0) return HS_ERR_RESIDENCY;
@@ -2131,32 +2550,19 @@ static int bfs_launch(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_ro
   p.n = n; p.row = d_row; p.col = d_col; p.src = src; p.level = d_level;
   p.q = (uint32_t *)d_work;
   p.ctr = (uint32_t *)((char *)d_work + align256(sizeof(uint32_t) * 2ull * n));
-  p.hq = (uint64_t *)((char *)p.ctr + align256(sizeof(uint32_t) * 12 * kCtr));
+  p.hq = (uint64_t *)((char *)p.ctr + align256(sizeof(uint32_t) * kBfsCounters * kCtr));
   p.hcap = bfs_hcap(m);
   p.lq = (uint64_t *)((char *)p.hq + align256(sizeof(uint64_t) * 2 * p.hcap));
   p.stats = d_stats;
   // the reference's DEGREE_LIMIT under -l is the grid's thread count
   // (LONESTAR/rt/include/ggcuda.h:19-22); at least kHeavy, so that the heavy
   // list of a level (at most m / limit entries) fits hcap
-  p.lb_limit = lb ? (degree_limit > 0 ? (uint32_t)degree_limit : (uint32_t)g * kWg) : 0u;
+  p.lb_limit = degree_limit > 0 ? (uint32_t)degree_limit : (uint32_t)g * kWg;
   p.ng = (uint32_t)ar->view.num_groups;
   p.nx = (uint32_t)hs_host::xcd_groups(g);
   hs::ArenaView v = ar->view;
   void *args[] = {(void *)&v, (void *)&p};
   return hs_host::launch_persistent(k, args, kind, g, kWg, 0, s);
-}
-
-int hs_bfs(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
-           int32_t src, int32_t *d_level, void *d_work, int kind, int num_wgs, uint32_t *d_stats,
-           void *stream) {
-  return bfs_launch(ar, n, m, d_row, d_col, src, d_level, d_work, kind, num_wgs, false, 0, d_stats, stream);
-}
-
-int hs_bfs_lb(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
-              int32_t src, int32_t *d_level, void *d_work, int kind, int num_wgs, int degree_limit,
-              uint32_t *d_stats, void *stream) {
-  return bfs_launch(ar, n, m, d_row, d_col, src, d_level, d_work, kind, num_wgs, true, degree_limit, d_stats,
-                    stream);
 }
 
 // ---------------------------------------------------------------- MS-BFS

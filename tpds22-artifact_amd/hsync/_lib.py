@@ -145,6 +145,7 @@ SIGNATURES = {
 GRAPH_SIGNATURES = {
     "hs_bfs_work_size": (_I, [_U32, _U64, _PU64]),
     "hs_bfs": (_I, [_P, _U32, _U64, _P, _P, C.c_int32, _P, _P, _I, _I, _P, _P]),
+    "hs_bfs_dir": (_I, [_P, _U32, _U64, _P, _P, _P, _P, C.c_int32, _P, _P, _I, _I, _P, _P]),
     "hs_bfs_lb": (_I, [_P, _U32, _U64, _P, _P, C.c_int32, _P, _P, _I, _I, _I, _P, _P]),
     "hs_msbfs_work_size": (_I, [_U32, _U64, _I, _PU64]),
     "hs_msbfs": (_I, [_P, _U32, _U64, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P, _P]),

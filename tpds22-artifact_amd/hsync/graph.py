@@ -126,7 +126,10 @@ def bfs(arena: Arena, g: Graph, src: int, barrier="xcd", num_wgs: int = 0, level
     level = level if level is not None else torch.empty(g.n, dtype=torch.int32, device="cuda")
     stats = torch.zeros(4, dtype=torch.int32, device="cuda")
     s = _stream(stream)
-    if lb is None:
+    if lb is None and hasattr(g, "rrow"):  # with the in-edges at hand, large levels are pulled
+        L.check(lib.hs_bfs_dir(arena.handle, g.n, g.m, _ptr(g.row), _ptr(g.col), _ptr(g.rrow), _ptr(g.rcol), src,
+                               _ptr(level), _ptr(work), barrier_kind(barrier), num_wgs, _ptr(stats), s), "hs_bfs_dir")
+    elif lb is None:
         L.check(lib.hs_bfs(arena.handle, g.n, g.m, _ptr(g.row), _ptr(g.col), src, _ptr(level), _ptr(work),
                            barrier_kind(barrier), num_wgs, _ptr(stats), s), "hs_bfs")
     else:
