@@ -25,6 +25,8 @@
 // Dijkstra.  A final pass transposes dist into the caller's [nsrc][n] array.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "hs_graph.h"
 #include "hs_internal.hpp"
 #include "hs_wave.hpp"
@@ -41,11 +43,12 @@ namespace {
 
 constexpr int kWg = 256;
 constexpr int32_t kInf = 0x7FFFFFFF;
-constexpr uint32_t kHeavy = 256;   // degree at which a vertex is cut into chunks
-constexpr uint32_t kChunk = 1024;  // edges per chunk of a heavy vertex
+constexpr uint32_t kHeavy = 64;    // degree at which a vertex is cut into chunks
+constexpr uint32_t kChunk = 64;    // edges per chunk of a heavy vertex
 constexpr int kCtr = 64;           // words between counters
 constexpr int kEdgeBatch = 8;      // edges whose head distances are in flight per wave
-constexpr int kGrab = 8;           // list entries a wave takes per atomic
+constexpr uint32_t kGrab = 16;    // list entries a wave takes per atomic, at most
+constexpr uint32_t kStageItems = 256;  // list entries a wave stages in LDS
 
 struct MsspArgs {
   uint32_t n;
@@ -77,10 +80,26 @@ __device__ __forceinline__ int32_t ld_i32(const int32_t *q) {
 // Phase A over all vertices: pend |= nx; expand the pending sources below
 // `bound`.  Per-workgroup totals go to part[wg].
 __device__ void mssp_select(const MsspArgs &p, uint32_t par, int32_t bound) {
+  // appends are staged per wave: every atomic on the list's counter serializes
+  // for ~11 ns, and one per 64 vertices cost a large round 0.3 ms (2M vertices)
+  __shared__ uint64_t stage[kWg / 64][kStageItems];
+  uint64_t *mine = stage[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+  uint32_t staged = 0;  // the same in every lane
   uint64_t expanded = 0, pending = 0, pairs = 0;
   int32_t minpend = kInf;
   uint64_t *list = p.items + (size_t)par * p.icap;
   uint32_t *cnt = items_cnt(p, par);
+  auto flush = [&]() {
+    if (staged == 0) return;
+    uint32_t at = 0;
+    if (lane_id() == 0) at = add_relaxed(cnt, staged);
+    at = __builtin_amdgcn_readfirstlane(at);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (uint32_t i = lane_id(); i < staged; i += 64)
+      if (at + i < p.icap) list[at + i] = mine[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    staged = 0;
+  };
   // whole waves step together (v = wave base + lane), so the list append can
   // be one atomic per wave
   for (uint32_t wb = blockIdx.x * kWg + (threadIdx.x & ~63u); wb < p.n; wb += gthreads()) {
@@ -113,16 +132,21 @@ __device__ void mssp_select(const MsspArgs &p, uint32_t par, int32_t bound) {
       const uint32_t b = p.row[v], deg = p.row[v + 1] - b;
       nc = deg >= kHeavy ? (deg + kChunk - 1) / kChunk : (deg ? 1u : 0u);
     }
-    // wave-aggregated append of the list entries (one atomic per wave)
     const uint32_t incl = wave_incl_scan(nc);
     const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-    if (total) {
+    if (staged + total > kStageItems) flush();
+    if (total > kStageItems) {
       uint32_t at = 0;
       if (lane_id() == 0) at = add_relaxed(cnt, total);
       at = __shfl(at, 0) + incl - nc;
       for (uint32_t c = 0; c < nc && at + c < p.icap; ++c) list[at + c] = v | ((uint64_t)c << 32);
+    } else {
+      const uint32_t at = staged + incl - nc;
+      for (uint32_t c = 0; c < nc; ++c) mine[at + c] = v | ((uint64_t)c << 32);
+      staged += total;
     }
   }
+  flush();
   // workgroup totals
   __shared__ uint64_t red[4][kWg / 64];
   uint64_t vals[4] = {expanded, pending, (uint64_t)(uint32_t)minpend, pairs};
@@ -187,14 +211,20 @@ __device__ void mssp_relax(const MsspArgs &p, uint32_t par) {
   const uint32_t total = ld_relaxed(items_cnt(p, par));
   const uint32_t nitems = total < p.icap ? total : (uint32_t)p.icap;
   uint32_t *steal = steal_cnt(p, par);
-  // kGrab entries per atomic: one shared counter serializes its atomics, so
-  // one per entry would cost ~11 ns x entries
+  // One shared counter serializes its atomics (~11 ns each), so in long lists a
+  // wave takes kGrab entries at once; in short ones few enough for every wave of
+  // the grid to get some.  Entries are at most kChunk edges, so that a grab is at
+  // most 1024: with chunks of 1024 edges the last grabs of a hub's entries took
+  // most of a round (R-MAT 21, 64 sources: chunks of 1024 / 256 / 128 / 64 edges
+  // by 8 / 8 / 8 / 16 take 35.4 / 22.8 / 21.3 / 20.6 ms, 64 by 32 22.5 ms).
+  const uint32_t even = nitems / (2u * gridDim.x * (kWg / 64)) + 1;
+  const uint32_t grab = even < kGrab ? even : kGrab;
   for (;;) {
     uint32_t it0 = 0;
-    if (lane == 0) it0 = add_relaxed(steal, (uint32_t)kGrab);
+    if (lane == 0) it0 = add_relaxed(steal, grab);
     it0 = __shfl(it0, 0);
     if (it0 >= nitems) break;
-    const uint32_t itn = it0 + (uint32_t)kGrab < nitems ? it0 + (uint32_t)kGrab : nitems;
+    const uint32_t itn = it0 + grab < nitems ? it0 + grab : nitems;
     // the grabbed entries in one load (lane k holds entry it0 + k)
     const uint64_t ents = lane < itn - it0 ? list[it0 + lane] : 0ull;
     // the next entry's mask, head distances and offsets are loaded while the
@@ -262,7 +292,7 @@ __device__ void mssp_relax(const MsspArgs &p, uint32_t par) {
 }
 
 template <int KIND>
-__global__ void __launch_bounds__(kWg) k_mssp(ArenaView a, MsspArgs p) {
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(6))) k_mssp(ArenaView a, MsspArgs p) {
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nxcd);
   // init: every distance INF, nothing pending; counters of both parities 0
@@ -381,9 +411,10 @@ int hs_mssp(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const u
     return HS_ERR_INVALID;
   const void *k = HS_KIND_SWITCH(k_mssp, kind);
   if (!k) return HS_ERR_INVALID;
-  // 4 workgroups per CU (measured: 36 / 41 ms at 4 / 2 per CU for 64 sources on
-  // R-MAT 20; the relaxation is latency-bound per wave)
-  if (num_wgs <= 0) num_wgs = hs_host::default_grid(k, kWg, 4);
+  // 6 workgroups per CU, what 80 registers leave room for (R-MAT 21, 64 sources:
+  // 20.5 / 17.7 / 17.0 / 20.4 ms at 4 / 5 / 6 / 8, where 8 spill): the relaxation is
+  // bound by the gathers in flight
+  if (num_wgs <= 0) num_wgs = std::min(hs_host::default_grid(k, kWg, 6), (int)ar->view.max_blocks);
   if (num_wgs > ar->view.max_blocks || num_wgs > 8192) return HS_ERR_INVALID;
   if (hs_host::check_residency(k, num_wgs, kWg, 0) != HS_OK) return HS_ERR_RESIDENCY;
   hipStream_t s = (hipStream_t)stream;
