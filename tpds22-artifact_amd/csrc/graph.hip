@@ -10,8 +10,7 @@
 // each wave takes up to 64 frontier vertices, scans their degrees with DPP and
 // hands the concatenated edge list out 64 edges at a time (fine grained, the
 // owner found by a 6-step shuffle search); vertices of degree >= 256 are
-// expanded by the whole workgroup (BFS/SSSP) or split into fixed chunks that
-// every wave of the grid shares (multi-source BFS, PageRank).
+// split into fixed chunks that every wave of the grid shares.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,16 +34,7 @@ namespace {
 constexpr int kWg = 256;
 constexpr int32_t kInf = 0x7FFFFFFF;
 constexpr uint32_t kHeavy = 256;     // degree at which a vertex leaves the fine-grained path
-constexpr uint32_t kChunk = 4096;    // edges per shared chunk of a heavy vertex
 constexpr int kCtr = 64;             // words between counters
-// PageRank: 64-edge steps in flight per wave (light blocks) and per lane (heavy
-// chunks).  The pull is bound by the L1's outstanding misses (the random
-// gathers), not by how many a wave can issue: on R-MAT 22 an iteration takes
-// 505 us with 8 and 8, 452 with 4 and 8, 439 with 4 and 2.  The step grouping
-// does not change any sum's order.
-constexpr int kPrSteps = 4;
-constexpr int kPrHeavySteps = 2;
-
 __device__ __forceinline__ uint32_t gtid() { return blockIdx.x * kWg + threadIdx.x; }
 __device__ __forceinline__ uint32_t gthreads() { return gridDim.x * kWg; }
 __device__ __forceinline__ uint32_t gwave() { return blockIdx.x * (kWg / 64) + (threadIdx.x >> 6); }
@@ -2078,24 +2068,31 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
 }
 
 // ===========================================================================
-// PageRank, FP32, pull over the transposed CSR in a fixed summation order.
+// PageRank, FP32 ranks and contributions, FP64 sums, pull over the transposed CSR
+// in a fixed summation order.
 //   x'[v] = (1-a)/n + a*(D/n + sum_{u->v} x[u]/deg(u)),  D = dangling mass
-// Light vertices (in-degree < kHeavy) are pulled by blocks of 64 consecutive
-// vertices, one wave per block: the block's in-edges are walked as one
-// flattened sequence, 64 per step (coalesced column loads), and summed per
-// vertex by a segmented wave scan; the step sums are added in step order.
-// Heavy vertices are cut into chunks of kChunk in-edges; a wave sums a chunk,
-// and the wave that finishes the vertex's last chunk of the iteration (a
-// per-vertex arrival counter) adds its chunk sums in chunk order and finalizes
-// the vertex.  Every vertex is finalized in the same phase as its sums, so an
-// iteration needs one grid barrier.  The dangling mass and the L1 change are
-// summed in 2^-60 fixed point (integer sums: the same bits whatever the grid
-// or the order).  Every order is fixed by the graph alone, so the ranks do not
-// depend on the grid.
-// Chunk slots: the chunk c of heavy vertex v lives at slot ceil(rrow[v]/kHeavy)+c.
-// A vertex with d >= kHeavy in-edges has at most d/kHeavy chunks, so its slots
-// stay below ceil(rrow[v+1]/kHeavy) and never meet another vertex's; slot i is
-// owned by the vertex whose in-edge range holds edge i*kHeavy.
+// The in-edges and the vertices form one sequence: a vertex's in-edges, then the
+// vertex itself (its "end"), vertex after vertex.  Span i is positions [i S, (i+1) S)
+// of it, whatever the degrees are, so every span costs about the same and a wave
+// needs no other balancing; the vertices a span starts with are found once per
+// launch.  A wave loads the span's sources 16 bytes per lane, gathers their
+// contributions (all in flight together: the gathers' L1 lookups are what bounds an
+// iteration), writes the running sums to LDS, and then each lane takes a vertex
+// that ends in the span as a difference of two of them.  A vertex cut by span
+// boundaries leaves one piece per span; the wave that adds the last of its pieces
+// (an arrival counter at the span it ends in) sums them in span order and
+// finalizes it.  So every vertex is finalized in the same phase as its sums, and an
+// iteration needs one grid barrier.  The dangling mass and the L1 change are summed
+// in 2^-60 fixed point (integer sums: the same bits whatever the grid or the
+// order).  Every order is fixed by the graph alone, so the ranks do not depend on
+// the grid.
+// R-MAT 22: 0.39 ms an iteration (0.45 with 64-vertex blocks, hub chunks and
+// segmented FP32 scans), 64M gathers that each miss the L1 (128-byte lines, 16 MB of
+// contributions): 0.6 requests per clock and L2 channel.  Streaming gathers take
+// twice as long, agent-scope ones the same; 512 positions per span 0.44 ms.
+constexpr int kPrQuads = 4;                   // S = 1024, of small graphs 256
+constexpr uint64_t kPrLargeFrom = 1ull << 22;  // vertices and edges from which spans are large
+
 struct PrArgs {
   uint32_t n;
   const uint32_t *row, *rrow, *rcol;
@@ -2104,37 +2101,15 @@ struct PrArgs {
   float *rank;      // output
   float *x;         // [2][n] iterates
   float *contrib;   // [2][n]
-  float *hsum;      // [nslots] heavy chunk sums
-  uint64_t *hent;   // [nslots] slot owner v | chunk << 32, or ~0 for an unused slot
-  uint32_t nslots;
-  uint32_t *harr;   // [nslots] per heavy vertex (at its first slot): chunk arrivals so far
-  uint64_t *lpre;   // [ceil(n/64)] light block weight prefix inside each workgroup range
-  uint64_t *spre;   // [nslots] slot weight prefix inside each workgroup range
-  uint64_t *wtot;   // [2][W] range totals: light blocks, slots
+  uint32_t *first;  // [nspans + 1] first vertex whose end is not before the span
+  double *tail;     // [nspans] piece of the vertex that runs on past the span
+  double *last;     // [nspans] last piece of the cut vertex that ends in the span
+  uint32_t *arr;    // [nspans] arrivals so far of that vertex's pieces
   uint64_t *part;   // [2][W][2] dangling mass, L1 change (2^-60 fixed point)
+  uint32_t nspans;
   uint32_t *stats;
   uint32_t ng, nx;
 };
-
-__device__ __forceinline__ uint32_t pr_nchunks(uint32_t d) { return (d + kChunk - 1) / kChunk; }
-
-// vertex whose in-edge range [rrow[v], rrow[v+1]) holds edge e (e < rrow[n])
-__device__ uint32_t pr_edge_owner(const uint32_t *rrow, uint32_t n, uint32_t e) {
-  uint32_t lo = 0, hi = n;  // rrow[lo] <= e < rrow[hi]
-  while (hi - lo > 1) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    if (rrow[mid] <= e) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
-// One wave, 64 consecutive vertices: lane j brings its vertex's first in-edge
-// `eb` and run length `len` (0 for heavy, empty or out-of-range vertices) and
-// returns the sum of the contributions over that run.
-__device__ __forceinline__ float pr_light_block(const PrArgs &p, const float *cin, uint32_t eb,
-                                                uint32_t len) {
-  return wave_run_gather_sum<kPrSteps>(p.rcol, cin, eb, len);
-}
 
 __device__ __forceinline__ uint64_t q60(double v) { return (uint64_t)(v * 0x1p60); }
 
@@ -2156,85 +2131,47 @@ __device__ double pr_fold(const uint64_t *part, uint32_t parity, int q) {
   return (double)block_sum_u64(acc) * 0x1p-60;
 }
 
-__device__ __forceinline__ uint64_t shfl_up64(uint64_t v, uint32_t d) {
-  const uint32_t lo = __shfl_up((uint32_t)v, d), hi = __shfl_up((uint32_t)(v >> 32), d);
-  return ((uint64_t)hi << 32) | lo;
+// v of another lane by a DPP control, 0 where it has none
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0u, (uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0u, (uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
-
-__device__ __forceinline__ uint64_t wave_incl_scan_u64(uint64_t v) {
-#pragma unroll
-  for (uint32_t d = 1; d < 64; d <<= 1) {
-    const uint64_t up = shfl_up64(v, d);
-    if (lane_id() >= d) v += up;
-  }
+// inclusive wave64 scan, a fixed order of additions
+__device__ __forceinline__ double wave_incl_scan_f64(double v) {
+  v += dpp_f64<0x111, 0xf>(v);
+  v += dpp_f64<0x112, 0xf>(v);
+  v += dpp_f64<0x114, 0xf>(v);
+  v += dpp_f64<0x118, 0xf>(v);
+  v += dpp_f64<0x142, 0xa>(v);
+  v += dpp_f64<0x143, 0xc>(v);
   return v;
 }
-
-// inclusive scan over the workgroup (thread order); *total = workgroup sum
-__device__ uint64_t block_incl_scan_u64(uint64_t v, uint64_t *total) {
-  __shared__ uint64_t wsum[kWg / 64];
-  const uint32_t wv = threadIdx.x >> 6;
-  v = wave_incl_scan_u64(v);
-  if (lane_id() == 63) wsum[wv] = v;
-  __syncthreads();
-  uint64_t off = 0, tot = 0;
-  for (uint32_t k = 0; k < kWg / 64; ++k) {
-    if (k < wv) off += wsum[k];
-    tot += wsum[k];
-  }
-  __syncthreads();
-  *total = tot;
-  return v + off;
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, lane), hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double ld_f64(const double *q) {
+  return __builtin_bit_cast(double, ld_u64(reinterpret_cast<const uint64_t *>(q)));
 }
 
-__device__ __forceinline__ uint32_t wg_range(uint32_t count, uint32_t w) {
-  return (uint32_t)((uint64_t)count * w / gridDim.x);
-}
+// sources of four consecutive in-edges; rcol is only 4-byte aligned there
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-// Sum of the per-workgroup totals of a unit space (one wave).
-__device__ uint64_t pr_space_total(const uint64_t *wtot) {
-  uint64_t acc = 0;
-  for (uint32_t j = lane_id(); j < gridDim.x; j += 64) acc += wtot[j];
-  return shfl64(wave_incl_scan_u64(acc), 63);
-}
-
-// First unit whose exclusive weight prefix is >= t, in a unit space cut into
-// per-workgroup ranges (pre = inclusive prefix inside each range, wtot = range
-// totals).  Weights are >= 1, so the prefix is strictly increasing.  One wave.
-__device__ uint32_t pr_split(const uint64_t *pre, const uint64_t *wtot, uint32_t count, uint64_t t) {
-  if (t == 0) return 0;
-  const uint32_t W = gridDim.x;
-  uint64_t before = 0;  // total of the ranges before g
-  uint32_t g = W;
-  for (uint32_t base = 0; base < W; base += 64) {
-    const uint32_t j = base + lane_id();
-    const uint64_t v = j < W ? wtot[j] : 0;
-    const uint64_t inc = wave_incl_scan_u64(v) + before;
-    const uint64_t hit = ballot(j < W && inc >= t);
-    if (hit) {
-      const uint32_t l = (uint32_t)__builtin_ctzll(hit);
-      g = base + l;
-      before = shfl64(inc - v, l);
-      break;
-    }
-    before = shfl64(inc, 63);
-  }
-  if (g >= W) return count;
-  uint32_t lo = wg_range(count, g), hi = wg_range(count, g + 1) - 1;
-  while (lo < hi) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    if (before + pre[mid] >= t) hi = mid; else lo = mid + 1;
-  }
-  return lo + 1;
-}
-
-template <int KIND>
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k_pagerank(ArenaView a, PrArgs p) {
+template <int KIND, int QUADS>
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(QUADS > 2 ? 4 : 8)))
+k_pagerank(ArenaView a, PrArgs p) {
+  constexpr uint32_t S = 256 * QUADS;
+  __shared__ __align__(16) double pre_s[kWg / 64][S + 2];
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   const float inv_n = 1.0f / (float)p.n;
-  const uint32_t m = p.rrow[p.n];
-  const uint32_t nblk = (p.n + 63) / 64;
+  const uint32_t m = p.rrow[p.n], lane = lane_id();
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double *pre = pre_s[wv];
   // iteration 0 state: x = 1/n, contributions and dangling mass of x
   uint64_t dang = 0;
   for (uint32_t v = gtid(); v < p.n; v += gthreads()) {
@@ -2243,83 +2180,20 @@ __global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k
     p.contrib[v] = d ? inv_n / (float)d : 0.f;
     if (!d) dang += q60(inv_n);
   }
-  for (uint32_t i = gtid(); i < p.nslots; i += gthreads()) p.harr[i] = 0;
-  // Work units and their weights (a cost model in memory round trips): light
-  // blocks of 64 vertices (1.5 x light in-edges + 256) and chunk slots (the
-  // chunk's in-edges + 256, weight 1 for an unused slot).  Each workgroup prefix-sums a contiguous
-  // range of each space; after the barrier every wave takes the units whose
-  // exclusive prefix falls in its equal share of the total.
-  __shared__ uint64_t s_w[kWg];
-  {
-    const uint32_t b0 = wg_range(nblk, blockIdx.x), b1 = wg_range(nblk, blockIdx.x + 1);
-    uint64_t carry = 0;
-    for (uint32_t cb = b0; cb < b1; cb += kWg) {
-      const uint32_t nb = min((uint32_t)kWg, b1 - cb);
-      for (uint32_t k = threadIdx.x >> 6; k < nb; k += kWg / 64) {
-        const uint32_t v = (cb + k) * 64 + lane_id();
-        uint32_t len = 0;
-        if (v < p.n) {
-          const uint32_t d = p.rrow[v + 1] - p.rrow[v];
-          len = d < kHeavy ? d : 0u;
-        }
-        // cost model: a pass of 512 positions costs two memory round trips, as
-        // does a 512-edge pass of a chunk (below), plus the shuffles of the
-        // segmented sums (half as much again)
-        const uint32_t tot = wave_sum(len);
-        if (lane_id() == 0) s_w[k] = (uint64_t)tot + tot / 2 + 256;
-      }
-      __syncthreads();
-      uint64_t tot;
-      const uint64_t inc = block_incl_scan_u64(threadIdx.x < nb ? s_w[threadIdx.x] : 0, &tot);
-      if (threadIdx.x < nb) p.lpre[cb + threadIdx.x] = carry + inc;
-      carry += tot;
+  for (uint32_t i = gtid(); i <= p.nspans; i += gthreads()) {
+    // vertices whose end (position rrow[v + 1] + v) is before the span
+    const uint64_t at = (uint64_t)i * S;
+    uint32_t lo = 0, hi = p.n;
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if ((uint64_t)p.rrow[mid + 1] + mid < at) lo = mid + 1; else hi = mid;
     }
-    if (threadIdx.x == 0) p.wtot[blockIdx.x] = carry;
-  }
-  {
-    // chunk slot owners: slot i belongs to chunk c of the vertex v holding edge
-    // i*kHeavy when v is heavy and c = i - ceil(rrow[v]/kHeavy) < chunks(v)
-    const uint32_t s0 = wg_range(p.nslots, blockIdx.x), s1 = wg_range(p.nslots, blockIdx.x + 1);
-    uint64_t carry = 0;
-    for (uint32_t cs = s0; cs < s1; cs += kWg) {
-      const uint32_t i = cs + threadIdx.x;
-      uint64_t wgt = 0;
-      if (i < s1) {
-        uint64_t ent = ~0ull;
-        wgt = 1;
-        const uint64_t e = (uint64_t)i * kHeavy;
-        if (e < m) {
-          const uint32_t v = pr_edge_owner(p.rrow, p.n, (uint32_t)e);
-          const uint32_t rb = p.rrow[v], d = p.rrow[v + 1] - rb;
-          const uint32_t first = (rb + kHeavy - 1) / kHeavy;
-          if (d >= kHeavy && i >= first && i - first < pr_nchunks(d)) {
-            const uint32_t c = i - first;
-            ent = v | ((uint64_t)c << 32);
-            wgt = (uint64_t)min(kChunk, d - c * kChunk) + 256;
-          }
-        }
-        p.hent[i] = ent;
-      }
-      uint64_t tot;
-      const uint64_t inc = block_incl_scan_u64(wgt, &tot);
-      if (i < s1) p.spre[i] = carry + inc;
-      carry += tot;
-    }
-    if (threadIdx.x == 0) p.wtot[gridDim.x + blockIdx.x] = carry;
+    p.first[i] = lo;
+    if (i < p.nspans) p.arr[i] = 0;
   }
   dang = block_sum_u64(dang);
   if (threadIdx.x == 0) p.part[((size_t)0 * gridDim.x + blockIdx.x) * 2 + 0] = dang;
   if (gb.sync<KIND>()) return;
-  // this wave's share of each unit space
-  uint32_t b_lo, b_hi, s_lo, s_hi;
-  {
-    const uint64_t W = gwaves(), w = gwave();
-    const uint64_t TL = pr_space_total(p.wtot), TS = pr_space_total(p.wtot + gridDim.x);
-    b_lo = pr_split(p.lpre, p.wtot, nblk, TL * w / W);
-    b_hi = pr_split(p.lpre, p.wtot, nblk, TL * (w + 1) / W);
-    s_lo = pr_split(p.spre, p.wtot + gridDim.x, p.nslots, TS * w / W);
-    s_hi = pr_split(p.spre, p.wtot + gridDim.x, p.nslots, TS * (w + 1) / W);
-  }
   int it = 0;
   double l1 = 0;
   uint32_t cur = 0;
@@ -2332,75 +2206,111 @@ __global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k
     const float base = (float)((1.0 - (double)p.alpha) / p.n + (double)p.alpha * D / p.n);
     uint64_t l1q = 0, dq = 0;  // this thread's share of the L1 change and dangling mass
     // y, L1 term, next contribution and dangling term of vertex v from its sum
-    auto finalize = [&](uint32_t v, float sum) {
+    auto finalize = [&](uint32_t v, float sum, float xv, uint32_t d) {
       const float y = base + p.alpha * sum;
-      l1q += q60(fabs((double)y - (double)xin[v]));
+      l1q += q60(fabs((double)y - (double)xv));
       xout[v] = y;
-      const uint32_t d = p.row[v + 1] - p.row[v];
       cout[v] = d ? y / (float)d : 0.f;
       if (!d) dq += q60(y);
     };
-    // heavy chunks, fixed order inside each chunk; the last chunk of a vertex
-    // to finish finalizes it
-    for (uint32_t sb = s_lo; sb < s_hi; sb += 64) {
-      const uint32_t i = sb + lane_id();
-      const uint64_t mine = i < s_hi ? p.hent[i] : ~0ull;
-      uint64_t used = ballot(mine != ~0ull);
-      while (used) {
-        const uint32_t l = (uint32_t)__builtin_ctzll(used);
-        used &= used - 1;
-        const uint64_t ent = shfl64(mine, l);
-        const uint32_t v = (uint32_t)ent, c = (uint32_t)(ent >> 32);
-        const uint32_t rb = p.rrow[v], re = p.rrow[v + 1];
-        const uint32_t eb = rb + c * kChunk, ee = min(re, eb + kChunk);
-        // passes of kPrHeavySteps x 64 edges: the column loads, then the
-        // gathers, in flight per lane; the lane's sum keeps edge order
-        float sum = 0.f;
-        for (uint32_t e = eb + lane_id(); e < ee; e += kPrHeavySteps * 64) {
-          uint32_t cs[kPrHeavySteps];
+    for (uint32_t i = blockIdx.x * (kWg / 64) + wv; i < p.nspans; i += gridDim.x * (kWg / 64)) {
+      const uint32_t v0 = p.first[i], v1 = p.first[i + 1];
+      const uint32_t e0 = (uint32_t)((uint64_t)i * S - v0);
+      const uint64_t e1w = (uint64_t)(i + 1) * S - v1;
+      const uint32_t e1 = e1w < m ? (uint32_t)e1w : m, cnt = e1 - e0;
+      // the first 64 vertices' state is loaded beside the gathers
+      uint32_t v = v0 + lane, rb = 0, re = 0, d = 0;
+      float xv = 0.f;
+      if (v < v1) { rb = p.rrow[v]; re = p.rrow[v + 1]; d = p.row[v + 1] - p.row[v]; xv = xin[v]; }
+      float g[QUADS][4];
+      {
+        u32x4_any c[QUADS];
 #pragma unroll
-          for (int u = 0; u < kPrHeavySteps; ++u) cs[u] = e + 64 * u < ee ? p.rcol[e + 64 * u] : 0xFFFFFFFFu;
-          float gs[kPrHeavySteps];
-#pragma unroll
-          for (int u = 0; u < kPrHeavySteps; ++u) gs[u] = cs[u] != 0xFFFFFFFFu ? cin[cs[u]] : 0.f;
-#pragma unroll
-          for (int u = 0; u < kPrHeavySteps; ++u) sum += gs[u];
+        for (int q = 0; q < QUADS; ++q) {
+          const uint32_t at = q * 256 + 4 * lane;
+          c[q] = u32x4_any{~0u, ~0u, ~0u, ~0u};
+          if (at + 4 <= cnt) {
+            c[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(p.rcol + e0 + at));
+          } else if (at < cnt) {
+            c[q].x = p.rcol[e0 + at];
+            if (at + 1 < cnt) c[q].y = p.rcol[e0 + at + 1];
+            if (at + 2 < cnt) c[q].z = p.rcol[e0 + at + 2];
+          }
         }
-        for (int k = 32; k >= 1; k >>= 1) sum += __shfl_xor(sum, k);
-        if (lane_id() == 0) {
-          // publish the chunk sum (agent scope: other XCDs read it), then arrive
-          __hip_atomic_store(p.hsum + sb + l, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          wait_stores();
-          const uint32_t first = (rb + kHeavy - 1) / kHeavy, nc = pr_nchunks(re - rb);
-          const uint32_t old = add_relaxed(p.harr + first, 1u);
-          if (old + 1u == (uint32_t)(it + 1) * nc) {
-            float t = 0.f;
-            for (uint32_t cc = 0; cc < nc && first + cc < p.nslots; ++cc)
-              t += __hip_atomic_load(p.hsum + first + cc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            finalize(v, t);
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) g[q][k] = c[q][k] != ~0u ? cin[c[q][k]] : 0.f;
+      }
+      double run = 0.0;
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q) {
+        const double d1 = (double)g[q][0], d2 = d1 + (double)g[q][1], d3 = d2 + (double)g[q][2], d4 = d3 + (double)g[q][3];
+        const double inc = wave_incl_scan_f64(d4);
+        // the lanes before this one: the scan's value one lane down
+        double ex = dpp_f64<0x138, 0xf>(inc);  // wave_shr:1, 0 into lane 0
+        ex += run;
+        run += readlane_f64(inc, 63);
+        double *o = pre + q * 256 + 4 * lane;
+        o[0] = ex;
+        o[1] = ex + d1;
+        o[2] = ex + d2;
+        o[3] = ex + d3;
+      }
+      if (lane == 0) pre[S] = run;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      double cut = 0.0;  // of v0, if it began before the span
+      while (v0 < v1) {
+        if (v < v1) {
+          const double sum = pre[re - e0] - pre[rb > e0 ? rb - e0 : 0u];
+          if (rb < e0) cut = sum;
+          else finalize(v, (float)sum, xv, d);
+        }
+        if (v - lane + 64 >= v1) break;
+        v += 64;
+        if (v < v1) { rb = p.rrow[v]; re = p.rrow[v + 1]; d = p.row[v + 1] - p.row[v]; xv = xin[v]; }
+      }
+      // pieces of cut vertices: lane 0 the last one of v0, lane 1 that of v1, which
+      // runs on; published, then arrived
+      const uint32_t tb = v1 < p.n ? p.rrow[v1] : m, te = v1 < p.n ? p.rrow[v1 + 1] : m;
+      const uint32_t hb = v0 < p.n ? p.rrow[v0] : m;
+      const bool ends = v0 < v1 && hb < e0, runs = v1 < p.n && tb < e1;
+      if (ends | runs) {
+        const double runs_sum = runs ? run - pre[tb > e0 ? tb - e0 : 0u] : 0.0;
+        uint32_t from = 0, to = 0;
+        bool mine = false;
+        if (lane == 0 && ends) {
+          __hip_atomic_store(reinterpret_cast<uint64_t *>(p.last + i), __builtin_bit_cast(uint64_t, cut), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+          from = (uint32_t)(((uint64_t)hb + v0) / S);
+          to = i;
+          mine = true;
+        }
+        if (lane == 1 && runs) {
+          __hip_atomic_store(reinterpret_cast<uint64_t *>(p.tail + i), __builtin_bit_cast(uint64_t, runs_sum),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          from = (uint32_t)(((uint64_t)tb + v1) / S);
+          to = (uint32_t)(((uint64_t)te + v1) / S);
+          mine = true;
+        }
+        wait_stores();
+        bool done = false;
+        if (mine) done = add_relaxed(p.arr + to, 1u) + 1u == (uint32_t)(it + 1) * (to - from + 1);
+        for (uint64_t todo = ballot(done); todo; todo &= todo - 1) {
+          const uint32_t l = (uint32_t)__builtin_ctzll(todo), f = __shfl(from, (int)l), t = __shfl(to, (int)l);
+          double sum = 0.0;
+          for (uint32_t k = f; k < t; k += 64) {
+            const double piece = k + lane < t ? ld_f64(p.tail + k + lane) : 0.0;
+            sum += readlane_f64(wave_incl_scan_f64(piece), 63);
+          }
+          if (lane == 0) {
+            sum += ld_f64(p.last + t);
+            const uint32_t cv = l == 0 ? v0 : v1;
+            finalize(cv, (float)sum, xin[cv], p.row[cv + 1] - p.row[cv]);
           }
         }
       }
-    }
-    // light blocks, one wave per block of 64 vertices (the next block's
-    // offsets are loaded while this one is summed)
-    uint32_t nb_eb = 0, nb_ee = 0;
-    if (b_lo < b_hi) {
-      const uint32_t v = b_lo * 64 + lane_id();
-      if (v < p.n) { nb_eb = p.rrow[v]; nb_ee = p.rrow[v + 1]; }
-    }
-    for (uint32_t blk = b_lo; blk < b_hi; ++blk) {
-      const uint32_t v = blk * 64 + lane_id();
-      const bool valid = v < p.n;
-      const uint32_t eb = nb_eb, din = nb_ee - nb_eb;
-      if (blk + 1 < b_hi) {
-        const uint32_t vn = v + 64;
-        nb_eb = vn < p.n ? p.rrow[vn] : 0u;
-        nb_ee = vn < p.n ? p.rrow[vn + 1] : 0u;
-      }
-      const bool light = din < kHeavy;
-      const float sum = pr_light_block(p, cin, eb, light ? din : 0u);
-      if (valid && light) finalize(v, sum);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read before the next span's sums
     }
     l1q = block_sum_u64(l1q);
     dq = block_sum_u64(dq);
@@ -2421,6 +2331,11 @@ __global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k
     p.stats[1] = __float_as_uint(l1f);
   }
 }
+
+template <int KIND>
+constexpr auto k_pagerank_large = k_pagerank<KIND, kPrQuads>;
+template <int KIND>
+constexpr auto k_pagerank_small = k_pagerank<KIND, 1>;
 
 #define HS_KIND_SWITCH(KERNEL, kind)                                            \
   [&]() -> const void * {                                                       \
@@ -2664,16 +2579,17 @@ int hs_sssp(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const u
 }
 
 // ---------------------------------------------------------------- PageRank
-// heavy chunk slots: ceil(m / kHeavy) (see PrArgs)
-static uint64_t pr_slots(uint64_t m) { return (m + kHeavy - 1) / kHeavy; }
+static bool pr_large(uint32_t n, uint64_t m) { return n + m >= kPrLargeFrom; }
+static uint64_t pr_spans(uint32_t n, uint64_t m) {
+  const uint64_t S = 256ull * (pr_large(n, m) ? kPrQuads : 1);
+  return (n + m + S - 1) / S;
+}
 
 int hs_pagerank_work_size(uint32_t n, uint64_t m, uint64_t *bytes) {
   if (!bytes) return HS_ERR_INVALID;
-  const uint64_t hc = pr_slots(m) + 1, nblk = (n + 63ull) / 64;
+  const uint64_t ns = std::max(pr_spans(n, m), (std::min(n + m, kPrLargeFrom) + 255) / 256) + 1;  // grows with n and m
   *bytes = align256(sizeof(float) * 2ull * n) * 2 + align256(sizeof(uint64_t) * 2 * 2 * 4096) +
-           align256(sizeof(uint64_t) * hc) * 2 + align256(sizeof(float) * hc) +
-           align256(sizeof(uint32_t) * hc) + align256(sizeof(uint64_t) * nblk) +
-           align256(sizeof(uint64_t) * 2 * 4096);
+           align256(sizeof(uint32_t) * ns) * 2 + align256(sizeof(double) * ns) * 2;
   return HS_OK;
 }
 
@@ -2684,9 +2600,13 @@ int hs_pagerank_f32(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row,
   if (!ar || !d_row || !d_rrow || (m && !d_rcol) || !d_rank || !d_work || n == 0 || !(alpha > 0.f) ||
       !(alpha < 1.f) || max_iter < 1 || m > 0xFFFFFFFFull)
     return HS_ERR_INVALID;
-  const void *k = HS_KIND_SWITCH(k_pagerank, kind);
+  const void *k = pr_large(n, m) ? HS_KIND_SWITCH(k_pagerank_large, kind) : HS_KIND_SWITCH(k_pagerank_small, kind);
   if (!k) return HS_ERR_INVALID;
-  const int g = grid_for(k, ar, num_wgs, 4);  // 4 WGs/CU: latency-bound gathers
+  // 4 WGs/CU (what the running sums in LDS leave room for); larger requests are
+  // served with those, up to 8 per CU
+  const int cus = hs_host::device_cus();
+  if (num_wgs > 8 * cus) return HS_ERR_RESIDENCY;
+  const int g = grid_for(k, ar, num_wgs > 4 * cus ? std::min(4 * cus, hs_host::default_grid(k, kWg, 4)) : num_wgs, 4);
   if (g < 0 || g > 4096) return HS_ERR_RESIDENCY;
   hipStream_t s = (hipStream_t)stream;
   int rc = hs_host::prepare_barrier(ar, kind, s);
@@ -2694,18 +2614,15 @@ int hs_pagerank_f32(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row,
   PrArgs p{};
   p.n = n; p.row = d_row; p.rrow = d_rrow; p.rcol = d_rcol; p.alpha = alpha; p.tol = tol;
   p.max_iter = max_iter; p.rank = d_rank;
-  const uint64_t hc = pr_slots(m) + 1;
+  p.nspans = (uint32_t)pr_spans(n, m);
   char *w = (char *)d_work;
   p.x = (float *)w; w += align256(sizeof(float) * 2ull * n);
   p.contrib = (float *)w; w += align256(sizeof(float) * 2ull * n);
   p.part = (uint64_t *)w; w += align256(sizeof(uint64_t) * 2 * 2 * 4096);
-  p.hent = (uint64_t *)w; w += align256(sizeof(uint64_t) * hc);
-  p.spre = (uint64_t *)w; w += align256(sizeof(uint64_t) * hc);
-  p.hsum = (float *)w; w += align256(sizeof(float) * hc);
-  p.harr = (uint32_t *)w; w += align256(sizeof(uint32_t) * hc);
-  p.lpre = (uint64_t *)w; w += align256(sizeof(uint64_t) * ((n + 63ull) / 64));
-  p.wtot = (uint64_t *)w;
-  p.nslots = (uint32_t)pr_slots(m);
+  p.first = (uint32_t *)w; w += align256(sizeof(uint32_t) * (p.nspans + 1ull));
+  p.arr = (uint32_t *)w; w += align256(sizeof(uint32_t) * (uint64_t)p.nspans);
+  p.tail = (double *)w; w += align256(sizeof(double) * (uint64_t)p.nspans);
+  p.last = (double *)w;
   p.stats = d_stats;
   p.ng = (uint32_t)ar->view.num_groups;
   p.nx = (uint32_t)hs_host::xcd_groups(g);
