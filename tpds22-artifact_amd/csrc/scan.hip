@@ -1,29 +1,34 @@
-// scan.hip -- persistent multi-phase u32 prefix sum with grid barriers.
+// scan.hip -- persistent u32 prefix sum with a grid barrier.
 //
 // Replaces gpu_prescan / gpu_add_block_sums / sum_scan_blelloch
 // (scan/scan_gsrb.cu:440-804).  The reference runs a padded-LDS Blelloch scan of
 // 64 elements per 32-thread block, a barrier per level, and two more host
 // launches, and is correct only up to 64^3 elements.  Here one co-resident grid
-// processes the input in rounds sized to stay resident in the Infinity Cache:
-//   phase 1  each workgroup sums its contiguous chunk of the round (one HBM read)
-//   barrier  (any hs_barrier_kind)
-//   phase 2  each workgroup folds the partials before it (its carry) and the
-//            round total
-//   phase 3  each workgroup re-reads its chunk (Infinity-Cache hit), scans it
-//            tile by tile (16 elements per thread, DPP wave scan, LDS block scan)
-//            and writes the result with the carry.
-// Partials are double-buffered by round parity, so one barrier per round
-// suffices.  uint32 wrap arithmetic: bit-exact for any grid and round size.
+// processes the input in rounds of what its registers hold, so that every element
+// is read once and written once: each workgroup loads a tile (up to 64 elements
+// per thread), scans it in place, publishes its sum and takes the sums of the
+// workgroups before it in the round and of the rounds before.  A workgroup
+// publishes a round only when it has read the whole round before, so two words per
+// workgroup suffice and nobody is more than a round ahead.  The one grid barrier
+// (any hs_barrier_kind) stands after the first round's words, which are all there
+// behind it, and clears the second's: an input of one round waits once (1M elements:
+// 12.1 us with the barrier before the first tile and the words polled, 9.9 so).
+// Bound by HBM: 2^28 elements 0.57 ms when each round was summed, crossed a barrier
+// and was read a second time from the Infinity Cache, 0.40 ms so (5.4 TB/s; a copy
+// of that size reaches 5.2); 100M 214 -> 157 us, 30M 64 -> 49, 13M 30 -> 24, 8M
+// 21 -> 18, 4M and less as before (12 us, 10 from 2M down).
+// uint32 wrap arithmetic: bit-exact for any grid and round size.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
 
 #include "hs_internal.hpp"
+#include "hs_wave.hpp"
 
 using namespace hs;
 
-// Partials of hs_scan_u32_noalloc: 2 words per workgroup (double-buffered by
-// round parity), for grids of up to kNoAllocMaxWgs workgroups (32 KiB).  Each
+// Words of hs_scan_u32_noalloc: 2 of 32 bits per workgroup asked for, as
+// hs_scan_scratch_size says, for up to kNoAllocMaxWgs workgroups (32 KiB).  Each
 // device holds its own copy until the process ends; host code reaches it only
 // through the address hipGetSymbolAddress returns for the current device.
 constexpr int kNoAllocMaxWgs = 4096;
@@ -31,285 +36,151 @@ static __device__ __align__(256) uint32_t scratch[2 * kNoAllocMaxWgs];
 
 namespace {
 
-constexpr int kWg = 256;
-constexpr int kItems = 16;                 // elements per thread per tile
-constexpr int kTile = kWg * kItems;        // 4096 elements
+constexpr int kWg = 1024;   // threads of a workgroup, one per CU
+constexpr int kWaves = kWg / 64;
+constexpr int kSpan = 256;  // elements of a wave's segment: 4 per lane, 1 KiB per instruction
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// inclusive wave64 scan (DPP row_shr + row_bcast)
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xa, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xc, 0xf, false);
-  return v;
-}
-
-// exclusive block scan of one value per thread; returns the exclusive prefix and
-// the block total
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t &total) {
-  __shared__ uint32_t wsum[kWg / 64];
-  const uint32_t inc = wave_incl_scan(v);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  uint32_t before = 0, tot = 0;
-#pragma unroll
-  for (int i = 0; i < kWg / 64; ++i) {
-    const uint32_t s = wsum[i];
-    before += i < w ? s : 0u;
-    tot += s;
-  }
-  __syncthreads();
-  total = tot;
-  return before + inc - v;
-}
-
-__device__ __forceinline__ uint32_t block_sum(uint32_t v) {
-  uint32_t total;
-  block_excl_scan(v, total);
-  return total;
-}
-
-// Each workgroup's chunk of a round is split into 4 contiguous wave
-// sub-chunks, so phase 3 needs no workgroup barrier per tile: a wave scans its
-// own sub-chunk 1024 elements (a wave-tile) at a time, its carry being the
-// chunk carry plus the sums of the waves before it (from phase 1).
-// Wave-tile layout: 4 segments of 256 elements; in segment s lane l holds
-// elements s*256 + 4l .. 4l+3, so every load and store instruction of a wave
-// covers 1 KiB of contiguous memory.  Each segment is one DPP wave scan.
-constexpr int kSeg = 4;
-
-__device__ __forceinline__ void wt_load(const uint32_t *in, uint64_t tile, uint32_t lane,
-                                        uint32_t (&x)[kSeg][4]) {
-  const uint4 *p = reinterpret_cast<const uint4 *>(in + tile) + lane;
-#pragma unroll
-  for (int s = 0; s < kSeg; ++s) {
-    const uint4 v = p[s * 64];
-    x[s][0] = v.x; x[s][1] = v.y; x[s][2] = v.z; x[s][3] = v.w;
-  }
-}
-
-// elements at or beyond `end` read as 0
-__device__ __forceinline__ void wt_load_part(const uint32_t *in, uint64_t tile, uint64_t end, uint32_t lane,
-                                             uint32_t (&x)[kSeg][4]) {
-#pragma unroll
-  for (int s = 0; s < kSeg; ++s)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint64_t i = tile + (uint64_t)s * 256 + 4u * lane + j;
-      x[s][j] = i < end ? in[i] : 0u;
-    }
-}
-
-// scans the wave-tile in place (x becomes the output) and advances run
+// scan of 256 elements (4 per lane) behind the prefix `run`, in place
 template <bool INCLUSIVE>
-__device__ __forceinline__ void wt_scan(uint32_t (&x)[kSeg][4], uint32_t &run) {
+__device__ __forceinline__ void seg_scan(u32x4 &x, uint32_t &run) {
+  const uint32_t v4 = x[0] + x[1] + x[2] + x[3];
+  const uint32_t inc = wave_incl_scan(v4);
+  uint32_t pre = run + inc - v4;
+  run += __builtin_amdgcn_readlane(inc, 63);
 #pragma unroll
-  for (int s = 0; s < kSeg; ++s) {
-    const uint32_t t = x[s][0] + x[s][1] + x[s][2] + x[s][3];
-    const uint32_t inc = wave_incl_scan(t);
-    uint32_t pre = run + inc - t;
-    run += __builtin_amdgcn_readlane(inc, 63);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t v = x[s][j];
-      if (INCLUSIVE) { pre += v; x[s][j] = pre; }
-      else { x[s][j] = pre; pre += v; }
-    }
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t v = x[k];
+    if (INCLUSIVE) { pre += v; x[k] = pre; }
+    else { x[k] = pre; pre += v; }
   }
 }
 
-// output stores are non-temporal (streaming: nothing reads them back in the
-// launch); the input's second read stays a plain load, meant to hit the
-// Infinity Cache the first read filled
-__device__ __forceinline__ void wt_store(uint32_t *out, uint64_t tile, uint32_t lane, const uint32_t (&y)[kSeg][4]) {
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  u32x4 *o = reinterpret_cast<u32x4 *>(out + tile) + lane;
-#pragma unroll
-  for (int s = 0; s < kSeg; ++s) {
-    const u32x4 v = {y[s][0], y[s][1], y[s][2], y[s][3]};
-    __builtin_nontemporal_store(v, o + s * 64);
-  }
+// A wave's part as a buffer: loads at or beyond its size give 0 and stores there are
+// dropped, which cuts the input's end without a second path (two paths to the data
+// registers took twice the registers).  Sizes are multiples of 16 bytes; the offset
+// is the lane's alone, as a scalar offset would be taken off the size.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t part_buffer(const uint32_t *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(p), 0, bytes, 0x00027000);
+}
+constexpr int kStream = 2;  // nt: every element is read once and written once
+
+__device__ __forceinline__ uint64_t ld_word(const uint64_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_word(uint64_t *p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void wt_store_part(uint32_t *out, uint64_t tile, uint64_t end, uint32_t lane,
-                                              const uint32_t (&y)[kSeg][4]) {
-#pragma unroll
-  for (int s = 0; s < kSeg; ++s)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint64_t i = tile + (uint64_t)s * 256 + 4u * lane + j;
-      if (i < end) out[i] = y[s][j];
-    }
-}
-
-__device__ __forceinline__ uint32_t wt_sum(const uint32_t (&x)[kSeg][4]) {
-  uint32_t t = 0;
-#pragma unroll
-  for (int s = 0; s < kSeg; ++s) t += x[s][0] + x[s][1] + x[s][2] + x[s][3];
-  return t;
-}
-
-// per-lane sum of the wave's range [sb, se) (16 x 16 B in flight per lane)
-__device__ __forceinline__ uint32_t range_sum(const uint32_t *in, uint64_t sb, uint64_t se, uint32_t lane) {
-  uint32_t acc = 0;
-  const uint64_t full = sb + (se - sb) / 4 * 4;
-  const uint4 *p4 = reinterpret_cast<const uint4 *>(in + sb);
-  const uint64_t n4 = (full - sb) / 4;
-  uint64_t i = lane;
-  for (; i + 15 * 64 < n4; i += 16 * 64) {
-    uint4 v[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) v[k] = p4[i + k * 64];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) acc += v[k].x + v[k].y + v[k].z + v[k].w;
-  }
-  for (; i < n4; i += 64) {
-    const uint4 v = p4[i];
-    acc += v.x + v.y + v.z + v.w;
-  }
-  for (uint64_t j = full + lane; j < se; j += 64) acc += in[j];
-  return acc;
-}
-
-// Rounds are software-pipelined: while a wave scans and writes its sub-chunk
-// of round r (re-read from the Infinity Cache), it also reads and sums its
-// sub-chunk of round r+1 (from HBM), so reads and writes stream together and
-// each round needs one grid barrier.  Partials are double-buffered by round
-// parity.
-template <int KIND, bool INCLUSIVE>
-__global__ void __launch_bounds__(kWg) k_scan_u32(ArenaView a, const uint32_t *__restrict__ in,
-                                                 uint32_t *__restrict__ out, uint64_t n,
-                                                 uint32_t *partials, uint64_t round_elems,
-                                                 uint32_t ngroups, uint32_t nxcd) {
-  constexpr int kWaves = kWg / 64;
-  constexpr int kWaveTile = 256 * kSeg;  // 1024 elements
-  __shared__ uint32_t s_wave[kWaves];
+// Workgroup w's tile of round r is [(r W + w) TILE, +TILE), a wave's part of it SEGS
+// segments.  words[2][W]: (round + 1) << 32 | the workgroup's sum, by round parity.
+template <int KIND, int SEGS, bool INCLUSIVE>
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(4)))
+k_scan_u32(ArenaView a, const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *words, uint32_t ngroups, uint32_t nxcd) {
+  constexpr uint32_t kPart = SEGS * kSpan, kTile = kWaves * kPart;
+  __shared__ uint32_t s_wave[kWaves], s_carry[kWaves], s_before[kWaves];
+  __shared__ int s_bad;
   GridBarrier gb;
   gb.init(a, KIND, ngroups, nxcd);
-  const uint32_t W = gridDim.x, w = blockIdx.x;
-  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint64_t chunk = round_elems / W;  // multiple of kTile
-  const uint64_t sub = chunk / kWaves;     // multiple of kWaveTile
-  const uint64_t off = (uint64_t)w * chunk + wv * sub;  // this wave's offset inside a round
-  auto bounds = [&](uint64_t rb, uint64_t &sb, uint64_t &se) {
-    const uint64_t re = rb + round_elems < n ? rb + round_elems : n;
-    sb = rb + off;
-    se = sb + sub;
-    if (sb > re) sb = re;
-    if (se > re) se = re;
-  };
-  // publish this workgroup's total of one round (from the per-wave sums)
-  auto publish = [&](uint32_t wave_sum, uint32_t *part, uint32_t &wave_before) {
-    if (lane == 0) s_wave[wv] = wave_sum;
-    __syncthreads();
-    uint32_t before = 0, total = 0;
-#pragma unroll
-    for (int k = 0; k < kWaves; ++k) {
-      before += k < (int)wv ? s_wave[k] : 0u;
-      total += s_wave[k];
-    }
-    wave_before = before;
-    if (threadIdx.x == 0) part[w] = total;
-    __syncthreads();  // s_wave is rewritten by the next publish
-  };
-  uint32_t carry = 0;  // sum of all previous rounds
-  uint64_t sb, se;
-  bounds(0, sb, se);
-  uint32_t wave_before;
-  publish(__builtin_amdgcn_readlane(wave_incl_scan(range_sum(in, sb, se, lane)), 63), partials, wave_before);
+  const uint32_t W = gridDim.x, w = blockIdx.x, lane = threadIdx.x & 63;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (threadIdx.x == 0) s_bad = 0;
+  const uint64_t n4 = n & ~3ull;
+  uint32_t carry = 0;  // sum of all rounds before
   uint32_t r = 0;
-  for (uint64_t rb = 0; rb < n; rb += round_elems, ++r) {
-    if (gb.sync<KIND>()) return;
-    const uint32_t *part = partials + (r & 1u) * W;
-    uint32_t before = 0, all = 0;
-    for (uint32_t j = threadIdx.x; j < W; j += kWg) {
-      const uint32_t v = part[j];
-      all += v;
-      before += j < w ? v : 0u;
+  for (uint64_t tile = (uint64_t)w * kTile;; tile += (uint64_t)W * kTile, ++r) {
+    const uint64_t base = tile + (uint64_t)wv * kPart;
+    const uint64_t left = base < n4 ? (n4 - base) * sizeof(uint32_t) : 0;
+    const uint32_t bytes = left < kPart * sizeof(uint32_t) ? (uint32_t)left : kPart * (uint32_t)sizeof(uint32_t);
+    uint32_t run = 0;
+    u32x4 x[SEGS];
+    {
+      const auto b = part_buffer(in + base, bytes);
+#pragma unroll
+      for (int q = 0; q < SEGS; ++q) x[q] = __builtin_amdgcn_raw_buffer_load_b128(b, lane * 16 + q * 1024, 0, kStream);
     }
-    before = block_sum(before);
-    all = block_sum(all);
-    uint32_t run = carry + before + wave_before;
-    const bool next = rb + round_elems < n;
-    uint64_t nb = 0, ne = 0;  // this wave's range in round r+1
-    if (next) bounds(rb + round_elems, nb, ne);
-    uint32_t nacc = 0;        // per-lane sum of [nb, ne)
-    const uint64_t nf = (se - sb) / kWaveTile;  // full tiles of round r
-    const uint64_t nfn = (ne - nb) / kWaveTile;  // full tiles of round r+1 (<= nf)
-    uint64_t t = 0;
-    // both rounds' tiles full: one tile of each in flight ahead
-    if (nfn > 0) {
-      uint32_t x[kSeg][4], y[kSeg][4];
-      wt_load(in, sb, lane, x);
-      wt_load(in, nb, lane, y);
-      for (; t + 1 < nfn; ++t) {
-        uint32_t x2[kSeg][4], y2[kSeg][4];
-        wt_load(in, sb + (t + 1) * kWaveTile, lane, x2);
-        wt_load(in, nb + (t + 1) * kWaveTile, lane, y2);
-        nacc += wt_sum(y);
-        wt_scan<INCLUSIVE>(x, run);
-        wt_store(out, sb + t * kWaveTile, lane, x);
 #pragma unroll
-        for (int q = 0; q < kSeg; ++q)
+    for (int q = 0; q < SEGS; ++q) {
+      seg_scan<INCLUSIVE>(x[q], run);
+      // keeps the scanned values and not their parts, whose sums would otherwise be
+      // put off to the stores: 16 more registers, and spills
+      asm volatile("" : "+v"(x[q]));
+    }
+    // the whole round before, then this round's word, then the ones before it
+    uint32_t got = 0;
+    if (W > 1 && r > 0 && threadIdx.x < W) {
+      const uint64_t *q = words + ((r - 1) & 1u) * W + threadIdx.x;
+      uint64_t v = 0;
+      if (spin_until(a, [&] { v = ld_word(q); return (uint32_t)(v >> 32) == r; }, 1)) s_bad = 1;
+      got = (uint32_t)v;
+    }
+    got = __builtin_amdgcn_readlane(wave_incl_scan(got), 63);
+    if (lane == 0) { s_wave[wv] = run; s_carry[wv] = got; }
+    __syncthreads();
+    uint32_t wave_before = 0, agg = 0;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) { x[q][j] = x2[q][j]; y[q][j] = y2[q][j]; }
+    for (uint32_t k = 0; k < kWaves; ++k) {
+      const uint32_t s = s_wave[k];
+      wave_before += k < wv ? s : 0u;
+      agg += s;
+      carry += s_carry[k];
+    }
+    if (W > 1 && threadIdx.x == 0) st_word(words + (r & 1u) * W + w, ((uint64_t)(r + 1) << 32) | agg);
+    if (r == 0) {
+      // the first round's words and the cleared ones of the second
+      if (W > 1 && threadIdx.x == 0) st_word(words + W + w, 0);
+      if (gb.sync<KIND>()) return;
+    }
+    if (tile >= n) return;  // only in the last round, whose later words nobody needs
+    got = 0;
+    if (threadIdx.x < w) {
+      const uint64_t *q = words + (r & 1u) * W + threadIdx.x;
+      uint64_t v = 0;
+      if (spin_until(a, [&] { v = ld_word(q); return (uint32_t)(v >> 32) == r + 1; }, 1)) s_bad = 1;
+      got = (uint32_t)v;
+    }
+    got = __builtin_amdgcn_readlane(wave_incl_scan(got), 63);
+    if (lane == 0) s_before[wv] = got;
+    __syncthreads();
+    if (s_bad) return;
+    uint32_t add = carry + wave_before;
+#pragma unroll
+    for (uint32_t k = 0; k < kWaves; ++k) add += s_before[k];
+    if (W == 1) carry += agg;
+    const auto b = part_buffer(out + base, bytes);
+#pragma unroll
+    for (int q = 0; q < SEGS; ++q) __builtin_amdgcn_raw_buffer_store_b128(x[q] + add, b, lane * 16 + q * 1024, 0, kStream);
+    // the one to three elements after the last whole four
+    if (n4 < n && n4 - tile < kTile && threadIdx.x == 0) {
+      uint32_t sum = add + agg;
+      for (uint64_t i = n4; i < n; ++i) {
+        const uint32_t v = in[i];
+        out[i] = INCLUSIVE ? sum + v : sum;
+        sum += v;
       }
-      nacc += wt_sum(y);
-      wt_scan<INCLUSIVE>(x, run);
-      wt_store(out, sb + t * kWaveTile, lane, x);
-      ++t;
     }
-    // remaining full tiles of round r, one ahead
-    if (t < nf) {
-      uint32_t x[kSeg][4];
-      wt_load(in, sb + t * kWaveTile, lane, x);
-      for (; t + 1 < nf; ++t) {
-        uint32_t x2[kSeg][4];
-        wt_load(in, sb + (t + 1) * kWaveTile, lane, x2);
-        wt_scan<INCLUSIVE>(x, run);
-        wt_store(out, sb + t * kWaveTile, lane, x);
-#pragma unroll
-        for (int q = 0; q < kSeg; ++q)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) x[q][j] = x2[q][j];
-      }
-      wt_scan<INCLUSIVE>(x, run);
-      wt_store(out, sb + t * kWaveTile, lane, x);
-      ++t;
-    }
-    // partial last tile of round r (only in the last round)
-    if (sb + nf * kWaveTile < se) {
-      uint32_t x[kSeg][4];
-      wt_load_part(in, sb + nf * kWaveTile, se, lane, x);
-      wt_scan<INCLUSIVE>(x, run);
-      wt_store_part(out, sb + nf * kWaveTile, se, lane, x);
-    }
-    if (!next) break;
-    // the rest of round r+1 (beyond its full tiles overlapped above)
-    nacc += range_sum(in, nb + nfn * kWaveTile, ne, lane);
-    carry += all;
-    sb = nb;
-    se = ne;
-    publish(__builtin_amdgcn_readlane(wave_incl_scan(nacc), 63), partials + ((r + 1) & 1u) * W, wave_before);
+    if (tile + (uint64_t)(W - w) * kTile >= n) return;  // this was the last round
   }
 }
 
-template <bool INC>
+template <int SEGS, bool INC>
 const void *scan_kernel(int kind) {
   switch (kind) {
-    case HS_BAR_FLAT: return (const void *)k_scan_u32<HS_BAR_FLAT, INC>;
-    case HS_BAR_TWO_LEVEL: return (const void *)k_scan_u32<HS_BAR_TWO_LEVEL, INC>;
-    case HS_BAR_XCD: return (const void *)k_scan_u32<HS_BAR_XCD, INC>;
-    case HS_BAR_XCD_FLAT_RELEASE: return (const void *)k_scan_u32<HS_BAR_XCD_FLAT_RELEASE, INC>;
-    case HS_BAR_TREE: return (const void *)k_scan_u32<HS_BAR_TREE, INC>;
-    case HS_BAR_LF: return (const void *)k_scan_u32<HS_BAR_LF, INC>;
-    case HS_BAR_COOP: return (const void *)k_scan_u32<HS_BAR_COOP, INC>;
-    case HS_BAR_NAIVE_ALL: return (const void *)k_scan_u32<HS_BAR_NAIVE_ALL, INC>;
+    case HS_BAR_FLAT: return (const void *)k_scan_u32<HS_BAR_FLAT, SEGS, INC>;
+    case HS_BAR_TWO_LEVEL: return (const void *)k_scan_u32<HS_BAR_TWO_LEVEL, SEGS, INC>;
+    case HS_BAR_XCD: return (const void *)k_scan_u32<HS_BAR_XCD, SEGS, INC>;
+    case HS_BAR_XCD_FLAT_RELEASE: return (const void *)k_scan_u32<HS_BAR_XCD_FLAT_RELEASE, SEGS, INC>;
+    case HS_BAR_TREE: return (const void *)k_scan_u32<HS_BAR_TREE, SEGS, INC>;
+    case HS_BAR_LF: return (const void *)k_scan_u32<HS_BAR_LF, SEGS, INC>;
+    case HS_BAR_COOP: return (const void *)k_scan_u32<HS_BAR_COOP, SEGS, INC>;
+    case HS_BAR_NAIVE_ALL: return (const void *)k_scan_u32<HS_BAR_NAIVE_ALL, SEGS, INC>;
     default: return nullptr;
   }
+}
+
+template <int SEGS>
+const void *scan_kernel(int kind, int inclusive) {
+  return inclusive ? scan_kernel<SEGS, true>(kind) : scan_kernel<SEGS, false>(kind);
 }
 
 }  // namespace
@@ -320,17 +191,14 @@ int launch_persistent(const void *k, void **args, int kind, int num_wgs, int wg_
                       hipStream_t s);
 }  // namespace hs_host
 
-// round size: ~64 MiB of input per round by default (two rounds in flight stay
-// resident in the 256 MiB Infinity Cache; measured best of 32..1024 MiB),
-// rounded to a whole number of tiles per workgroup
-static uint64_t scan_round_elems(int num_wgs, uint64_t n, uint64_t target_bytes) {
-  const uint64_t per_wg_target = target_bytes / 4 / (uint64_t)num_wgs;
-  uint64_t tiles = per_wg_target / kTile;
-  if (tiles < 1) tiles = 1;
-  // no more tiles per workgroup than the whole input needs
-  const uint64_t need = (n + (uint64_t)num_wgs * kTile - 1) / ((uint64_t)num_wgs * kTile);
-  if (tiles > need && need > 0) tiles = need;
-  return tiles * kTile * (uint64_t)num_wgs;
+// Segments per wave: 4 (64 KiB per workgroup) where the input is then one round, as
+// more compute units have a tile, and where the round size in force asks for it;
+// else 16 (256 KiB: 8M elements in 18.3 us against 20.1 with two rounds of 4, 13M in
+// 23.6 against 32.8).  With 1 segment for less than 1M elements the words of 256
+// workgroups cost more than they bring (1M: 10.8 us against 9.9).
+static int scan_segs(int grid, uint64_t n, uint64_t round_bytes) {
+  const uint64_t round4 = (uint64_t)grid * kWaves * kSpan * 4;
+  return n <= round4 || 4 * round4 * sizeof(uint32_t) > round_bytes ? 4 : 16;
 }
 
 static uint64_t g_scan_round_bytes = 64ull << 20;
@@ -387,21 +255,32 @@ int hs_scan_u32(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n,
                 uint32_t *d_scratch, int kind, int num_wgs, void *stream) {
   if (!ar || !d_scratch || (n && (!d_in || !d_out))) return HS_ERR_INVALID;
   if (((uintptr_t)d_in & 15u) || ((uintptr_t)d_out & 15u)) return HS_ERR_INVALID;
-  const void *k = inclusive ? scan_kernel<true>(kind) : scan_kernel<false>(kind);
-  if (!k) return HS_ERR_INVALID;
-  if (num_wgs <= 0) num_wgs = hs_host::default_grid(k, kWg, 2);
+  if (!scan_kernel<4>(kind, inclusive)) return HS_ERR_INVALID;
+  const int cus = hs_host::device_cus();
+  if (num_wgs <= 0) num_wgs = 2 * cus;
   if (num_wgs > ar->view.max_blocks) return HS_ERR_INVALID;
-  int rc = hs_host::check_residency(k, num_wgs, kWg, 0);
+  if (num_wgs > 3 * cus) return HS_ERR_RESIDENCY;
+  // The grid that num_wgs asks for (counted in the 256-thread workgroups that
+  // d_scratch is sized by, 2 words each): workgroups of 1024 threads with 4 words
+  // each, 8-byte aligned, at most one per CU.  One workgroup needs no words.
+  const uint32_t odd = ((uintptr_t)d_scratch & 4u) ? 1u : 0u;
+  int g = (int)((2u * (uint32_t)num_wgs - odd) / 4u);
+  g = g < 1 ? 1 : g < cus ? g : cus;
+  const int segs = scan_segs(g, n, g_scan_round_bytes);
+  const void *k = segs == 4 ? scan_kernel<4>(kind, inclusive) : scan_kernel<16>(kind, inclusive);
+  int rc = hs_host::check_residency(k, g, kWg, 0);
   if (rc) return rc;
   if (n == 0) return HS_OK;
+  // no more workgroups than tiles
+  const uint64_t tiles = (n + (uint64_t)segs * kWaves * kSpan - 1) / ((uint64_t)segs * kWaves * kSpan);
+  if ((uint64_t)g > tiles) g = (int)tiles;
   hipStream_t s = (hipStream_t)stream;
   if ((rc = hs_host::prepare_barrier(ar, kind, s))) return rc;
-  uint64_t round = scan_round_elems(num_wgs, n, g_scan_round_bytes);
+  uint64_t *words = (uint64_t *)(d_scratch + odd);
   hs::ArenaView v = ar->view;
-  uint32_t ng = (uint32_t)v.num_groups, nx = (uint32_t)hs_host::xcd_groups(num_wgs);
-  void *args[] = {(void *)&v, (void *)&d_in, (void *)&d_out, (void *)&n, (void *)&d_scratch,
-                  (void *)&round, (void *)&ng, (void *)&nx};
-  return hs_host::launch_persistent(k, args, kind, num_wgs, kWg, 0, s);
+  uint32_t ng = (uint32_t)v.num_groups, nx = (uint32_t)hs_host::xcd_groups(g);
+  void *args[] = {(void *)&v, (void *)&d_in, (void *)&d_out, (void *)&n, (void *)&words, (void *)&ng, (void *)&nx};
+  return hs_host::launch_persistent(k, args, kind, g, kWg, 0, s);
 }
 
 int hs_scan_u32_noalloc(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n, int inclusive,
@@ -411,9 +290,8 @@ int hs_scan_u32_noalloc(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uin
     fprintf(stderr, "libhs: hs_scan_u32_noalloc: the cooperative-launch barrier kind is not offered\n");
     return HS_ERR_INVALID;
   }
-  const void *k = inclusive ? scan_kernel<true>(kind) : scan_kernel<false>(kind);
-  if (!k) return HS_ERR_INVALID;
-  if (num_wgs <= 0) num_wgs = hs_host::default_grid(k, kWg, 2);
+  if (!scan_kernel<4>(kind, inclusive)) return HS_ERR_INVALID;
+  if (num_wgs <= 0) num_wgs = 2 * hs_host::device_cus();
   if (num_wgs > kNoAllocMaxWgs) {
     fprintf(stderr, "libhs: hs_scan_u32_noalloc: %d workgroups exceed the static scratch (%d at most)\n",
             num_wgs, kNoAllocMaxWgs);
