@@ -126,16 +126,12 @@ int default_grid(const void *kernel, int wg_size, int wgs_per_cu) {
   return wgs_per_cu * device_cus();
 }
 
-int clear_status(hs_arena *a, hipStream_t s) {
-  // a fill kernel, not hipMemsetAsync: the launchers may be captured in a graph
-  return launch_fill(a->view.status, 1, 0u, s);
-}
-
 int finish(hs_arena *a, hipStream_t s) {
   HS_TRY_HIP(hipGetLastError());
   HS_TRY_HIP(hipStreamSynchronize(s));
-  uint32_t st = 0;
-  HS_TRY_HIP(hipMemcpy(&st, a->view.status, sizeof(st), hipMemcpyDeviceToHost));
+  // the first failure's code, written to host memory by the failing wait: a copy
+  // of the device word cost another round trip per synchronous call
+  const uint32_t st = __atomic_load_n(a->abort_host + hs::kHostStatus, __ATOMIC_SEQ_CST);
   if (st != 0) {
     // a failed wait leaves counters half-way through an episode and semaphore
     // records half-acquired: start clean (hs_arena_reset restores every
@@ -166,6 +162,8 @@ int arena_init_words(hs_arena *a, hipStream_t s) {
   // semaphore records are not touched here: hs_arena_reset re-creates each one
   // with its created capacity
   if ((rc = launch_fill(v.episode, (size_t)v.max_blocks, 0u, s))) return rc;
+  // the host's copy first: a failure after the fill sets both
+  __atomic_store_n(a->abort_host + hs::kHostStatus, 0u, __ATOMIC_SEQ_CST);
   if ((rc = launch_fill(v.status, 1, 0u, s))) return rc;
   return HS_OK;
 }

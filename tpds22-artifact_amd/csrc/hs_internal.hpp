@@ -41,10 +41,8 @@ int xcd_groups(int num_wgs);
 int xcd_groups_override();
 // co-residency check of a grid for a kernel: HS_OK or HS_ERR_RESIDENCY
 int check_residency(const void *kernel, int num_wgs, int wg_size, size_t dyn_lds);
-// after a persistent launch: synchronize on stream and translate the device status
+// after a persistent launch: synchronize on stream and translate the status
 int finish(hs_arena *arena, hipStream_t stream);
-// clear the arena's device status word before a launch
-int clear_status(hs_arena *arena, hipStream_t stream);
 // initialize all barrier/lock words (fill kernels; no per-int memset)
 int arena_init_words(hs_arena *arena, hipStream_t stream);
 // default persistent grid: wgs_per_cu * CUs capped by residency

@@ -207,10 +207,14 @@ def reduce_i32(arena: Arena, x, barrier="xcd", num_wgs: int = 0, out=None, parti
     L.check(lib.hs_reduce_partials_size(num_wgs, n, C.byref(nw)))
     if partials is None:
         partials = torch.empty(max(nw.value, 1), dtype=torch.int32, device=x.device)
-    if out is None:
+    # a sum the caller takes as a number is written to host memory by the kernel
+    host = out is None and sync and x.is_cuda
+    if host:
+        out = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    elif out is None:
         out = torch.empty(1, dtype=torch.int32, device=x.device)
     s = _stream(stream)
-    L.check(lib.hs_reduce_i32(arena.handle, _ptr(x), n, _ptr(partials), _ptr(out),
+    L.check(lib.hs_reduce_i32(arena.handle, _ptr(x), n, _ptr(partials), out.data_ptr() if host else _ptr(out),
                               barrier_kind(barrier), num_wgs, s), "hs_reduce_i32")
     if not sync:
         return out
