@@ -20,6 +20,7 @@
 #include "hs_internal.hpp"
 #include "hs_wave.hpp"
 #include "hs_worklist.hpp"
+#include "team_rounds.hpp"
 
 using namespace hs;
 
@@ -974,9 +975,11 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 //    single pass of short code.
 // Correctness does not depend on the placement: everything the rounds write is
 // written and read with agent-scope operations, and every wave's stores have
-// completed before its workgroup arrives.  The other workgroups wait in the grid
-// barrier meanwhile; a stretch is at most kTeamRounds rounds, so that wait stays
-// short.
+// completed before its workgroup arrives.  Nor on timing: the other workgroups wait
+// in the grid barrier meanwhile (a stretch is at most kTeamRounds rounds, so that
+// wait stays short), and what they read before it, to find out that this stretch is
+// not theirs, is not written until it is over (team_rounds.hpp: the counters of the
+// phase and the report of the stretch before; the team counts in others).
 constexpr int kTeamWg = 1024;               // threads per workgroup of the kernels that run team rounds
 constexpr uint32_t kTeamMax = 32;           // workgroups of a team
 constexpr uint32_t kTeamRounds = 256;
@@ -1023,6 +1026,43 @@ struct Segments {
     return i < n ? s * kSegCap + i : 0xFFFFFFFFu;
   }
 };
+
+// The counters of one round and of the next: of the grid, by phase, or of the team.
+struct Round {
+  uint32_t *ctr;
+  hs_rounds::Side side;
+  uint32_t i;
+  __device__ __forceinline__ uint32_t *at(hs_rounds::Counter c, uint32_t ahead = 0) const {
+    return ctr + hs_rounds::slot(side, c, i + ahead) * kCtr;
+  }
+  // one thread: clears what the rounds after this one use
+  __device__ __forceinline__ void open() const {
+    hs_rounds::open_round(side, i, [&](uint32_t s) { st_relaxed(ctr + s * kCtr, 0u); });
+  }
+};
+
+// What a stretch leaves to the next phase: lane l's word l, of which the last 32 are
+// the segments' counts.
+struct Report {
+  uint32_t w;
+  __device__ __forceinline__ void write(uint32_t *ctr, uint32_t k, uint32_t seg_cnt, const uint32_t (&head)[8]) {
+    const uint32_t lane = lane_id(), cnt = __shfl(seg_cnt, (int)(lane & 31));
+    w = cnt;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) w = lane == i ? head[i] : w;
+    st_relaxed(ctr + hs_rounds::report(k) * kCtr + lane, w);
+  }
+  __device__ __forceinline__ void read(const uint32_t *ctr, uint32_t k) {
+    w = ld_relaxed(ctr + hs_rounds::report(k) * kCtr + lane_id());
+  }
+  __device__ __forceinline__ uint32_t head(int i) const { return __builtin_amdgcn_readlane(w, i); }
+  // (every lane takes part in the shuffle)
+  __device__ __forceinline__ uint32_t segment() const {
+    const uint32_t cnt = __shfl(w, (int)(32 | (lane_id() & 31)));
+    return lane_id() < 32 ? cnt : 0u;
+  }
+};
+static_assert(kTeamMax == 32 && kCtr == 64, "a report is 32 words and the segments' counts");
 
 struct Team {
   uint64_t *word;       // [2][kTeamMax] episode << 32 | segment word, zero before the first grid barrier
@@ -1306,12 +1346,13 @@ struct BfsArgs1 {
   uint64_t hcap;
   uint64_t *seg;  // [2][kTeamMax][kSegCap] segments of a team: v | first edge << 32
   uint64_t *fbm[2];  // frontier bitmaps
-  uint32_t *ctr;  // light counts [3] (0..2), grab [3] (3..5), chunk counts [3] (6..8), pull chunks
-                  // [3] (9..11), the state a team stretch ends in (12), the team's words (13..14)
+  uint32_t *ctr;  // hs_rounds::kSlots, kCtr words apart
   uint32_t *stats;
   uint32_t mean_degree;
   uint32_t ng, nx;
 };
+static_assert(2 * kTeamMax * sizeof(uint64_t) <= (hs_rounds::kSlots - hs_rounds::kTeamWords) * kCtr * sizeof(uint32_t),
+              "the team's words fit their slots");
 
 struct BfInput {
   Segments seg;
@@ -1321,10 +1362,10 @@ struct BfInput {
 
 __device__ __forceinline__ uint32_t *bf_q(const BfsArgs1 &p, uint32_t r) { return p.q + (size_t)(r & 1) * p.n; }
 __device__ __forceinline__ uint64_t *bf_hq(const BfsArgs1 &p, uint32_t r) { return p.hq + (size_t)(r & 1) * p.hcap; }
-__device__ __forceinline__ uint32_t *bf_cnt(const BfsArgs1 &p, uint32_t r) { return p.ctr + (r % 3) * kCtr; }
-__device__ __forceinline__ uint32_t *bf_grab(const BfsArgs1 &p, uint32_t r) { return p.ctr + (3 + r % 3) * kCtr; }
-__device__ __forceinline__ uint32_t *bf_hcnt(const BfsArgs1 &p, uint32_t r) { return p.ctr + (6 + r % 3) * kCtr; }
-__device__ __forceinline__ uint32_t *bf_pcnt(const BfsArgs1 &p, uint32_t r) { return p.ctr + (9 + r % 3) * kCtr; }
+// chunks that the pull of phase k leaves
+__device__ __forceinline__ uint32_t *bf_pcnt(const BfsArgs1 &p, uint32_t k) {
+  return p.ctr + hs_rounds::other(k) * kCtr;
+}
 __device__ __forceinline__ uint64_t *bf_seg(const BfsArgs1 &p, uint32_t r, uint32_t rank) {
   return p.seg + ((size_t)(r & 1) * kTeamMax + rank) * kSegCap;
 }
@@ -1340,11 +1381,12 @@ struct BfStep {
   __device__ __forceinline__ void flush() { light.flush(); chunks.flush(); }
 };
 
-__device__ __forceinline__ BfStep bf_step(const BfsArgs1 &p, uint32_t r, Output *out, uint32_t rank, WaveBuffers *wb) {
+__device__ __forceinline__ BfStep bf_step(const BfsArgs1 &p, uint32_t r, const Round &rd, Output *out, uint32_t rank,
+                                          WaveBuffers *wb) {
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   return BfStep{p, r, out, rank,
-                {wb ? wb->near[wv] : nullptr, 0, bf_q(p, r + 1), bf_cnt(p, r + 1)},
-                {wb ? wb->chunks[wv] : nullptr, 0, bf_hq(p, r + 1), bf_hcnt(p, r + 1)}};
+                {wb ? wb->near[wv] : nullptr, 0, bf_q(p, r + 1), rd.at(hs_rounds::kLight, 1)},
+                {wb ? wb->chunks[wv] : nullptr, 0, bf_hq(p, r + 1), rd.at(hs_rounds::kChunks, 1)}};
 }
 
 // new vertices of level r + 1 to its input
@@ -1410,10 +1452,10 @@ __device__ __forceinline__ void bf_expand(BfStep &s, uint32_t eb, uint32_t deg) 
 }
 
 template <bool TEAM>
-__device__ __forceinline__ void bf_push_level(const BfsArgs1 &p, uint32_t r, const BfInput &in, const Crew &crew,
+__device__ __forceinline__ void bf_push_level(const BfsArgs1 &p, uint32_t r, const Round &rd, const BfInput &in, const Crew &crew,
                                               Output *out, uint32_t rank, WaveBuffers *wb) {
   const uint32_t lane = lane_id();
-  BfStep s = bf_step(p, r, out, rank, wb);
+  BfStep s = bf_step(p, r, rd, out, rank, wb);
   for (uint32_t b = crew.wave; b < in.seg.blocks; b += crew.waves) {
     const uint32_t i = in.seg.entry(b), x = lane & 3;
     const uint64_t ent = i != 0xFFFFFFFFu ? ld_u64(bf_seg(p, r, 0) + i) : 0ull;
@@ -1460,7 +1502,7 @@ __device__ __forceinline__ void bf_push_level(const BfsArgs1 &p, uint32_t r, con
     bf_expand<TEAM>(s, eb, deg);
     if ((uint64_t)crew.waves * share >= in.nin) break;
     uint32_t g = 0;
-    if (lane == 0) g = add_relaxed(bf_grab(p, r), 1u);
+    if (lane == 0) g = add_relaxed(rd.at(hs_rounds::kGrab), 1u);
     b = crew.waves + __builtin_amdgcn_readfirstlane(g);
   }
   if (!TEAM) s.flush();
@@ -1494,11 +1536,11 @@ __device__ __forceinline__ void bf_pull_found(BfStep &s, bool found, uint32_t v)
   bf_push<false, 1>(s, won, vs, eb, deg);
 }
 
-__device__ __forceinline__ void bf_pull_level(const BfsArgs1 &p, uint32_t r, const Crew &crew, WaveBuffers *wb) {
+__device__ __forceinline__ void bf_pull_level(const BfsArgs1 &p, uint32_t r, const Round &rd, const Crew &crew, WaveBuffers *wb) {
   __shared__ uint32_t hit_sh[kTeamWg];
   const uint32_t lane = lane_id();
   uint32_t *hit = hit_sh + (threadIdx.x & ~63u);
-  BfStep s = bf_step(p, r, nullptr, 0, wb);
+  BfStep s = bf_step(p, r, rd, nullptr, 0, wb);
   const uint64_t *fbm = p.fbm[r & 1];
   uint64_t *nbm = p.fbm[(r + 1) & 1];
   const uint32_t nblk = (p.n + 63) / 64, kb = log2_ceil(nblk);
@@ -1531,7 +1573,7 @@ __device__ __forceinline__ void bf_pull_level(const BfsArgs1 &p, uint32_t r, con
           const uint32_t nc = rest ? (rem + kPullChunk - 1) / kPullChunk : 0u;
           const uint32_t incl = wave_incl_scan(nc);
           uint32_t base = 0;
-          if (lane == 63) base = add_relaxed(bf_pcnt(p, r), incl);
+          if (lane == 63) base = add_relaxed(bf_pcnt(p, rd.i), incl);
           base = __builtin_amdgcn_readlane(base, 63) + incl - nc;
           for (uint32_t c = 0; c < nc; ++c) st_u64(bf_hq(p, r) + base + c, v | ((uint64_t)(b + c * kPullChunk) << 32));
           if (rest) rem = 0;
@@ -1563,10 +1605,10 @@ __device__ __forceinline__ void bf_pull_level(const BfsArgs1 &p, uint32_t r, con
 }
 
 // the hubs' chunks: the first wave that finds a parent reaches the vertex
-__device__ __forceinline__ void bf_pull_chunks(const BfsArgs1 &p, uint32_t r, uint32_t count, const Crew &crew,
+__device__ __forceinline__ void bf_pull_chunks(const BfsArgs1 &p, uint32_t r, const Round &rd, uint32_t count, const Crew &crew,
                                                WaveBuffers *wb) {
   const uint32_t lane = lane_id();
-  BfStep s = bf_step(p, r, nullptr, 0, wb);
+  BfStep s = bf_step(p, r, rd, nullptr, 0, wb);
   const uint64_t *fbm = p.fbm[r & 1];
   for (uint32_t i = crew.wave; i < count; i += crew.waves) {
     const uint64_t ent = ld_u64(bf_hq(p, r) + i);
@@ -1596,21 +1638,22 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;
-  team.init(reinterpret_cast<uint64_t *>(p.ctr + 13 * kCtr), p.nx);
-  uint32_t *ctl = p.ctr + 12 * kCtr;
+  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx);
   __shared__ Output out;
   __shared__ WaveBuffers wb;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
+  Round grid{p.ctr, hs_rounds::kGrid, 0};   // of this phase
+  Round round{p.ctr, hs_rounds::kTeam, 0};  // of the team's next round (of use to the team)
   for (uint64_t v = t0; v < p.n; v += nt) p.level[v] = v == (uint32_t)p.src ? 0 : kInf;
   if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
   if (t0 < 2 * kTeamMax) team.word[t0] = 0;
   if (t0 == 0) {
-    for (int i = 0; i < 12; ++i) p.ctr[i * kCtr] = 0;
+    for (uint32_t i = 0; i < hs_rounds::kReport; ++i) p.ctr[i * kCtr] = 0;
     const uint32_t nc = bfs_chunks(p.row[p.src + 1] - p.row[p.src]);
     for (uint32_t c = 0; c < nc; ++c) p.hq[c] = (uint32_t)p.src | ((uint64_t)c << 32);
-    p.ctr[6 * kCtr] = nc;
+    *grid.at(hs_rounds::kChunks) = nc;
     p.q[0] = (uint32_t)p.src;
-    p.ctr[0] = nc ? 0u : 1u;
+    *grid.at(hs_rounds::kLight) = nc ? 0u : 1u;
   }
   if (gb.sync<KIND>()) return;
   const Crew all(blockIdx.x, gridDim.x), few(team.rank, team.size);
@@ -1618,22 +1661,14 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   uint64_t behind = 0;        // edges of the frontiers so far, by the same estimate as `ahead` below
   bool have_bitmap = false;   // of the present frontier
   BfInput in;
+  auto look = [&](const Round &rd) {
+    in.nin = ld_relaxed(rd.at(hs_rounds::kLight));
+    in.nh = ld_relaxed(rd.at(hs_rounds::kChunks));
+  };
   in.seg.none();
-  auto look = [&]() {
-    in.nin = ld_relaxed(bf_cnt(p, r));
-    in.nh = ld_relaxed(bf_hcnt(p, r));
-  };
+  look(grid);
   auto edges = [&]() { return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk; };
-  auto clear_next = [&]() {  // counters last used two levels ago
-    if (t0 != 0) return;
-    st_relaxed(bf_cnt(p, r + 2), 0u);
-    st_relaxed(bf_hcnt(p, r + 2), 0u);
-    st_relaxed(bf_pcnt(p, r + 1), 0u);
-    st_relaxed(bf_grab(p, r + 1), 0u);
-  };
-  for (;;) {
-    look();
-    if (!in.any()) break;
+  while (in.any()) {
     const uint64_t ahead = edges();
     const bool by_team = team.usable && ahead <= kTeamEdges;
     // Pull once the frontier's edges are 1/kPullEdges of those left (they are
@@ -1647,30 +1682,32 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
       continue;
     }
     behind += ahead;
+    if (t0 == 0) {
+      grid.open();
+      st_relaxed(bf_pcnt(p, grid.i + 1), 0u);
+    }
     if (pull) {
-      clear_next();
-      bf_pull_level(p, r, all, &wb);
+      bf_pull_level(p, r, grid, all, &wb);
     } else if (!by_team) {
-      clear_next();
-      bf_push_level<false>(p, r, in, all, nullptr, 0, &wb);
+      bf_push_level<false>(p, r, grid, in, all, nullptr, 0, &wb);
     } else if (team.in) {
-      for (uint32_t k = 0; k < kTeamRounds; ++k) {
+      for (uint32_t q = 0; q < kTeamRounds; ++q) {
         const uint32_t par = r & 1;
         if (threadIdx.x == 0) out.clear(par ^ 1);
-        clear_next();
-        bf_push_level<true>(p, r, in, few, &out, team.rank, nullptr);
+        if (t0 == 0) round.open();
+        bf_push_level<true>(p, r, round, in, few, &out, team.rank, nullptr);
         ++r;
+        ++round.i;
         __syncthreads();
         if (team.sync(a, out.segment_word(par), in.seg)) return;
         in.nin = in.nh = 0;
-        if (in.seg.queued) look();
+        if (in.seg.queued) look(round);
         if (!in.any() || edges() > kTeamEdges) break;
         behind += edges();
       }
-      if (t0 == 0) {
-        st_relaxed(ctl, r);
-        st_relaxed(ctl + 1, team.episode);
-        st_u64(reinterpret_cast<uint64_t *>(ctl + 2), behind);
+      if (t0 < 64) {
+        Report rep;
+        rep.write(p.ctr, grid.i, in.seg.cnt, {r, in.nin, in.nh, (uint32_t)behind, (uint32_t)(behind >> 32), 0u, 0u, 0u});
       }
     } else {
       gb.poll_sleep = kTeamIdleSleep;
@@ -1679,22 +1716,27 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
     gb.poll_sleep = 0;
     have_bitmap = pull;
     if (by_team) {
-      r = ld_relaxed(ctl);
-      team.episode = ld_relaxed(ctl + 1);
-      behind = ld_u64(reinterpret_cast<uint64_t *>(ctl + 2));
-      // the segments of the last team level are still there
-      in.seg.take(lane_id() < team.size ? (uint32_t)ld_u64(team.word + (team.episode & 1) * kTeamMax + lane_id()) : 0u);
+      Report rep;
+      rep.read(p.ctr, grid.i);
+      r = rep.head(0);
+      in.nin = rep.head(1);
+      in.nh = rep.head(2);
+      behind = rep.head(3) | (uint64_t)rep.head(4) << 32;
+      in.seg.take(rep.segment());  // the segments of the last team level are still there
+      ++grid.i;
       continue;
     }
-    in.seg.none();
     if (pull) {
-      const uint32_t hubs = ld_relaxed(bf_pcnt(p, r));
+      const uint32_t hubs = ld_relaxed(bf_pcnt(p, grid.i));
       if (hubs) {
-        bf_pull_chunks(p, r, hubs, all, &wb);
+        bf_pull_chunks(p, r, grid, hubs, all, &wb);
         if (gb.sync<KIND>()) return;
       }
     }
     ++r;
+    ++grid.i;
+    in.seg.none();
+    look(grid);
   }
   if (t0 == 0 && p.stats) p.stats[0] = r;
 }
@@ -1712,16 +1754,11 @@ struct SsspArgs {
   uint64_t hcap;
   uint32_t *fq;      // [3][n] far lists
   uint64_t *seg;     // [2][kTeamMax][kSegCap] near segments of a team: v | first edge << 32
-  uint32_t *ctr;     // near counts [3] (0..2), grab [3] (3..5), far counts [3] (6..8),
-                     // near chunk counts [3] (9..11), the state a team stretch ends in (12),
-                     // the team's words (13..14)
+  uint32_t *ctr;     // hs_rounds::kSlots, kCtr words apart
   uint32_t *stats;
   uint32_t mean_degree;  // rounded up, for the size of a round
   uint32_t ng, nx;
 };
-constexpr int kSsCounters = 15;
-static_assert(2 * kTeamMax * sizeof(uint64_t) <= 2 * kCtr * sizeof(uint32_t), "the team's words fit slots 13 and 14");
-
 constexpr int kSsBatch = 4;
 
 __device__ __forceinline__ uint64_t ss_key(int32_t d, uint32_t stamp) {
@@ -1746,10 +1783,10 @@ __device__ __forceinline__ int32_t ss_bound(const SsspArgs &p, uint32_t epoch) {
   return (int32_t)min((int64_t)(epoch + 1) * p.delta, (int64_t)kInf - 1);
 }
 __device__ __forceinline__ uint32_t *ss_near_q(const SsspArgs &p, uint32_t r) { return p.nq + (size_t)(r & 1) * p.n; }
-__device__ __forceinline__ uint32_t *ss_near_cnt(const SsspArgs &p, uint32_t r) { return p.ctr + (r % 3) * kCtr; }
-__device__ __forceinline__ uint32_t *ss_heavy_cnt(const SsspArgs &p, uint32_t r) { return p.ctr + (9 + r % 3) * kCtr; }
 __device__ __forceinline__ uint32_t *ss_far_q(const SsspArgs &p, uint32_t e) { return p.fq + (size_t)(e % 3) * p.n; }
-__device__ __forceinline__ uint32_t *ss_far_cnt(const SsspArgs &p, uint32_t e) { return p.ctr + (6 + e % 3) * kCtr; }
+__device__ __forceinline__ uint32_t *ss_far_cnt(const SsspArgs &p, uint32_t e) {
+  return p.ctr + hs_rounds::other(e) * kCtr;
+}
 __device__ __forceinline__ uint64_t *ss_seg(const SsspArgs &p, uint32_t r, uint32_t rank) {
   return p.seg + ((size_t)(r & 1) * kTeamMax + rank) * kSegCap;
 }
@@ -1762,6 +1799,7 @@ struct SsStep {
   SsState st;
   int32_t bound;
   uint32_t far_epoch;  // bucket whose far list is appended to
+  Round rd;
   Output *out;         // of a team, else null, and the wave's lists instead
   uint32_t rank;
   WaveList<uint32_t, kWaveNear> near;
@@ -1782,9 +1820,11 @@ __device__ __forceinline__ void sssp_push(SsStep &s, const bool (&near)[B], cons
     light[x] = near[x] && nc[x] == 0;
   }
   if constexpr (TEAM) {
-    segment_push<B>(*s.out, r & 1, ss_seg(p, r + 1, s.rank), ss_near_q(p, r + 1), ss_near_cnt(p, r + 1), light, v, eb);
+    segment_push<B>(*s.out, r & 1, ss_seg(p, r + 1, s.rank), ss_near_q(p, r + 1), s.rd.at(hs_rounds::kLight, 1), light,
+                    v, eb);
     kept_push<B>(*s.out, ss_far_q(p, s.far_epoch), ss_far_cnt(p, s.far_epoch), far, v);
-    if (team_push_chunks<B>(p.hq + (size_t)((r + 1) & 1) * p.hcap, ss_heavy_cnt(p, r + 1), nc, v) && lane_id() == 0)
+    if (team_push_chunks<B>(p.hq + (size_t)((r + 1) & 1) * p.hcap, s.rd.at(hs_rounds::kChunks, 1), nc, v) &&
+        lane_id() == 0)
       s.out->queued[r & 1] = 1;
   } else {
     wave_list_push<B>(s.near, light, v);
@@ -1870,21 +1910,17 @@ __device__ __forceinline__ void sssp_expand(SsStep &s, uint32_t eb, uint32_t deg
 // One round, or with an empty near input one bucket step, by the given crew.
 // `first`: the thread that clears the counters.
 template <bool TEAM>
-__device__ __forceinline__ void sssp_step(const SsspArgs &p, SsState &st, const SsInput &in, const Crew &crew, bool first,
-                                          Output *out, uint32_t rank, WaveBuffers *wb) {
+__device__ __forceinline__ void sssp_step(const SsspArgs &p, SsState &st, const Round &rd, const SsInput &in,
+                                          const Crew &crew, bool first, Output *out, uint32_t rank, WaveBuffers *wb) {
   const uint32_t r = st.r, lane = lane_id();
   if (TEAM && threadIdx.x == 0) out->clear((r + 1) & 1);
-  if (first) {  // counters last used two rounds ago
-    st_relaxed(ss_near_cnt(p, r + 2), 0u);
-    st_relaxed(ss_heavy_cnt(p, r + 2), 0u);
-    st_relaxed(p.ctr + (3 + (r + 1) % 3) * kCtr, 0u);
-  }
+  if (TEAM && first) rd.open();
   const uint32_t far_epoch = in.near() ? st.epoch : st.epoch + 1;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  SsStep s{p, st, ss_bound(p, st.epoch), far_epoch, out, rank,
-           {TEAM ? nullptr : wb->near[wv], 0, ss_near_q(p, r + 1), ss_near_cnt(p, r + 1)},
+  SsStep s{p, st, ss_bound(p, st.epoch), far_epoch, rd, out, rank,
+           {TEAM ? nullptr : wb->near[wv], 0, ss_near_q(p, r + 1), rd.at(hs_rounds::kLight, 1)},
            {TEAM ? nullptr : wb->far[wv], 0, ss_far_q(p, far_epoch), ss_far_cnt(p, far_epoch)},
-           {TEAM ? nullptr : wb->chunks[wv], 0, p.hq + (size_t)((r + 1) & 1) * p.hcap, ss_heavy_cnt(p, r + 1)}};
+           {TEAM ? nullptr : wb->chunks[wv], 0, p.hq + (size_t)((r + 1) & 1) * p.hcap, rd.at(hs_rounds::kChunks, 1)}};
   if (in.near()) {
     // segments of a team's round
     for (uint32_t b = crew.wave; b < in.seg.blocks; b += crew.waves) {
@@ -1929,7 +1965,7 @@ __device__ __forceinline__ void sssp_step(const SsspArgs &p, SsState &st, const 
     // light near queue: the first share of each wave is dealt, further ones are
     // taken from the round's grab counter
     const uint32_t *qin = ss_near_q(p, r);
-    uint32_t *grab = p.ctr + (3 + r % 3) * kCtr;
+    uint32_t *grab = rd.at(hs_rounds::kGrab);
     const uint32_t share = queue_share(in.nin, crew.waves);
     for (uint32_t b = crew.wave; (uint64_t)b * share < in.nin;) {
       const uint32_t i = b * share + lane;
@@ -1982,86 +2018,97 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;
-  team.init(reinterpret_cast<uint64_t *>(p.ctr + 13 * kCtr), p.nx);
-  uint32_t *ctl = p.ctr + 12 * kCtr;
+  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx);
   __shared__ Output out;
   __shared__ WaveBuffers wb;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
+  Round grid{p.ctr, hs_rounds::kGrid, 0};   // of this phase
+  Round round{p.ctr, hs_rounds::kTeam, 0};  // of the team's next round (of use to the team)
   for (uint64_t v = t0; v < p.n; v += nt) p.key[v] = ss_key(v == (uint32_t)p.src ? 0 : kInf, 0);
   if (threadIdx.x == 0) { out.clear(0); out.clear(1); out.kept = out.fill = 0; }
   if (t0 < 2 * kTeamMax) team.word[t0] = 0;
   if (t0 == 0) {
-    for (int i = 0; i < 12; ++i) p.ctr[i * kCtr] = 0;
+    for (uint32_t i = 0; i < hs_rounds::kReport; ++i) p.ctr[i * kCtr] = 0;
     const uint32_t nc = bfs_chunks(p.row[p.src + 1] - p.row[p.src]);
     if (nc) {
       for (uint32_t c = 0; c < nc; ++c) p.hq[c] = (uint32_t)p.src | ((uint64_t)c << 32);
-      p.ctr[9 * kCtr] = nc;
+      *grid.at(hs_rounds::kChunks) = nc;
     } else {
       p.nq[0] = (uint32_t)p.src;
-      p.ctr[0] = 1;
+      *grid.at(hs_rounds::kLight) = 1;
     }
   }
   if (gb.sync<KIND>()) return;
   const Crew all(blockIdx.x, gridDim.x), few(team.rank, team.size);
   SsState st{0, 0, 0, 0};
   SsInput in;
-  in.seg.none();
-  // the queues' part of the next step's input
-  auto look = [&]() {
-    in.nin = ld_relaxed(ss_near_cnt(p, st.r));
-    in.nh = ld_relaxed(ss_heavy_cnt(p, st.r));
-    in.nfar = ld_relaxed(ss_far_cnt(p, st.epoch));
+  auto look = [&](const Round &rd) {
+    in.nin = ld_relaxed(rd.at(hs_rounds::kLight));
+    in.nh = ld_relaxed(rd.at(hs_rounds::kChunks));
+    // a round adds to the far list, a bucket step only reads it: its count is looked
+    // at where the next step is one
+    in.nfar = in.near() ? 1u : ld_relaxed(ss_far_cnt(p, st.epoch));
   };
+  in.seg.none();
+  look(grid);
+  bool told = false;  // the input is a stretch's report
   auto small = [&]() {
     if (!team.usable) return false;
     if (!in.near()) return in.nfar <= kTeamEdges / 4;
     return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk <= kTeamEdges;
   };
-  for (;;) {
-    look();
-    if (!in.near() && in.nfar == 0) break;
+  while (in.near() || in.nfar != 0) {
     const bool by_team = small();
+    // the others may read the far count of this bucket as long as the stretch runs
+    // (team_rounds.hpp): it stops before the bucket step that would clear it
+    const bool one_bucket = !told && !in.near();
+    if (t0 == 0) grid.open();
     if (!by_team) {
-      sssp_step<false>(p, st, in, all, t0 == 0, nullptr, 0, &wb);
+      sssp_step<false>(p, st, grid, in, all, t0 == 0, nullptr, 0, &wb);
     } else if (team.in) {
       for (uint32_t k = 0; k < kTeamRounds; ++k) {
         const uint32_t par = st.r & 1;
-        sssp_step<true>(p, st, in, few, t0 == 0, &out, team.rank, nullptr);
+        sssp_step<true>(p, st, round, in, few, t0 == 0, &out, team.rank, nullptr);
+        ++round.i;
         __syncthreads();
         if (team.sync(a, out.segment_word(par), in.seg)) return;
         in.nin = in.nh = 0;
         in.nfar = 1;  // not looked at while there are near vertices
-        if (in.seg.queued) look();
+        if (in.seg.queued) look(round);
         if (!in.near()) {
           // the kept far entries join the bucket's list
           kept_flush(out, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
           if (team.sync(a, 0, in.seg)) return;
-          look();
-          if (in.nfar == 0) break;
+          look(round);
+          if (in.nfar == 0 || one_bucket) break;
         }
         if (!small()) break;
       }
       kept_flush(out, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
-      if (t0 == 0) {
-        st_relaxed(ctl, st.r);
-        st_relaxed(ctl + 1, st.epoch);
-        st_relaxed(ctl + 2, st.relax);
-        st_relaxed(ctl + 3, st.far_since);
-        st_relaxed(ctl + 4, team.episode);
+      if (t0 < 64) {
+        Report rep;
+        rep.write(p.ctr, grid.i, in.seg.cnt, {st.r, st.epoch, st.relax, st.far_since, in.nin, in.nh, in.nfar, 0u});
       }
     } else {
       gb.poll_sleep = kTeamIdleSleep;
     }
     if (gb.sync<KIND>()) return;
     gb.poll_sleep = 0;
-    if (!by_team) {
+    told = by_team;
+    if (by_team) {
+      Report rep;
+      rep.read(p.ctr, grid.i);
+      st = SsState{rep.head(0), rep.head(1), rep.head(2), rep.head(3)};
+      in.nin = rep.head(4);
+      in.nh = rep.head(5);
+      in.nfar = rep.head(6);
+      in.seg.take(rep.segment());  // the segments of the last team round are still there
+      ++grid.i;
+    } else {
+      ++grid.i;
       in.seg.none();
-      continue;
+      look(grid);
     }
-    st = SsState{ld_relaxed(ctl), ld_relaxed(ctl + 1), ld_relaxed(ctl + 2), ld_relaxed(ctl + 3)};
-    team.episode = ld_relaxed(ctl + 4);
-    // the segments of the last team round are still there
-    in.seg.take(lane_id() < team.size ? (uint32_t)ld_u64(team.word + (team.episode & 1) * kTeamMax + lane_id()) : 0u);
   }
   for (uint64_t v = t0; v < p.n; v += nt) p.dist[v] = ss_dist(p.key[v]);
   if (t0 == 0 && p.stats) { p.stats[0] = st.relax; p.stats[1] = st.epoch; }
@@ -2394,7 +2441,7 @@ static uint64_t bfs_bitmap_bytes(uint32_t n) { return align256(sizeof(uint64_t) 
 
 int hs_bfs_work_size(uint32_t n, uint64_t m, uint64_t *bytes) {
   if (!bytes) return HS_ERR_INVALID;
-  *bytes = align256(sizeof(uint32_t) * 2ull * n) + align256(sizeof(uint32_t) * kBfsCounters * kCtr) +
+  *bytes = align256(sizeof(uint32_t) * 2ull * n) + align256(sizeof(uint32_t) * hs_rounds::kSlots * kCtr) +
            2 * align256(sizeof(uint64_t) * 2 * bfs_hcap(m)) + 2 * bfs_bitmap_bytes(n) +
            align256(sizeof(uint64_t) * 2 * kTeamMax * kSegCap);
   return HS_OK;
@@ -2422,7 +2469,7 @@ static int bfs_launch(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_ro
   p.src = src; p.level = d_level;
   char *w = (char *)d_work;
   p.q = (uint32_t *)w; w += align256(sizeof(uint32_t) * 2ull * n);
-  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * kBfsCounters * kCtr);
+  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * hs_rounds::kSlots * kCtr);
   p.hq = (uint64_t *)w; w += align256(sizeof(uint64_t) * 2 * bfs_hcap(m));
   p.hcap = bfs_hcap(m);
   for (auto &f : p.fbm) { f = (uint64_t *)w; w += bfs_bitmap_bytes(n); }
@@ -2538,7 +2585,7 @@ int hs_msbfs(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const 
 int hs_sssp_work_size(uint32_t n, uint64_t m, uint64_t *bytes) {
   if (!bytes) return HS_ERR_INVALID;
   *bytes = align256(sizeof(uint32_t) * 2ull * n) + align256(sizeof(uint32_t) * 3ull * n) +
-           align256(sizeof(uint64_t) * (uint64_t)n) + align256(sizeof(uint32_t) * kSsCounters * kCtr) +
+           align256(sizeof(uint64_t) * (uint64_t)n) + align256(sizeof(uint32_t) * hs_rounds::kSlots * kCtr) +
            align256(sizeof(uint64_t) * 2 * kTeamMax * kSegCap) +
            align256(sizeof(uint64_t) * 2 * bfs_hcap(m));
   return HS_OK;
@@ -2565,7 +2612,7 @@ int hs_sssp(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const u
   p.nq = (uint32_t *)w; w += align256(sizeof(uint32_t) * 2ull * n);
   p.fq = (uint32_t *)w; w += align256(sizeof(uint32_t) * 3ull * n);
   p.key = (uint64_t *)w; w += align256(sizeof(uint64_t) * (uint64_t)n);
-  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * kSsCounters * kCtr);
+  p.ctr = (uint32_t *)w; w += align256(sizeof(uint32_t) * hs_rounds::kSlots * kCtr);
   p.seg = (uint64_t *)w; w += align256(sizeof(uint64_t) * 2 * kTeamMax * kSegCap);
   p.hq = (uint64_t *)w;
   p.hcap = bfs_hcap(m);

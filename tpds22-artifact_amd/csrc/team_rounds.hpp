@@ -1,0 +1,59 @@
+// team_rounds.hpp -- where the BFS and SSSP kernels keep their counters, shared by
+// the kernels (graph.hip) and a host check (tests/test_team_rounds.py builds
+// tests/team_rounds_check.cpp with g++).
+//
+// The launch is a sequence of phases with a grid barrier after each: phase k is one
+// round of the whole grid, or a stretch of rounds by a team while the other
+// workgroups wait in the barrier.  At the start of a phase EVERY workgroup reads the
+// phase's input and decides from it what the phase is, and nothing makes the team
+// wait until the others have read: a workgroup may read at any time up to its
+// arrival at the phase's barrier, when the team has done any number of rounds.  So
+// no word that is read there may be written in the same phase:
+//  - the input a grid phase left is read from the grid's counters.  They are
+//    indexed by the phase, a round of the grid adds to those of k + 1 and clears
+//    those of k + 2, and a stretch only clears k + 2; the counters of phase k are
+//    next written in phase k + 1 (cleared) or k + 2 (added to), behind a barrier
+//    that every workgroup reaches only after it has read them;
+//  - the team's rounds count in counters of their own, indexed by the number of
+//    team rounds so far (`j`), which nobody else reads;
+//  - what a stretch left is read from its report, in one of two places by the
+//    phase's parity, next written in phase k + 2;
+//  - the words of the team's own barrier are read by the team alone.
+// The SSSP's far counters, one per bucket and three in turn, are added to by both
+// sides.  Bucket e's is read where the next step is a bucket step, which adds to
+// e + 1's and clears e + 2's; the bucket step after it would clear e's, so a stretch
+// that begins with a bucket step whose count was read from the counter ends before
+// the second one, and the next stretch has the count from the report.
+#pragma once
+
+#include <stdint.h>
+
+#if defined(__HIPCC__)
+#define HS_ROUND_FN __host__ __device__ inline
+#else
+#define HS_ROUND_FN inline
+#endif
+
+namespace hs_rounds {
+
+enum Side : uint32_t { kGrid = 0, kTeam = 12 };                // first slot of each side's counters
+enum Counter : uint32_t { kLight = 0, kGrab = 3, kChunks = 6 };  // three of each
+constexpr uint32_t kOther = 9;       // three more: the BFS's pull chunks by phase, the SSSP's far lists by bucket
+constexpr uint32_t kReport = 21;     // two reports
+constexpr uint32_t kTeamWords = 23;  // the words of the team's barrier, two slots
+constexpr uint32_t kSlots = 25;
+
+// counter of round i (a phase of the grid, or a team round j)
+HS_ROUND_FN uint32_t slot(Side side, Counter c, uint32_t i) { return side + c + i % 3; }
+HS_ROUND_FN uint32_t other(uint32_t i) { return kOther + i % 3; }
+HS_ROUND_FN uint32_t report(uint32_t k) { return kReport + (k & 1); }
+
+// the counters that round i of a side clears for the rounds after it
+template <class Clear>
+HS_ROUND_FN void open_round(Side side, uint32_t i, Clear clear) {
+  clear(slot(side, kLight, i + 2));
+  clear(slot(side, kChunks, i + 2));
+  clear(slot(side, kGrab, i + 1));
+}
+
+}  // namespace hs_rounds
