@@ -1231,7 +1231,9 @@ __device__ __forceinline__ void wave_list_push_chunks(WaveList<uint64_t, CAP> &l
 // to the queues, and a list kept in LDS until it is asked for (the SSSP far list).
 constexpr uint32_t kStage = 4096;
 struct Output {
-  uint32_t cnt[2], queued[2];  // by round parity
+  // by round parity; a round clears the other one, a stretch begins with both clear
+  // (the count of the last round of the stretch before is still there)
+  uint32_t cnt[2], queued[2];
   uint32_t kept, fill;         // slots handed out of `keep`, end of the filled ones
   uint32_t keep[kStage];
 
@@ -1645,7 +1647,6 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   Round grid{p.ctr, hs_rounds::kGrid, 0};   // of this phase
   Round round{p.ctr, hs_rounds::kTeam, 0};  // of the team's next round (of use to the team)
   for (uint64_t v = t0; v < p.n; v += nt) p.level[v] = v == (uint32_t)p.src ? 0 : kInf;
-  if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
   if (t0 < 2 * kTeamMax) team.word[t0] = 0;
   if (t0 == 0) {
     for (uint32_t i = 0; i < hs_rounds::kReport; ++i) p.ctr[i * kCtr] = 0;
@@ -1691,6 +1692,8 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
     } else if (!by_team) {
       bf_push_level<false>(p, r, grid, in, all, nullptr, 0, &wb);
     } else if (team.in) {
+      if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
+      __syncthreads();
       for (uint32_t q = 0; q < kTeamRounds; ++q) {
         const uint32_t par = r & 1;
         if (threadIdx.x == 0) out.clear(par ^ 1);
@@ -2025,7 +2028,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   Round grid{p.ctr, hs_rounds::kGrid, 0};   // of this phase
   Round round{p.ctr, hs_rounds::kTeam, 0};  // of the team's next round (of use to the team)
   for (uint64_t v = t0; v < p.n; v += nt) p.key[v] = ss_key(v == (uint32_t)p.src ? 0 : kInf, 0);
-  if (threadIdx.x == 0) { out.clear(0); out.clear(1); out.kept = out.fill = 0; }
+  if (threadIdx.x == 0) out.kept = out.fill = 0;
   if (t0 < 2 * kTeamMax) team.word[t0] = 0;
   if (t0 == 0) {
     for (uint32_t i = 0; i < hs_rounds::kReport; ++i) p.ctr[i * kCtr] = 0;
@@ -2066,6 +2069,8 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
     if (!by_team) {
       sssp_step<false>(p, st, grid, in, all, t0 == 0, nullptr, 0, &wb);
     } else if (team.in) {
+      if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
+      __syncthreads();
       for (uint32_t k = 0; k < kTeamRounds; ++k) {
         const uint32_t par = st.r & 1;
         sssp_step<true>(p, st, round, in, few, t0 == 0, &out, team.rank, nullptr);
