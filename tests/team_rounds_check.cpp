@@ -144,6 +144,12 @@ int main(int argc, char **argv) {
     bad += l.wrong != 0;
     ++launches;
   }
+  // a team leaves the kernel when a wait fails: not beside a barrier that never does
+  for (uint32_t grid = 1; grid < 300; ++grid)
+    for (uint32_t size = 1; size <= grid; ++size) {
+      bad += team_usable(size, grid, false);
+      bad += team_usable(size, grid, true) != (size < grid && size <= 32);
+    }
   printf("launches %ld reads %ld failures %ld\n", launches, reads, bad);
   return bad ? 1 : 0;
 }

@@ -39,4 +39,6 @@ def test_the_kernels_use_these_counters():
     text = open(os.path.join(CSRC, "graph.hip")).read()
     assert '#include "team_rounds.hpp"' in text
     body = text[text.index("struct BfsArgs1"):text.index("struct PrArgs")]
+    # no team where the grid's barrier has no limit
+    assert len(re.findall(r"team\.init\(", body)) == len(re.findall(r"KIND != HS_BAR_COOP\);", body)) == 2
     assert not re.search(r"% 3\) \* kCtr|p\.ctr \+ \d|p\.ctr\[\d", body)

@@ -981,7 +981,7 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 // not theirs, is not written until it is over (team_rounds.hpp: the counters of the
 // phase and the report of the stretch before; the team counts in others).
 constexpr int kTeamWg = 1024;               // threads per workgroup of the kernels that run team rounds
-constexpr uint32_t kTeamMax = 32;           // workgroups of a team
+using hs_rounds::kTeamMax;                  // workgroups of a team
 constexpr uint32_t kTeamRounds = 256;
 constexpr uint64_t kTeamEdges = 1ull << 17;  // edges of a round up to which the team runs it
 constexpr uint32_t kTeamIdleSleep = 32;     // s_sleep units between the idle workgroups' polls
@@ -1070,13 +1070,13 @@ struct Team {
   bool in, usable;
   uint32_t episode;
 
-  __device__ void init(uint64_t *w, uint32_t nxcd) {
+  __device__ void init(uint64_t *w, uint32_t nxcd, bool bounded) {
     const uint32_t x = nxcd < gridDim.x ? nxcd : gridDim.x;
     word = w;
     size = (gridDim.x + x - 1) / x;
     rank = blockIdx.x / x;
     in = blockIdx.x % x == 0;
-    usable = size < gridDim.x && size <= kTeamMax;
+    usable = hs_rounds::team_usable(size, gridDim.x, bounded);
     episode = 0;
   }
   // Barrier of the team; `mine` (thread 0): this workgroup's segment word, `seg`:
@@ -1640,7 +1640,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;
-  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx);
+  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
   __shared__ Output out;
   __shared__ WaveBuffers wb;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
@@ -2021,7 +2021,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;
-  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx);
+  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
   __shared__ Output out;
   __shared__ WaveBuffers wb;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;

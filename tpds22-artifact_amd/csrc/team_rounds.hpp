@@ -48,6 +48,15 @@ HS_ROUND_FN uint32_t slot(Side side, Counter c, uint32_t i) { return side + c + 
 HS_ROUND_FN uint32_t other(uint32_t i) { return kOther + i % 3; }
 HS_ROUND_FN uint32_t report(uint32_t k) { return kReport + (k & 1); }
 
+// Whether a launch has a team: some workgroups, at most kTeamMax, of a grid that has
+// others, whose barrier gives up like the team's own waits do (an abort, the spin
+// limit).  A cooperative grid sync does not: a team whose wait failed would leave the
+// others in it for good.
+constexpr uint32_t kTeamMax = 32;
+HS_ROUND_FN bool team_usable(uint32_t size, uint32_t grid, bool bounded) {
+  return bounded && size < grid && size <= kTeamMax;
+}
+
 // the counters that round i of a side clears for the rounds after it
 template <class Clear>
 HS_ROUND_FN void open_round(Side side, uint32_t i, Clear clear) {
