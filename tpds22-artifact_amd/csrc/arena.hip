@@ -22,6 +22,15 @@ __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v) {
     p[i] = v;
 }
 
+// the status word and the host's copy of it, both in stream order: work enqueued
+// before a reset may still fail, and sets both
+__global__ void k_clear_status(uint32_t *status, uint32_t *host) {
+  if (threadIdx.x == 0) {
+    hs::st_relaxed(status, 0u);
+    __hip_atomic_store(host, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // ring buffers: slot 0 of every (mutex, group) ring = 1, others = -1
 // (Heterosync/cudaLocks.cu:50-63)
 __global__ void k_init_rings(int32_t *rings, size_t n, int stride) {
@@ -162,9 +171,8 @@ int arena_init_words(hs_arena *a, hipStream_t s) {
   // semaphore records are not touched here: hs_arena_reset re-creates each one
   // with its created capacity
   if ((rc = launch_fill(v.episode, (size_t)v.max_blocks, 0u, s))) return rc;
-  // the host's copy first: a failure after the fill sets both
-  __atomic_store_n(a->abort_host + hs::kHostStatus, 0u, __ATOMIC_SEQ_CST);
-  if ((rc = launch_fill(v.status, 1, 0u, s))) return rc;
+  hipLaunchKernelGGL(k_clear_status, dim3(1), dim3(64), 0, s, v.status, a->abort_host + hs::kHostStatus);
+  HS_TRY_HIP(hipGetLastError());
   return HS_OK;
 }
 
