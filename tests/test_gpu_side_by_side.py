@@ -1,0 +1,91 @@
+"""Two persistent launches at once on one GPU: on two streams with an arena each, and
+beside a serving loop of the default size."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+class Work:
+    """One kind of launch with its inputs and buffers: enqueue() on a stream, check()."""
+
+    def __init__(self, hs, name):
+        import torch
+        import hsync.graph as G
+        self.hs, self.name, self.arena = hs, name, hs.Arena()
+        if name in ("bfs", "sssp"):
+            row, col = G.rmat_csr(14, 16, 5)
+            self.g = G.Graph(row, col, G.weights(col.size, 5))
+            self.src = int(np.argmax(np.diff(row.astype(np.int64))))
+            self.out = torch.empty(self.g.n, dtype=torch.int32, device="cuda")
+            self.work = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+
+    def enqueue(self, stream):
+        import torch
+        import hsync.graph as G
+        with torch.cuda.stream(stream):  # a call's own tensors belong to its stream
+            if self.name == "bfs":
+                G.bfs(self.arena, self.g, self.src, level=self.out, work=self.work, sync=False)
+            elif self.name == "sssp":
+                G.sssp(self.arena, self.g, self.src, dist=self.out, work=self.work, sync=False)
+
+    def check(self, stream, oracle):
+        self.arena.sync(stream.cuda_stream)
+        got = self.out.cpu().numpy()
+        if self.name == "bfs":
+            assert np.array_equal(got, oracle.bfs(self.g.h_row, self.g.h_col, self.src))
+        elif self.name == "sssp":
+            assert np.array_equal(got, oracle.sssp(self.g.h_row, self.g.h_col, self.g.h_w, self.src))
+
+    def close(self):
+        self.arena.close()
+
+
+NAMES = ["bfs", "sssp"]
+
+
+@pytest.mark.parametrize("a", NAMES)
+@pytest.mark.parametrize("b", NAMES)
+def test_on_two_streams(hs, oracle, a, b):
+    import torch
+    jobs = [Work(hs, a), Work(hs, b)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    try:
+        for _ in range(10):
+            for j, s in zip(jobs, streams):
+                j.enqueue(s)
+        for j, s in zip(jobs, streams):
+            j.check(s, oracle)
+    finally:
+        for s in streams:
+            s.synchronize()
+        for j in jobs:
+            j.close()
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_beside_the_serving_loop(hs, oracle, name):
+    """While the loop runs, nothing waits for the whole device: buffers and the arena
+    are there before it starts, and a first call has made the allocations of a call."""
+    import torch
+    from hsync.serve import Server
+    job = Work(hs, name)
+    s = torch.cuda.current_stream()
+    job.enqueue(s)
+    job.check(s, oracle)
+    job.out.zero_()
+    x = torch.arange(5000, dtype=torch.int32, device="cuda")
+    total = torch.zeros(1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    srv = Server()
+    try:
+        idx = srv.reduce(x, total)
+        for _ in range(3):
+            job.enqueue(s)
+        job.check(s, oracle)
+        assert srv.wait(idx)["status"] == 0
+    finally:
+        srv.stop()
+    assert int(total.item()) == 5000 * 4999 // 2
+    job.close()

@@ -47,6 +47,8 @@ __device__ __forceinline__ int32_t ld_i32(const int32_t *p) {
 __device__ __forceinline__ uint64_t ld_u64(const uint64_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// a word that every lane reads alike, in a scalar register
+__device__ __forceinline__ uint32_t ld_uniform(const uint32_t *p) { return __builtin_amdgcn_readfirstlane(ld_relaxed(p)); }
 __device__ __forceinline__ uint64_t shfl64(uint64_t v, uint32_t lane) {
   const uint32_t lo = __shfl((uint32_t)v, (int)lane), hi = __shfl((uint32_t)(v >> 32), (int)lane);
   return ((uint64_t)hi << 32) | lo;
@@ -980,7 +982,15 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 // wait stays short), and what they read before it, to find out that this stretch is
 // not theirs, is not written until it is over (team_rounds.hpp: the counters of the
 // phase and the report of the stretch before; the team counts in others).
-constexpr int kTeamWg = 1024;               // threads per workgroup of the kernels that run team rounds
+// Threads per workgroup of the kernels that run team rounds: with 128 registers and
+// 33 KB of LDS at most, one workgroup is half of a CU, so that two searches on two
+// streams, or one beside the serving loop (one workgroup of 248 registers per CU),
+// are resident together.  1024 threads fill the CU, and each of two such launches may
+// get part of the CUs and wait for the rest; they take R-MAT 22 in 334 us (BFS) and
+// 2.87 ms (SSSP) against 357 us and 3.20 ms, a mesh of 1.1M vertices in 13.7 ms
+// against 12.9 and 200k vertices in 164 us against 135.  64 registers, for four
+// searches at once, spill: 392 us, 3.34 ms and 24.6 ms.
+constexpr int kTeamWg = 512;
 using hs_rounds::kTeamMax;                  // workgroups of a team
 constexpr uint32_t kTeamRounds = 256;
 constexpr uint64_t kTeamEdges = 1ull << 17;  // edges of a round up to which the team runs it
@@ -1182,7 +1192,6 @@ constexpr uint32_t kWaveNear = 512, kWaveFar = 256, kWaveChunks = 128;
 struct WaveBuffers {
   uint64_t chunks[kTeamWg / 64][kWaveChunks];
   uint32_t near[kTeamWg / 64][kWaveNear];
-  uint32_t far[kTeamWg / 64][kWaveFar];
 };
 
 template <int B, uint32_t CAP>
@@ -1227,20 +1236,26 @@ __device__ __forceinline__ void wave_list_push_chunks(WaveList<uint64_t, CAP> &l
   }
 }
 
-// A workgroup's outputs of a team round: its segment's count, whether it appended
-// to the queues, and a list kept in LDS until it is asked for (the SSSP far list).
-constexpr uint32_t kStage = 4096;
+// A workgroup's outputs of a team round: its segment's count and whether it appended
+// to the queues.
 struct Output {
   // by round parity; a round clears the other one, a stretch begins with both clear
   // (the count of the last round of the stretch before is still there)
   uint32_t cnt[2], queued[2];
-  uint32_t kept, fill;         // slots handed out of `keep`, end of the filled ones
-  uint32_t keep[kStage];
 
   __device__ void clear(uint32_t par) { cnt[par] = queued[par] = 0; }  // one thread
   __device__ uint32_t segment_word(uint32_t par) const {
     return min(cnt[par], kSegCap) | (queued[par] ? 0x80000000u : 0u);
   }
+};
+
+// A list kept in LDS over the rounds of a stretch until it is asked for (the SSSP
+// far list).
+constexpr uint32_t kStage = 4096;
+struct Kept {
+  uint32_t slots, fill;  // slots handed out of `keep`, end of the filled ones
+  uint32_t keep[kStage];
+  __device__ void clear() { slots = fill = 0; }  // one thread
 };
 
 // Appends vertices (with their first edges) to the workgroup's segment, those
@@ -1277,7 +1292,7 @@ __device__ __forceinline__ void segment_push(Output &out, uint32_t par, uint64_t
 
 // Appends to the kept list, what does not fit to its queue.
 template <int B>
-__device__ __forceinline__ void kept_push(Output &out, uint32_t *q, uint32_t *cnt, const bool (&want)[B],
+__device__ __forceinline__ void kept_push(Kept &k, uint32_t *q, uint32_t *cnt, const bool (&want)[B],
                                           const uint32_t (&v)[B]) {
   uint64_t mask[B];
   uint32_t total = 0;
@@ -1289,8 +1304,8 @@ __device__ __forceinline__ void kept_push(Output &out, uint32_t *q, uint32_t *cn
   if (total == 0) return;
   uint32_t base = 0;
   if (lane_id() == 0) {
-    base = atomicAdd(&out.kept, total);
-    if (base + total <= kStage) atomicMax(&out.fill, base + total);  // slots in order: those that fit form a prefix
+    base = atomicAdd(&k.slots, total);
+    if (base + total <= kStage) atomicMax(&k.fill, base + total);  // slots in order: those that fit form a prefix
   }
   base = __builtin_amdgcn_readfirstlane(base);
   if (base + total > kStage) {
@@ -1299,21 +1314,21 @@ __device__ __forceinline__ void kept_push(Output &out, uint32_t *q, uint32_t *cn
   }
 #pragma unroll
   for (int x = 0; x < B; ++x) {
-    if (mask[x] >> lane_id() & 1) out.keep[base + lanes_below(mask[x])] = v[x];
+    if (mask[x] >> lane_id() & 1) k.keep[base + lanes_below(mask[x])] = v[x];
     base += (uint32_t)__builtin_popcountll(mask[x]);
   }
 }
 
 // Moves the kept list to its queue (every thread of the workgroup calls it).
-__device__ __forceinline__ void kept_flush(Output &out, uint32_t *q, uint32_t *cnt) {
+__device__ __forceinline__ void kept_flush(Kept &k, uint32_t *q, uint32_t *cnt) {
   __shared__ uint32_t base_sh;
   __syncthreads();
-  const uint32_t n = out.fill;
+  const uint32_t n = k.fill;
   if (threadIdx.x == 0) base_sh = n ? add_relaxed(cnt, n) : 0u;
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n; i += kTeamWg) st_relaxed(q + base_sh + i, out.keep[i]);
+  for (uint32_t i = threadIdx.x; i < n; i += kTeamWg) st_relaxed(q + base_sh + i, k.keep[i]);
   __syncthreads();
-  if (threadIdx.x == 0) out.kept = out.fill = 0;
+  if (threadIdx.x == 0) k.clear();
   __syncthreads();
 }
 
@@ -1663,8 +1678,8 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   bool have_bitmap = false;   // of the present frontier
   BfInput in;
   auto look = [&](const Round &rd) {
-    in.nin = ld_relaxed(rd.at(hs_rounds::kLight));
-    in.nh = ld_relaxed(rd.at(hs_rounds::kChunks));
+    in.nin = ld_uniform(rd.at(hs_rounds::kLight));
+    in.nh = ld_uniform(rd.at(hs_rounds::kChunks));
   };
   in.seg.none();
   look(grid);
@@ -1730,7 +1745,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
       continue;
     }
     if (pull) {
-      const uint32_t hubs = ld_relaxed(bf_pcnt(p, grid.i));
+      const uint32_t hubs = ld_uniform(bf_pcnt(p, grid.i));
       if (hubs) {
         bf_pull_chunks(p, r, grid, hubs, all, &wb);
         if (gb.sync<KIND>()) return;
@@ -1804,6 +1819,7 @@ struct SsStep {
   uint32_t far_epoch;  // bucket whose far list is appended to
   Round rd;
   Output *out;         // of a team, else null, and the wave's lists instead
+  Kept *kept;
   uint32_t rank;
   WaveList<uint32_t, kWaveNear> near;
   WaveList<uint32_t, kWaveFar> far;
@@ -1825,7 +1841,7 @@ __device__ __forceinline__ void sssp_push(SsStep &s, const bool (&near)[B], cons
   if constexpr (TEAM) {
     segment_push<B>(*s.out, r & 1, ss_seg(p, r + 1, s.rank), ss_near_q(p, r + 1), s.rd.at(hs_rounds::kLight, 1), light,
                     v, eb);
-    kept_push<B>(*s.out, ss_far_q(p, s.far_epoch), ss_far_cnt(p, s.far_epoch), far, v);
+    kept_push<B>(*s.kept, ss_far_q(p, s.far_epoch), ss_far_cnt(p, s.far_epoch), far, v);
     if (team_push_chunks<B>(p.hq + (size_t)((r + 1) & 1) * p.hcap, s.rd.at(hs_rounds::kChunks, 1), nc, v) &&
         lane_id() == 0)
       s.out->queued[r & 1] = 1;
@@ -1910,20 +1926,29 @@ __device__ __forceinline__ void sssp_expand(SsStep &s, uint32_t eb, uint32_t deg
   });
 }
 
+// a workgroup's lists: of its waves in a round of the grid, kept in a stretch
+union SsLists {
+  struct {
+    WaveBuffers lists;
+    uint32_t far[kTeamWg / 64][kWaveFar];
+  } wave;
+  Kept kept;
+};
+
 // One round, or with an empty near input one bucket step, by the given crew.
 // `first`: the thread that clears the counters.
 template <bool TEAM>
 __device__ __forceinline__ void sssp_step(const SsspArgs &p, SsState &st, const Round &rd, const SsInput &in,
-                                          const Crew &crew, bool first, Output *out, uint32_t rank, WaveBuffers *wb) {
+                                          const Crew &crew, bool first, Output *out, uint32_t rank, SsLists *lists) {
   const uint32_t r = st.r, lane = lane_id();
   if (TEAM && threadIdx.x == 0) out->clear((r + 1) & 1);
   if (TEAM && first) rd.open();
   const uint32_t far_epoch = in.near() ? st.epoch : st.epoch + 1;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  SsStep s{p, st, ss_bound(p, st.epoch), far_epoch, rd, out, rank,
-           {TEAM ? nullptr : wb->near[wv], 0, ss_near_q(p, r + 1), rd.at(hs_rounds::kLight, 1)},
-           {TEAM ? nullptr : wb->far[wv], 0, ss_far_q(p, far_epoch), ss_far_cnt(p, far_epoch)},
-           {TEAM ? nullptr : wb->chunks[wv], 0, p.hq + (size_t)((r + 1) & 1) * p.hcap, rd.at(hs_rounds::kChunks, 1)}};
+  SsStep s{p, st, ss_bound(p, st.epoch), far_epoch, rd, out, &lists->kept, rank,
+           {TEAM ? nullptr : lists->wave.lists.near[wv], 0, ss_near_q(p, r + 1), rd.at(hs_rounds::kLight, 1)},
+           {TEAM ? nullptr : lists->wave.far[wv], 0, ss_far_q(p, far_epoch), ss_far_cnt(p, far_epoch)},
+           {TEAM ? nullptr : lists->wave.lists.chunks[wv], 0, p.hq + (size_t)((r + 1) & 1) * p.hcap, rd.at(hs_rounds::kChunks, 1)}};
   if (in.near()) {
     // segments of a team's round
     for (uint32_t b = crew.wave; b < in.seg.blocks; b += crew.waves) {
@@ -2023,12 +2048,11 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   Team team;
   team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
   __shared__ Output out;
-  __shared__ WaveBuffers wb;
+  __shared__ SsLists lists;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
   Round grid{p.ctr, hs_rounds::kGrid, 0};   // of this phase
   Round round{p.ctr, hs_rounds::kTeam, 0};  // of the team's next round (of use to the team)
   for (uint64_t v = t0; v < p.n; v += nt) p.key[v] = ss_key(v == (uint32_t)p.src ? 0 : kInf, 0);
-  if (threadIdx.x == 0) out.kept = out.fill = 0;
   if (t0 < 2 * kTeamMax) team.word[t0] = 0;
   if (t0 == 0) {
     for (uint32_t i = 0; i < hs_rounds::kReport; ++i) p.ctr[i * kCtr] = 0;
@@ -2046,11 +2070,11 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   SsState st{0, 0, 0, 0};
   SsInput in;
   auto look = [&](const Round &rd) {
-    in.nin = ld_relaxed(rd.at(hs_rounds::kLight));
-    in.nh = ld_relaxed(rd.at(hs_rounds::kChunks));
+    in.nin = ld_uniform(rd.at(hs_rounds::kLight));
+    in.nh = ld_uniform(rd.at(hs_rounds::kChunks));
     // a round adds to the far list, a bucket step only reads it: its count is looked
     // at where the next step is one
-    in.nfar = in.near() ? 1u : ld_relaxed(ss_far_cnt(p, st.epoch));
+    in.nfar = in.near() ? 1u : ld_uniform(ss_far_cnt(p, st.epoch));
   };
   in.seg.none();
   look(grid);
@@ -2067,13 +2091,13 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
     const bool one_bucket = !told && !in.near();
     if (t0 == 0) grid.open();
     if (!by_team) {
-      sssp_step<false>(p, st, grid, in, all, t0 == 0, nullptr, 0, &wb);
+      sssp_step<false>(p, st, grid, in, all, t0 == 0, nullptr, 0, &lists);
     } else if (team.in) {
-      if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
+      if (threadIdx.x == 0) { out.clear(0); out.clear(1); lists.kept.clear(); }
       __syncthreads();
       for (uint32_t k = 0; k < kTeamRounds; ++k) {
         const uint32_t par = st.r & 1;
-        sssp_step<true>(p, st, round, in, few, t0 == 0, &out, team.rank, nullptr);
+        sssp_step<true>(p, st, round, in, few, t0 == 0, &out, team.rank, &lists);
         ++round.i;
         __syncthreads();
         if (team.sync(a, out.segment_word(par), in.seg)) return;
@@ -2082,14 +2106,14 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
         if (in.seg.queued) look(round);
         if (!in.near()) {
           // the kept far entries join the bucket's list
-          kept_flush(out, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
+          kept_flush(lists.kept, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
           if (team.sync(a, 0, in.seg)) return;
           look(round);
           if (in.nfar == 0 || one_bucket) break;
         }
         if (!small()) break;
       }
-      kept_flush(out, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
+      kept_flush(lists.kept, ss_far_q(p, st.epoch), ss_far_cnt(p, st.epoch));
       if (t0 < 64) {
         Report rep;
         rep.write(p.ctr, grid.i, in.seg.cnt, {st.r, st.epoch, st.relax, st.far_since, in.nin, in.nh, in.nfar, 0u});
