@@ -216,8 +216,9 @@ int hs_scan_scratch_size(int num_wgs, uint64_t n, uint64_t *elems_out);
    stream are ordered. */
 int hs_scan_u32_noalloc(hs_arena *arena, const uint32_t *d_in, uint32_t *d_out, uint64_t n,
                         int inclusive, int barrier_kind, int num_wgs, void *stream);
-/* bytes of input per round of hs_scan_u32 in this process, at most (default 64 MiB:
-   the 256 KiB that each CU's registers hold), but no less than 64 KiB per CU in use */
+/* bytes of input per round of hs_scan_u32 in this process, at most (default 64 MiB,
+   which is no limit up to 512 CUs: a round is the 128 KiB that half of each CU's
+   registers hold), but no less than 32 KiB per CU in use */
 int hs_scan_set_round_bytes(uint64_t bytes);
 int hs_scan_get_round_bytes(uint64_t *bytes_out);
 

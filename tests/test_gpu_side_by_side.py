@@ -1,5 +1,9 @@
 """Two persistent launches at once on one GPU: on two streams with an arena each, and
 beside a serving loop of the default size."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -19,6 +23,12 @@ class Work:
             self.src = int(np.argmax(np.diff(row.astype(np.int64))))
             self.out = torch.empty(self.g.n, dtype=torch.int32, device="cuda")
             self.work = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+        else:
+            n = 9_000_001  # more than a round of half the CUs' registers
+            self.x = torch.empty(n, dtype=torch.int32, device="cuda")
+            hs.gen_uniform_u32(self.x, 6, 0, 2**32 - 1)
+            self.out = torch.empty_like(self.x)
+            self.scratch = torch.empty(8192, dtype=torch.int32, device="cuda")
         torch.cuda.synchronize()
 
     def enqueue(self, stream):
@@ -29,6 +39,8 @@ class Work:
                 G.bfs(self.arena, self.g, self.src, level=self.out, work=self.work, sync=False)
             elif self.name == "sssp":
                 G.sssp(self.arena, self.g, self.src, dist=self.out, work=self.work, sync=False)
+            else:
+                self.hs.scan_u32(self.arena, self.x, out=self.out, scratch=self.scratch, sync=False)
 
     def check(self, stream, oracle):
         self.arena.sync(stream.cuda_stream)
@@ -37,12 +49,15 @@ class Work:
             assert np.array_equal(got, oracle.bfs(self.g.h_row, self.g.h_col, self.src))
         elif self.name == "sssp":
             assert np.array_equal(got, oracle.sssp(self.g.h_row, self.g.h_col, self.g.h_w, self.src))
+        else:
+            x = oracle.gen_uniform_u32(6, got.size, 0, 2**32 - 1)
+            assert np.array_equal(got.view(np.uint32), np.cumsum(x, dtype=np.uint32))
 
     def close(self):
         self.arena.close()
 
 
-NAMES = ["bfs", "sssp"]
+NAMES = ["bfs", "sssp", "scan"]
 
 
 @pytest.mark.parametrize("a", NAMES)
@@ -64,28 +79,47 @@ def test_on_two_streams(hs, oracle, a, b):
             j.close()
 
 
-@pytest.mark.parametrize("name", NAMES)
-def test_beside_the_serving_loop(hs, oracle, name):
-    """While the loop runs, nothing waits for the whole device: buffers and the arena
-    are there before it starts, and a first call has made the allocations of a call."""
+def test_beside_the_serving_loop():
+    """In a process of its own: HIP spreads a process's streams over four hardware
+    queues, and a launch whose stream shares the queue of a kernel that does not end
+    waits for it whatever room there is.  This one has two streams."""
+    r = subprocess.run([sys.executable, "-u", os.path.abspath(__file__)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split()[-1:] == ["done"], r.stdout + r.stderr[-2000:]
+
+
+def _beside_the_serving_loop():
+    """While the loop runs, nothing waits for the whole device: buffers and arenas are
+    there before it starts, and a first call has made the allocations of a call."""
+    import conftest  # noqa: F401  (the import paths)
     import torch
+    import hsync as hs
+    import oracle_lib
     from hsync.serve import Server
-    job = Work(hs, name)
+    oracle = oracle_lib.load()
+    jobs = [Work(hs, name) for name in NAMES]
     s = torch.cuda.current_stream()
-    job.enqueue(s)
-    job.check(s, oracle)
-    job.out.zero_()
+    for job in jobs:
+        job.enqueue(s)
+        job.check(s, oracle)
+        job.out.zero_()
     x = torch.arange(5000, dtype=torch.int32, device="cuda")
     total = torch.zeros(1, dtype=torch.int32, device="cuda")
     torch.cuda.synchronize()
     srv = Server()
     try:
         idx = srv.reduce(x, total)
-        for _ in range(3):
+        for job in jobs:
+            print(job.name, flush=True)
             job.enqueue(s)
-        job.check(s, oracle)
+            job.check(s, oracle)
         assert srv.wait(idx)["status"] == 0
     finally:
         srv.stop()
     assert int(total.item()) == 5000 * 4999 // 2
-    job.close()
+    for job in jobs:
+        job.close()
+    print("done", flush=True)
+
+
+if __name__ == "__main__":
+    _beside_the_serving_loop()

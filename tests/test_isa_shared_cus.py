@@ -19,6 +19,7 @@ VGPRS, LDS = 512, 160 * 1024  # per SIMD and lane, per CU
 DEFAULT = {
     r"5k_bfsI": ("graph", 512, 1),
     r"6k_ssspI": ("graph", 512, 1),
+    r"10k_scan_u32I": ("scan", 512, 1),
 }
 
 

@@ -14,9 +14,9 @@
 // behind it, and clears the second's: an input of one round waits once (1M elements:
 // 12.1 us with the barrier before the first tile and the words polled, 9.9 so).
 // Bound by HBM: 2^28 elements 0.57 ms when each round was summed, crossed a barrier
-// and was read a second time from the Infinity Cache, 0.40 ms so (5.4 TB/s; a copy
-// of that size reaches 5.2); 100M 214 -> 157 us, 30M 64 -> 49, 13M 30 -> 24, 8M
-// 21 -> 18, 4M and less as before (12 us, 10 from 2M down).
+// and was read a second time from the Infinity Cache, 0.43 ms so (5.0 TB/s; a copy
+// of that size reaches 5.2); 100M 211 -> 162 us, 30M 63 -> 53, 13M 30 -> 26, 8M and
+// less as before (16 us, 12 at 4M, 10 from 2M down).
 // uint32 wrap arithmetic: bit-exact for any grid and round size.
 #include <hip/hip_runtime.h>
 
@@ -36,7 +36,11 @@ static __device__ __align__(256) uint32_t scratch[2 * kNoAllocMaxWgs];
 
 namespace {
 
-constexpr int kWg = 1024;   // threads of a workgroup, one per CU
+// Threads of a workgroup, one per CU: with 128 registers half of the CU, so that a scan
+// and another launch, or the serving loop, are resident together (1024 threads fill the
+// CU; they scan 2^28 elements in 407 us against 428, 13M in 22.8 against 26.1, 8M in
+// 17.6 against 15.7).
+constexpr int kWg = 512;
 constexpr int kWaves = kWg / 64;
 constexpr int kSpan = 256;  // elements of a wave's segment: 4 per lane, 1 KiB per instruction
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -191,14 +195,13 @@ int launch_persistent(const void *k, void **args, int kind, int num_wgs, int wg_
                       hipStream_t s);
 }  // namespace hs_host
 
-// Segments per wave: 4 (64 KiB per workgroup) where the input is then one round, as
-// more compute units have a tile, and where the round size in force asks for it;
-// else 16 (256 KiB: 8M elements in 18.3 us against 20.1 with two rounds of 4, 13M in
-// 23.6 against 32.8).  With 1 segment for less than 1M elements the words of 256
-// workgroups cost more than they bring (1M: 10.8 us against 9.9).
-static int scan_segs(int grid, uint64_t n, uint64_t round_bytes) {
-  const uint64_t round4 = (uint64_t)grid * kWaves * kSpan * 4;
-  return n <= round4 || 4 * round4 * sizeof(uint32_t) > round_bytes ? 4 : 16;
+// Segments per wave: 16 (128 KiB per workgroup), what its registers hold, or 4 where the
+// round size in force asks for less than that of the grid.  Fewer segments give more
+// compute units a tile, but bring nothing (2 / 4 / 8 / 16 of them: 1M elements 10.0 /
+// 10.0 / 10.1 / 10.1 us, 2M 13.1 / 10.2 / 10.1 / 10.2, 4.1M 21.5 / 14.4 / 12.1 / 12.2, 8M
+// 38.6 / 25.2 / 19.1 / 15.7).
+static int scan_segs(int grid, uint64_t round_bytes) {
+  return (uint64_t)grid * kWaves * kSpan * 16 * sizeof(uint32_t) > round_bytes ? 4 : 16;
 }
 
 static uint64_t g_scan_round_bytes = 64ull << 20;
@@ -261,12 +264,13 @@ int hs_scan_u32(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n,
   if (num_wgs > ar->view.max_blocks) return HS_ERR_INVALID;
   if (num_wgs > 3 * cus) return HS_ERR_RESIDENCY;
   // The grid that num_wgs asks for (counted in the 256-thread workgroups that
-  // d_scratch is sized by, 2 words each): workgroups of 1024 threads with 4 words
+  // d_scratch is sized by, 2 words each): workgroups of 512 threads with 4 words
   // each, 8-byte aligned, at most one per CU.  One workgroup needs no words.
   const uint32_t odd = ((uintptr_t)d_scratch & 4u) ? 1u : 0u;
   int g = (int)((2u * (uint32_t)num_wgs - odd) / 4u);
-  g = g < 1 ? 1 : g < cus ? g : cus;
-  const int segs = scan_segs(g, n, g_scan_round_bytes);
+  const int most = cus < kWg ? cus : kWg;  // a thread per word
+  g = g < 1 ? 1 : g < most ? g : most;
+  const int segs = scan_segs(g, g_scan_round_bytes);
   const void *k = segs == 4 ? scan_kernel<4>(kind, inclusive) : scan_kernel<16>(kind, inclusive);
   int rc = hs_host::check_residency(k, g, kWg, 0);
   if (rc) return rc;
