@@ -200,15 +200,18 @@ int hs_reduce_i32_stamped(hs_arena *arena, const int32_t *d_in, uint64_t n, int3
                           void *stream);
 
 /* ---- persistent u32/int32 scan (replaces sum_scan_blelloch, scan/scan_gsrb.cu:687-804) ----
-   inclusive != 0 -> inclusive scan, else exclusive (the reference's). */
+   inclusive != 0 -> inclusive scan, else exclusive (the reference's).  num_wgs: the
+   grid, served with at most one workgroup per CU; refused above 3 per CU (HS_BAR_XCD)
+   or 4.  The words that the workgroups exchange are the arena's; d_scratch must be
+   given but is not used. */
 int hs_scan_u32(hs_arena *arena, const uint32_t *d_in, uint32_t *d_out, uint64_t n,
                 int inclusive, uint32_t *d_scratch, int barrier_kind, int num_wgs,
                 void *stream);
 int hs_scan_scratch_size(int num_wgs, uint64_t n, uint64_t *elems_out);
 /* hs_scan_u32 without d_scratch, for callers that cannot allocate device memory
    (code under stream capture, serving loops, harnesses that forbid hipMalloc).
-   No reference counterpart.  The partials live in a static device array of the
-   library (32 KiB per device, held until the process ends), so the call makes no
+   No reference counterpart.  The workgroups' words live in a static device array of
+   the library (8 KiB per device, held until the process ends), so the call makes no
    allocation of its own; its address is looked up once per device by
    hs_arena_create.  Limits: num_wgs <= 4096 (the default grid is 2 per CU),
    kind != HS_BAR_COOP, the arena's device current.  Calls on one device share

@@ -262,6 +262,7 @@ int hs_arena_create(const hs_arena_desc *desc, hs_arena **out) {
   const size_t o_sem = take(sizeof(uint32_t) * (size_t)v.num_sems * v.num_groups * hs::kSemWords);
   const size_t o_ep = take(sizeof(uint32_t) * v.max_blocks);
   const size_t o_st = take(sizeof(uint32_t) * hs::kPadWords);
+  const size_t o_scan = take(sizeof(uint64_t) * 2 * kScanMaxWgs);
   a->bytes = off;
   if (hipMalloc(&a->base, a->bytes) != hipSuccess) {
     free(a);
@@ -280,6 +281,7 @@ int hs_arena_create(const hs_arena_desc *desc, hs_arena **out) {
   v.sem_queues = nullptr;
   v.episode = (uint32_t *)(b + o_ep);
   v.status = (uint32_t *)(b + o_st);
+  a->scan_words = (uint64_t *)(b + o_scan);  // a launch writes them before it reads them
   if (hipHostMalloc((void **)&a->abort_host, sizeof(uint32_t) * 64, hipHostMallocCoherent) !=
       hipSuccess) {
     (void)hipFree(a->base);

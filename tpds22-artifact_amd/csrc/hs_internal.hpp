@@ -14,9 +14,13 @@ struct hs_arena {
   void *base;              // single device allocation holding every region
   size_t bytes;
   uint32_t *abort_host;    // hipHostMalloc'd, coherent, polled by device waits
+  uint64_t *scan_words;    // [2][kScanMaxWgs] words of hs_scan_u32's workgroups
   int device;
   int num_cus;
 };
+
+// workgroups of a scan, at most (a thread of each reads one word)
+constexpr int kScanMaxWgs = 512;
 
 #define HS_TRY_HIP(expr)                                                           \
   do {                                                                             \

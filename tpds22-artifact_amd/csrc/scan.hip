@@ -20,6 +20,7 @@
 // uint32 wrap arithmetic: bit-exact for any grid and round size.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "hs_internal.hpp"
@@ -27,12 +28,11 @@
 
 using namespace hs;
 
-// Words of hs_scan_u32_noalloc: 2 of 32 bits per workgroup asked for, as
-// hs_scan_scratch_size says, for up to kNoAllocMaxWgs workgroups (32 KiB).  Each
-// device holds its own copy until the process ends; host code reaches it only
-// through the address hipGetSymbolAddress returns for the current device.
-constexpr int kNoAllocMaxWgs = 4096;
-static __device__ __align__(256) uint32_t scratch[2 * kNoAllocMaxWgs];
+// Words of hs_scan_u32_noalloc.  Each device holds its own copy until the process
+// ends; host code reaches it only through the address hipGetSymbolAddress returns for
+// the current device.
+constexpr int kNoAllocMaxWgs = 4096;  // requests above this are refused
+static __device__ __align__(256) uint64_t scratch[2 * kScanMaxWgs];
 
 namespace {
 
@@ -41,6 +41,7 @@ namespace {
 // CU; they scan 2^28 elements in 407 us against 428, 13M in 22.8 against 26.1, 8M in
 // 17.6 against 15.7).
 constexpr int kWg = 512;
+static_assert(kScanMaxWgs <= kWg, "a thread per workgroup's word");
 constexpr int kWaves = kWg / 64;
 constexpr int kSpan = 256;  // elements of a wave's segment: 4 per lane, 1 KiB per instruction
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -209,7 +210,7 @@ static uint64_t g_scan_round_bytes = 64ull << 20;
 namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
-uint32_t *g_scratch_dev[kMaxDevices];  // device address of `scratch`, per device
+uint64_t *g_scratch_dev[kMaxDevices];  // device address of `scratch`, per device
 }  // namespace
 
 namespace hs_host {
@@ -227,7 +228,7 @@ int scan_scratch_init(int device) {
             hipGetErrorString(e));
     return HS_ERR_HIP;
   }
-  g_scratch_dev[device] = (uint32_t *)p;
+  g_scratch_dev[device] = (uint64_t *)p;
   return HS_OK;
 }
 }  // namespace hs_host
@@ -254,22 +255,20 @@ int hs_scan_get_round_bytes(uint64_t *bytes_out) {
   return HS_OK;
 }
 
-int hs_scan_u32(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n, int inclusive,
-                uint32_t *d_scratch, int kind, int num_wgs, void *stream) {
-  if (!ar || !d_scratch || (n && (!d_in || !d_out))) return HS_ERR_INVALID;
+// The grid: num_wgs workgroups, at most one per CU.  Requests that 256-thread
+// workgroups could not serve are refused as they would be (3 per CU under the XCD
+// barrier, whose kernel took 136 registers, else 4).  num_wgs / 2 workgroups, as the 2
+// words of d_scratch for each would have it, take twice as long on small grids (30M
+// elements, 64 workgroups: 190 us against 93).
+static int scan_launch(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n, int inclusive,
+                       uint64_t *words, int kind, int num_wgs, void *stream) {
   if (((uintptr_t)d_in & 15u) || ((uintptr_t)d_out & 15u)) return HS_ERR_INVALID;
   if (!scan_kernel<4>(kind, inclusive)) return HS_ERR_INVALID;
   const int cus = hs_host::device_cus();
   if (num_wgs <= 0) num_wgs = 2 * cus;
   if (num_wgs > ar->view.max_blocks) return HS_ERR_INVALID;
-  if (num_wgs > 3 * cus) return HS_ERR_RESIDENCY;
-  // The grid that num_wgs asks for (counted in the 256-thread workgroups that
-  // d_scratch is sized by, 2 words each): workgroups of 512 threads with 4 words
-  // each, 8-byte aligned, at most one per CU.  One workgroup needs no words.
-  const uint32_t odd = ((uintptr_t)d_scratch & 4u) ? 1u : 0u;
-  int g = (int)((2u * (uint32_t)num_wgs - odd) / 4u);
-  const int most = cus < kWg ? cus : kWg;  // a thread per word
-  g = g < 1 ? 1 : g < most ? g : most;
+  if (num_wgs > (kind == HS_BAR_XCD ? 3 : 4) * cus) return HS_ERR_RESIDENCY;
+  int g = std::min({num_wgs, cus, kScanMaxWgs});
   const int segs = scan_segs(g, g_scan_round_bytes);
   const void *k = segs == 4 ? scan_kernel<4>(kind, inclusive) : scan_kernel<16>(kind, inclusive);
   int rc = hs_host::check_residency(k, g, kWg, 0);
@@ -280,11 +279,16 @@ int hs_scan_u32(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n,
   if ((uint64_t)g > tiles) g = (int)tiles;
   hipStream_t s = (hipStream_t)stream;
   if ((rc = hs_host::prepare_barrier(ar, kind, s))) return rc;
-  uint64_t *words = (uint64_t *)(d_scratch + odd);
   hs::ArenaView v = ar->view;
   uint32_t ng = (uint32_t)v.num_groups, nx = (uint32_t)hs_host::xcd_groups(g);
   void *args[] = {(void *)&v, (void *)&d_in, (void *)&d_out, (void *)&n, (void *)&words, (void *)&ng, (void *)&nx};
   return hs_host::launch_persistent(k, args, kind, g, kWg, 0, s);
+}
+
+int hs_scan_u32(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n, int inclusive,
+                uint32_t *d_scratch, int kind, int num_wgs, void *stream) {
+  if (!ar || !d_scratch || (n && (!d_in || !d_out))) return HS_ERR_INVALID;
+  return scan_launch(ar, d_in, d_out, n, inclusive, ar->scan_words, kind, num_wgs, stream);
 }
 
 int hs_scan_u32_noalloc(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uint64_t n, int inclusive,
@@ -304,7 +308,7 @@ int hs_scan_u32_noalloc(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uin
   int dev = -1;
   HS_TRY_HIP(hipGetDevice(&dev));
   if (dev != ar->device || dev < 0 || dev >= kMaxDevices) return HS_ERR_INVALID;
-  uint32_t *p;
+  uint64_t *p;
   {
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     p = g_scratch_dev[dev];
@@ -313,7 +317,7 @@ int hs_scan_u32_noalloc(hs_arena *ar, const uint32_t *d_in, uint32_t *d_out, uin
     fprintf(stderr, "libhs: hs_scan_u32_noalloc: no scratch address for device %d\n", dev);
     return HS_ERR_NOT_INIT;
   }
-  return hs_scan_u32(ar, d_in, d_out, n, inclusive, p, kind, num_wgs, stream);
+  return scan_launch(ar, d_in, d_out, n, inclusive, p, kind, num_wgs, stream);
 }
 
 }  // extern "C"
