@@ -23,6 +23,12 @@ class Work:
             self.src = int(np.argmax(np.diff(row.astype(np.int64))))
             self.out = torch.empty(self.g.n, dtype=torch.int32, device="cuda")
             self.work = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+        elif name == "batch":
+            lens = np.exp2(np.random.default_rng(4).uniform(0, 21, 90)).astype(np.int64)
+            self.off = np.concatenate([[3], 3 + np.cumsum(np.concatenate([lens, [7 << 22]]))]).astype(np.uint64)
+            self.x = torch.empty(int(self.off[-1]), dtype=torch.int32, device="cuda")
+            hs.gen_uniform_u32(self.x, 7, 0, 2**32 - 1)
+            self.out = torch.zeros_like(self.x)
         else:
             n = 9_000_001  # more than a round of half the CUs' registers
             self.x = torch.empty(n, dtype=torch.int32, device="cuda")
@@ -39,6 +45,8 @@ class Work:
                 G.bfs(self.arena, self.g, self.src, level=self.out, work=self.work, sync=False)
             elif self.name == "sssp":
                 G.sssp(self.arena, self.g, self.src, dist=self.out, work=self.work, sync=False)
+            elif self.name == "batch":
+                self.hs.scan_batch_u32(self.x, self.off, out=self.out, sync=False)
             else:
                 self.hs.scan_u32(self.arena, self.x, out=self.out, scratch=self.scratch, sync=False)
 
@@ -49,6 +57,11 @@ class Work:
             assert np.array_equal(got, oracle.bfs(self.g.h_row, self.g.h_col, self.src))
         elif self.name == "sssp":
             assert np.array_equal(got, oracle.sssp(self.g.h_row, self.g.h_col, self.g.h_w, self.src))
+        elif self.name == "batch":
+            stream.synchronize()
+            x = oracle.gen_uniform_u32(7, got.size, 0, 2**32 - 1)
+            for a, b in zip(self.off[:-1].astype(int), self.off[1:].astype(int)):
+                assert np.array_equal(got[a:b].view(np.uint32), np.cumsum(x[a:b], dtype=np.uint32))
         else:
             x = oracle.gen_uniform_u32(6, got.size, 0, 2**32 - 1)
             assert np.array_equal(got.view(np.uint32), np.cumsum(x, dtype=np.uint32))
@@ -57,7 +70,7 @@ class Work:
         self.arena.close()
 
 
-NAMES = ["bfs", "sssp", "scan"]
+NAMES = ["bfs", "sssp", "scan", "batch"]
 
 
 @pytest.mark.parametrize("a", NAMES)

@@ -20,6 +20,9 @@ DEFAULT = {
     r"5k_bfsI": ("graph", 512, 1),
     r"6k_ssspI": ("graph", 512, 1),
     r"10k_scan_u32I": ("scan", 512, 1),
+    # no workgroup of these waits for one that has not started: one has to find room
+    r"12k_scan_batchI": ("batch", 512, 1),
+    r"14k_reduce_batch": ("batch", 256, 1),
 }
 
 

@@ -39,15 +39,22 @@ namespace {
 constexpr int kWg = 256;  // prep and reduce
 constexpr int kWaves = kWg / 64;
 // Shapes of the scan's tiles: workgroup size and wave span in 256-element segments
-// (4 registers per lane each).
-struct Large { static constexpr int kWg = 1024, kSegs = 16; };  // 65536 elements (256 KiB), one workgroup per CU
-struct Small { static constexpr int kWg = 1024, kSegs = 4; };   // 16384 elements
+// (4 registers per lane each).  With 128 registers a workgroup is half of a CU: two run
+// on each, and one finds room beside the serving loop's workgroup (1024 threads, one
+// workgroup per CU, waited there until the loop's end; 512 ragged segments in 392 us
+// against 399, one of 2^24 elements in 53 against 58).
+// Early: the next tile is claimed when this one's carry is known, so that the atomic's
+// round trip runs beside the stores (one segment of 2^22 elements 38.1 -> 35.2 us).
+// With large tiles it starts them out of order, and the look-backs wait (2^27: 229 ->
+// 239 us).
+struct Large { static constexpr int kWg = 512, kSegs = 16; static constexpr bool kEarly = false; };  // 32768 elements
+struct Small { static constexpr int kWg = 512, kSegs = 8; static constexpr bool kEarly = true; };    // 16384 elements
 constexpr int kSegsReduce = 8;
 // Elements from which a scan takes the large tiles (one segment, us per call with
-// small and large tiles: 2^22 35.8 / 45.5, 2^23 43.2 / 46.0, 2^24 58.4 / 54.5, 2^25
-// 89.5 / 78.9, 2^27 280 / 224): more elements per tile mean fewer look-backs and
-// claims, fewer mean that more compute units have one.
-constexpr uint64_t kLargeFrom = 3ull << 22;
+// small and large tiles: 2^22 35.2 / 43.9, 2^23 44.8 / 45.8, 2^24 57.7 / 59.2, 2^24.6
+// 72.4 / 73.3, 2^25 87.3 / 82.9, 2^27 260 / 229): more elements per tile mean fewer
+// look-backs and claims, fewer mean that more compute units have one.
+constexpr uint64_t kLargeFrom = 7ull << 22;
 constexpr uint64_t kFlagAgg = 1, kFlagInc = 2;
 constexpr uint32_t kSpinLimit = 1u << 26;
 
@@ -200,11 +207,7 @@ template <class T, bool INCLUSIVE>
 __global__ void __launch_bounds__(T::kWg) __attribute__((amdgpu_waves_per_eu(4))) k_scan_batch(BatchArgs p) {
   constexpr int SEGS = T::kSegs;
   constexpr uint32_t kSpan = span_of(SEGS), kWaves = T::kWg / 64;
-  // one workgroup per CU claims its next tile when this one's carry is known, so
-  // the atomic's round trip runs beside the stores (403 -> 391 us for 512
-  // segments); with more of them tiles then start out of order, and the
-  // look-backs wait (401 -> 413 us)
-  constexpr bool kEarly = T::kWg == 1024;
+  constexpr bool kEarly = T::kEarly;
   __shared__ uint32_t s_tile, s_prefix;
   __shared__ uint32_t s_wave[kWaves], s_seen[kWaves], s_fh0;
   __shared__ uint32_t s_bits[kWaves][kSpan / 32];
@@ -457,7 +460,7 @@ uint64_t batch_bytes(const Shape &sh, uint32_t nseg) {
   const uint64_t cells = 2ull * nseg + 4 + (sh.hi - sh.lo + 3ull * nseg) / 32768;
   return 512 + 2 * (16 * sizeof(uint32_t) + sizeof(uint64_t)) * cells;
 }
-static_assert(tile_of<Small>() == 16384 && Small::kWg == 1024, "batch_bytes counts these tiles and spans");
+static_assert(tile_of<Small>() == 16384 && Small::kWg <= 1024, "batch_bytes counts these tiles, with 16 spans at most");
 
 template <class T>
 const void *scan_kernel(int inclusive) {
