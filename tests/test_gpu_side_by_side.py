@@ -17,11 +17,11 @@ class Work:
         import torch
         import hsync.graph as G
         self.hs, self.name, self.arena = hs, name, hs.Arena()
-        if name in ("bfs", "sssp"):
-            row, col = G.rmat_csr(14, 16, 5)
+        if name in ("bfs", "sssp", "pagerank"):
+            row, col = G.rmat_csr(18 if name == "pagerank" else 14, 16, 5)
             self.g = G.Graph(row, col, G.weights(col.size, 5))
             self.src = int(np.argmax(np.diff(row.astype(np.int64))))
-            self.out = torch.empty(self.g.n, dtype=torch.int32, device="cuda")
+            self.out = torch.empty(self.g.n, dtype=torch.float32 if name == "pagerank" else torch.int32, device="cuda")
             self.work = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
         elif name == "batch":
             lens = np.exp2(np.random.default_rng(4).uniform(0, 21, 90)).astype(np.int64)
@@ -45,6 +45,8 @@ class Work:
                 G.bfs(self.arena, self.g, self.src, level=self.out, work=self.work, sync=False)
             elif self.name == "sssp":
                 G.sssp(self.arena, self.g, self.src, dist=self.out, work=self.work, sync=False)
+            elif self.name == "pagerank":
+                G.pagerank(self.arena, self.g, rank=self.out, work=self.work, sync=False)
             elif self.name == "batch":
                 self.hs.scan_batch_u32(self.x, self.off, out=self.out, sync=False)
             else:
@@ -57,6 +59,9 @@ class Work:
             assert np.array_equal(got, oracle.bfs(self.g.h_row, self.g.h_col, self.src))
         elif self.name == "sssp":
             assert np.array_equal(got, oracle.sssp(self.g.h_row, self.g.h_col, self.g.h_w, self.src))
+        elif self.name == "pagerank":
+            want, _ = oracle.pagerank(self.g.h_row, self.g.h_col, alpha=0.85, tol=1e-6, max_iter=1000)
+            assert float(np.abs(got - want).max()) < 1e-6
         elif self.name == "batch":
             stream.synchronize()
             x = oracle.gen_uniform_u32(7, got.size, 0, 2**32 - 1)
@@ -70,7 +75,7 @@ class Work:
         self.arena.close()
 
 
-NAMES = ["bfs", "sssp", "scan", "batch"]
+NAMES = ["bfs", "sssp", "scan", "batch", "pagerank"]
 
 
 @pytest.mark.parametrize("a", NAMES)

@@ -19,6 +19,8 @@ VGPRS, LDS = 512, 160 * 1024  # per SIMD and lane, per CU
 DEFAULT = {
     r"5k_bfsI": ("graph", 512, 1),
     r"6k_ssspI": ("graph", 512, 1),
+    r"10k_pagerankILi\dELi3E": ("graph", 256, 3),
+    r"10k_pagerankILi\dELi1E": ("graph", 256, 4),
     r"10k_scan_u32I": ("scan", 512, 1),
     # no workgroup of these waits for one that has not started: one has to find room
     r"12k_scan_batchI": ("batch", 512, 1),

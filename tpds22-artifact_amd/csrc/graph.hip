@@ -2162,11 +2162,14 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
 // in 2^-60 fixed point (integer sums: the same bits whatever the grid or the
 // order).  Every order is fixed by the graph alone, so the ranks do not depend on
 // the grid.
-// R-MAT 22: 0.39 ms an iteration (0.45 with 64-vertex blocks, hub chunks and
+// R-MAT 22: 0.42 ms an iteration (0.45 with 64-vertex blocks, hub chunks and
 // segmented FP32 scans), 64M gathers that each miss the L1 (128-byte lines, 16 MB of
-// contributions): 0.6 requests per clock and L2 channel.  Streaming gathers take
-// twice as long, agent-scope ones the same; 512 positions per span 0.44 ms.
-constexpr int kPrQuads = 4;                   // S = 1024, of small graphs 256
+// contributions) and are bound by how many are in flight.  Streaming gathers take
+// twice as long, agent-scope ones the same.  768 positions and 3 workgroups per CU are
+// 240 of a SIMD's 512 registers and 74 KB of LDS, so that another launch or the
+// serving loop fits beside them; in that room 512 positions and 4 workgroups take 0.44
+// ms, 1024 and 2 0.46 ms (with 4, which fill the CU, 0.39 ms).
+constexpr int kPrQuads = 3;                   // S = 768, of small graphs 256
 constexpr uint64_t kPrLargeFrom = 1ull << 22;  // vertices and edges from which spans are large
 
 struct PrArgs {
@@ -2238,7 +2241,7 @@ __device__ __forceinline__ double ld_f64(const double *q) {
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int KIND, int QUADS>
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(QUADS > 2 ? 4 : 8)))
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(QUADS > 1 ? 6 : 8)))
 k_pagerank(ArenaView a, PrArgs p) {
   constexpr uint32_t S = 256 * QUADS;
   __shared__ __align__(16) double pre_s[kWg / 64][S + 2];
@@ -2678,11 +2681,11 @@ int hs_pagerank_f32(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row,
     return HS_ERR_INVALID;
   const void *k = pr_large(n, m) ? HS_KIND_SWITCH(k_pagerank_large, kind) : HS_KIND_SWITCH(k_pagerank_small, kind);
   if (!k) return HS_ERR_INVALID;
-  // 4 WGs/CU (what the running sums in LDS leave room for); larger requests are
-  // served with those, up to 8 per CU
-  const int cus = hs_host::device_cus();
+  // 3 WGs/CU (small graphs: 4), half of the registers; larger requests are served with
+  // those, up to 8 per CU
+  const int cus = hs_host::device_cus(), per = pr_large(n, m) ? 3 : 4;
   if (num_wgs > 8 * cus) return HS_ERR_RESIDENCY;
-  const int g = grid_for(k, ar, num_wgs > 4 * cus ? std::min(4 * cus, hs_host::default_grid(k, kWg, 4)) : num_wgs, 4);
+  const int g = grid_for(k, ar, num_wgs > per * cus ? hs_host::default_grid(k, kWg, per) : num_wgs, per);
   if (g < 0 || g > 4096) return HS_ERR_RESIDENCY;
   hipStream_t s = (hipStream_t)stream;
   int rc = hs_host::prepare_barrier(ar, kind, s);
