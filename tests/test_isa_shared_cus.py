@@ -27,6 +27,10 @@ DEFAULT = {
     r"14k_reduce_batch": ("batch", 256, 1),
 }
 
+# the 64-source SSSP by kind: workgroups per CU, and the registers that these launches
+# leave to others (what 4 workgroups of 113 and of 104 registers left)
+MSSP = {r"6k_msspILi2E": (6, 480), r"6k_msspILi[013-7]E": (5, 416)}
+
 
 def _granule(v):
     return -(-v // 8) * 8
@@ -48,7 +52,7 @@ def kernel_lds(asm):
 @pytest.fixture(scope="module")
 def asm():
     from concurrent.futures import ThreadPoolExecutor
-    names = sorted({"serve"} | {f for f, _, _ in DEFAULT.values()})
+    names = sorted({"serve"} | {f for f, _, _ in DEFAULT.values()} | {"mssp"})
     with ThreadPoolExecutor(max_workers=4) as ex:
         return dict(zip(names, ex.map(lambda n: _compile(os.path.join(CSRC, n + ".hip")), names)))
 
@@ -67,3 +71,14 @@ def test_default_launches_leave_room_for_another(asm):
             took = per_cu * threads // 256 * _granule(regs[k][1])
             assert took <= VGPRS // 2, (k, took)
             assert per_cu * lds[k] <= LDS // 2, (k, lds[k])
+
+
+@pytest.mark.skipif(not _HAVE_HIPCC, reason="hipcc absent")
+def test_mssp_leaves_what_it_left(asm):
+    regs, lds = kernel_registers(asm["mssp"]), kernel_lds(asm["mssp"])
+    for pattern, (per_cu, most) in MSSP.items():
+        hits = [k for k in regs if re.search(pattern, k)]
+        assert hits, pattern
+        for k in hits:
+            assert per_cu * _granule(regs[k][1]) <= most, (k, regs[k])
+            assert per_cu * lds[k] <= LDS

@@ -411,11 +411,18 @@ int hs_mssp(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row, const u
     return HS_ERR_INVALID;
   const void *k = HS_KIND_SWITCH(k_mssp, kind);
   if (!k) return HS_ERR_INVALID;
-  // 6 workgroups per CU, what 80 registers leave room for (R-MAT 21, 64 sources:
-  // 20.5 / 17.7 / 17.0 / 20.4 ms at 4 / 5 / 6 / 8, where 8 spill): the relaxation is
-  // bound by the gathers in flight
-  if (num_wgs <= 0) num_wgs = std::min(hs_host::default_grid(k, kWg, 6), (int)ar->view.max_blocks);
+  // 6 workgroups per CU of 80 registers: the relaxation is bound by the gathers in
+  // flight (R-MAT 21, 64 sources: 20.0 / 17.7 / 16.8 ms at 4 / 5 / 6 per CU).  27-91
+  // registers are spilled for it (104-136 bytes per lane), which costs nothing that
+  // shows: 4 per CU without spills, 113 registers, take 20.0 ms as well.  5 under the
+  // other kinds, so that a sum or a barrier kernel of 48 registers still fits beside
+  // them (with 4 workgroups of 104 they took 416 of 512; under the XCD kind, of 113,
+  // 480 as now).  Grids above 4 per CU are refused, as they were then.
+  const int cus = hs_host::device_cus();
+  const bool given = num_wgs > 0;
+  if (!given) num_wgs = std::min(hs_host::default_grid(k, kWg, kind == HS_BAR_XCD ? 6 : 5), (int)ar->view.max_blocks);
   if (num_wgs > ar->view.max_blocks || num_wgs > 8192) return HS_ERR_INVALID;
+  if (given && num_wgs > 4 * cus) return HS_ERR_RESIDENCY;
   if (hs_host::check_residency(k, num_wgs, kWg, 0) != HS_OK) return HS_ERR_RESIDENCY;
   hipStream_t s = (hipStream_t)stream;
   int rc = hs_host::prepare_barrier(ar, kind, s);
