@@ -29,3 +29,28 @@ def test_mssp_grids(hs, arena, graph, oracle):
             d, _ = G.mssp(arena, graph, srcs, barrier=kind, num_wgs=wgs)
             assert np.array_equal(d.cpu().numpy(), want), (kind, wgs)
         _refused(hs, 3, lambda: G.mssp(arena, graph, srcs, barrier=kind, num_wgs=4 * cus + 1))
+
+
+def test_bfs_and_sssp_grids(hs, arena, graph, oracle):
+    import hsync.graph as G
+    cus = hs.device_info()["num_cus"]
+    src = int(np.argmax(np.diff(graph.h_row.astype(np.int64))))
+    lv, ds = oracle.bfs(graph.h_row, graph.h_col, src), oracle.sssp(graph.h_row, graph.h_col, graph.h_w, src)
+    for wgs in (0, 2, 3, 9, cus // 2 + 1, cus, cus + 1, 8 * cus):
+        assert np.array_equal(G.bfs(arena, graph, src, num_wgs=wgs)[0].cpu().numpy(), lv), wgs
+        assert np.array_equal(G.sssp(arena, graph, src, num_wgs=wgs)[0].cpu().numpy(), ds), wgs
+    for call in (lambda: G.bfs(arena, graph, src, num_wgs=8 * cus + 1), lambda: G.sssp(arena, graph, src, num_wgs=8 * cus + 1)):
+        _refused(hs, 3, call)
+
+
+def test_the_grid_is_the_request(hs, graph):
+    """An arena of 3 barrier slots serves a grid of 3 and of less, and refuses 4."""
+    import hsync.graph as G
+    a = hs.Arena(max_blocks=3)
+    try:
+        for call in (G.bfs, G.sssp):
+            for wgs in (0, 3):
+                call(a, graph, 0, num_wgs=wgs)
+            _refused(hs, 3, lambda: call(a, graph, 0, num_wgs=4))
+    finally:
+        a.close()

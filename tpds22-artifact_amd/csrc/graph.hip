@@ -2433,16 +2433,13 @@ constexpr auto k_pagerank_small = k_pagerank<KIND, 1>;
 
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
-// Grid of a kernel of kTeamWg-thread workgroups for a request of num_wgs
-// workgroups of kWg threads (0: one workgroup per CU), at most one per CU.
-// Requests that kWg-thread workgroups could not serve (8 per CU) are refused as
-// they would be there.
+// Grid of a kernel of kTeamWg-thread workgroups: num_wgs of them (0: one per CU), at
+// most one per CU.  Requests that kWg-thread workgroups could not serve (8 per CU) are
+// refused as they would be there.
 int team_grid_for(const void *k, hs_arena *ar, int num_wgs) {
-  constexpr int kPer = kTeamWg / kWg;
   const int cus = hs_host::device_cus();
   if (num_wgs > 8 * cus || num_wgs > ar->view.max_blocks) return -1;
-  int g = num_wgs > 0 ? (num_wgs + kPer - 1) / kPer : cus;
-  g = std::min({g, cus, ar->view.max_blocks});
+  const int g = std::min({num_wgs > 0 ? num_wgs : cus, cus, ar->view.max_blocks});
   return hs_host::check_residency(k, g, kTeamWg, 0) == HS_OK ? g : -1;
 }
 
