@@ -149,6 +149,7 @@ int main(int argc, char **argv) {
     for (uint32_t size = 1; size <= grid; ++size) {
       bad += team_usable(size, grid, false);
       bad += team_usable(size, grid, true) != (size < grid && size <= 32);
+      bad += team_edges(size) != size * team_edges(32) / 32;  // a small team takes its share
     }
   printf("launches %ld reads %ld failures %ld\n", launches, reads, bad);
   return bad ? 1 : 0;

@@ -993,7 +993,6 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 constexpr int kTeamWg = 512;
 using hs_rounds::kTeamMax;                  // workgroups of a team
 constexpr uint32_t kTeamRounds = 256;
-constexpr uint64_t kTeamEdges = 1ull << 17;  // edges of a round up to which the team runs it
 constexpr uint32_t kTeamIdleSleep = 32;     // s_sleep units between the idle workgroups' polls
 constexpr uint32_t kSegCap = 2048;          // entries of a workgroup's output segment; the rest goes to the queue
 constexpr uint32_t kSegBlock = 16;          // entries a wave takes at once: 4 lanes each
@@ -1078,6 +1077,7 @@ struct Team {
   uint64_t *word;       // [2][kTeamMax] episode << 32 | segment word, zero before the first grid barrier
   uint32_t size, rank;  // rank: position in the team (workgroups outside it: any value)
   bool in, usable;
+  uint64_t most;  // edges of a round that the team runs
   uint32_t episode;
 
   __device__ void init(uint64_t *w, uint32_t nxcd, bool bounded) {
@@ -1087,6 +1087,7 @@ struct Team {
     rank = blockIdx.x / x;
     in = blockIdx.x % x == 0;
     usable = hs_rounds::team_usable(size, gridDim.x, bounded);
+    most = hs_rounds::team_edges(size);
     episode = 0;
   }
   // Barrier of the team; `mine` (thread 0): this workgroup's segment word, `seg`:
@@ -1686,7 +1687,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   auto edges = [&]() { return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk; };
   while (in.any()) {
     const uint64_t ahead = edges();
-    const bool by_team = team.usable && ahead <= kTeamEdges;
+    const bool by_team = team.usable && ahead <= team.most;
     // Pull once the frontier's edges are 1/kPullEdges of those left (they are
     // estimated by the mean degree, which a frontier of hubs exceeds).  Any factor
     // from 4 to 64 gives the same times at R-MAT 12..22; 2 costs 45% at R-MAT 22.
@@ -1720,7 +1721,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
         if (team.sync(a, out.segment_word(par), in.seg)) return;
         in.nin = in.nh = 0;
         if (in.seg.queued) look(round);
-        if (!in.any() || edges() > kTeamEdges) break;
+        if (!in.any() || edges() > team.most) break;
         behind += edges();
       }
       if (t0 < 64) {
@@ -2081,8 +2082,8 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   bool told = false;  // the input is a stretch's report
   auto small = [&]() {
     if (!team.usable) return false;
-    if (!in.near()) return in.nfar <= kTeamEdges / 4;
-    return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk <= kTeamEdges;
+    if (!in.near()) return in.nfar <= team.most / 4;
+    return (uint64_t)(in.seg.total + in.nin) * p.mean_degree + (uint64_t)in.nh * kBfsChunk <= team.most;
   };
   while (in.near() || in.nfar != 0) {
     const bool by_team = small();
