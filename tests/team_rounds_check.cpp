@@ -151,6 +151,12 @@ int main(int argc, char **argv) {
       bad += team_usable(size, grid, true) != (size < grid && size <= 32);
       bad += team_edges(size) != size * team_edges(32) / 32;  // a small team takes its share
     }
+  // a mesh of mean degree 3.4, counted as 4, 1000 levels of 1000 vertices: never pulled;
+  // a power-law graph's wide levels: pulled, its first and last: not
+  for (uint64_t level = 0; level < 1000; ++level) bad += pull_pays(4000, 4000 * level, 3400000, 1000000);
+  const uint64_t n = 1 << 22, m = 16 * n;
+  bad += pull_pays(16, 0, m, n) || pull_pays(16 * 20000, 16, m, n) || pull_pays(16 * 400, m, m, n);
+  bad += !pull_pays(m / 6, m / 100, m, n) || !pull_pays(m / 2, m / 5, m, n) || !pull_pays(n, m, m, n);
   printf("launches %ld reads %ld failures %ld\n", launches, reads, bad);
   return bad ? 1 : 0;
 }

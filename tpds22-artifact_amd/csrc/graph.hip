@@ -1544,7 +1544,6 @@ __device__ __forceinline__ bool bf_in_frontier(const uint64_t *fbm, uint32_t u) 
 // wave, in rounds of 8, 16, ... 256 edges each, so that a vertex that finds its
 // parent early costs no more.  What is left of a vertex with more than kPullRest
 // in-edges becomes chunks that all waves share after the level's barrier.
-constexpr uint64_t kPullEdges = 8;
 constexpr uint32_t kPullFirst = 4, kPullRest = 8192, kPullChunk = 4096;
 
 __device__ __forceinline__ void bf_pull_found(BfStep &s, bool found, uint32_t v) {
@@ -1688,10 +1687,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   while (in.any()) {
     const uint64_t ahead = edges();
     const bool by_team = team.usable && ahead <= team.most;
-    // Pull once the frontier's edges are 1/kPullEdges of those left (they are
-    // estimated by the mean degree, which a frontier of hubs exceeds).  Any factor
-    // from 4 to 64 gives the same times at R-MAT 12..22; 2 costs 45% at R-MAT 22.
-    const bool pull = p.rrow && !by_team && ahead * kPullEdges > (p.m > behind ? p.m - behind : 0);
+    const bool pull = p.rrow && !by_team && hs_rounds::pull_pays(ahead, behind, p.m, p.n);
     if (pull && !have_bitmap) {
       bf_make_bitmap(p, r, all);
       if (gb.sync<KIND>()) return;

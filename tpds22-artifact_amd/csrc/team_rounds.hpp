@@ -63,6 +63,17 @@ HS_ROUND_FN bool team_usable(uint32_t size, uint32_t grid, bool bounded) {
 // ms, 24 so, 37 without a team).
 HS_ROUND_FN uint64_t team_edges(uint32_t size) { return 4096ull * size; }
 
+// Whether a BFS pulls a level whose frontier has `ahead` of the graph's m edges, when
+// `behind` were those of the levels before (both by the mean degree, which a frontier of
+// hubs exceeds).  It has to be 1/8 of the edges left: any factor from 4 to 64 gives the
+// same times at R-MAT 12..22; 2 costs 45% at R-MAT 22.  And as a pull looks at every
+// vertex, whatever the frontier is, 1/16 of the vertices: the rounded-up mean degree
+// runs out of edges before a mesh or a road network ends, and with the first rule alone
+// a grid without a team then pulled every narrow level that was left.
+HS_ROUND_FN bool pull_pays(uint64_t ahead, uint64_t behind, uint64_t m, uint64_t n) {
+  return ahead * 8 > (m > behind ? m - behind : 0) && ahead * 16 > n;
+}
+
 // the counters that round i of a side clears for the rounds after it
 template <class Clear>
 HS_ROUND_FN void open_round(Side side, uint32_t i, Clear clear) {
