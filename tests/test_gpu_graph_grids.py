@@ -54,3 +54,19 @@ def test_the_grid_is_the_request(hs, graph):
             _refused(hs, 3, lambda: call(a, graph, 0, num_wgs=4))
     finally:
         a.close()
+
+
+def test_pagerank_grids(hs, arena, graph):
+    import torch
+    import hsync.graph as G
+    cus = hs.device_info()["num_cus"]
+    want, _ = G.pagerank(arena, graph)
+    a = hs.Arena(max_blocks=5 * cus)
+    try:
+        for wgs in (0, 1, 4 * cus, 5 * cus):
+            assert torch.equal(G.pagerank(a, graph, num_wgs=wgs)[0], want), wgs
+        _refused(hs, 3, lambda: G.pagerank(a, graph, num_wgs=5 * cus + 1))  # more than the arena's slots
+    finally:
+        a.close()
+    assert torch.equal(G.pagerank(arena, graph, num_wgs=8 * cus)[0], want)
+    _refused(hs, 3, lambda: G.pagerank(arena, graph, num_wgs=8 * cus + 1))

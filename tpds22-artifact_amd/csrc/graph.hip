@@ -2678,7 +2678,7 @@ int hs_pagerank_f32(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row,
   // 3 WGs/CU (small graphs: 4), half of the registers; larger requests are served with
   // those, up to 8 per CU
   const int cus = hs_host::device_cus(), per = pr_large(n, m) ? 3 : 4;
-  if (num_wgs > 8 * cus) return HS_ERR_RESIDENCY;
+  if (num_wgs > 8 * cus || num_wgs > ar->view.max_blocks) return HS_ERR_RESIDENCY;
   const int g = grid_for(k, ar, num_wgs > per * cus ? hs_host::default_grid(k, kWg, per) : num_wgs, per);
   if (g < 0 || g > 4096) return HS_ERR_RESIDENCY;
   hipStream_t s = (hipStream_t)stream;
