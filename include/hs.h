@@ -324,12 +324,12 @@ int hs_tune_reduce_i32(hs_arena *arena, const int32_t *d_in, uint64_t n, int rep
    keeps at least 4 members); apply out->xcd_groups with hs_set_xcd_groups */
 int hs_tune_barrier(hs_arena *arena, float *d_storage, int num_wgs, int wg_size, int num_ldst,
                     int episodes, int reps, hs_tune_result *out, void *stream);
-/* hs_scan_u32 (grid 1/2/4 per CU x round 32/64/192 MiB, and 2x the XCD groups)
-   and the look-back scan (2/4/8 per CU); the process's round size and XCD
-   groups are left as they were */
+/* hs_scan_u32 (grid 1/2 and 1 per CU x 128 and 32 KiB per workgroup and round, and
+   2x the XCD groups) and the look-back scan (1/2 per CU); the process's round size
+   and XCD groups are left as they were */
 int hs_tune_scan_u32(hs_arena *arena, const uint32_t *d_in, uint32_t *d_out, uint64_t n,
                      int inclusive, int reps, hs_tune_result *out, void *stream);
-/* hs_scan_batch_u32: workgroups per CU 1/2/4/8 (the batch's carries pass by
+/* hs_scan_batch_u32: workgroups per CU 1/2 (the batch's carries pass by
    look-back, so there is no barrier to tune); out->num_wgs is the grid to pass */
 int hs_tune_scan_batch_u32(const uint32_t *d_in, uint32_t *d_out, const uint64_t *d_offsets,
                            const uint64_t *h_offsets, uint32_t nseg, int inclusive, int reps,

@@ -114,7 +114,8 @@ int hs_pagerank_f32(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uin
 
 /* autotuners of the graph launches (the role of LONESTAR/tuning/bfstuner.py,
    which searches the block factor of LONESTAR/apps/bfs/kernel_gsrb.cu:716-719):
-   workgroups per CU 1/2/4/8 x barrier (XCD, XCD with 2x the groups, two-level),
+   the grids that a launch serves (BFS 1/4, 1/2, 1 workgroup per CU, the others 1, 2, 4,
+   PageRank on large graphs 3) x barrier (XCD, XCD with 2x the groups, two-level),
    each timed `reps` times after a warm-up on the caller's graph; the default
    configuration is timed first and the choice is never slower than it in the
    same call.  Every configuration computes the same result (it is left in the
@@ -123,6 +124,10 @@ int hs_pagerank_f32(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uin
 int hs_tune_bfs(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uint32_t *d_row,
                 const uint32_t *d_col, int32_t src, int32_t *d_level, int reps, hs_tune_result *out,
                 void *stream);
+/* of hs_bfs_dir */
+int hs_tune_bfs_dir(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uint32_t *d_row,
+                    const uint32_t *d_col, const uint32_t *d_rrow, const uint32_t *d_rcol, int32_t src,
+                    int32_t *d_level, int reps, hs_tune_result *out, void *stream);
 int hs_tune_msbfs(hs_arena *arena, uint32_t nnodes, uint64_t nedges, const uint32_t *d_row,
                   const uint32_t *d_col, const uint32_t *d_rrow, const uint32_t *d_rcol,
                   const int32_t *d_srcs, int nsrc, int32_t *d_levels, int schedule, const float *d_mlp,

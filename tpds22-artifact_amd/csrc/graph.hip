@@ -2658,6 +2658,13 @@ static uint64_t pr_spans(uint32_t n, uint64_t m) {
   return (n + m + S - 1) / S;
 }
 
+}  // extern "C"
+
+// half of a CU's registers
+int hs_host::pagerank_wgs_per_cu(uint32_t n, uint64_t m) { return pr_large(n, m) ? 3 : 4; }
+
+extern "C" {
+
 int hs_pagerank_work_size(uint32_t n, uint64_t m, uint64_t *bytes) {
   if (!bytes) return HS_ERR_INVALID;
   const uint64_t ns = std::max(pr_spans(n, m), (std::min(n + m, kPrLargeFrom) + 255) / 256) + 1;  // grows with n and m
@@ -2675,9 +2682,8 @@ int hs_pagerank_f32(hs_arena *ar, uint32_t n, uint64_t m, const uint32_t *d_row,
     return HS_ERR_INVALID;
   const void *k = pr_large(n, m) ? HS_KIND_SWITCH(k_pagerank_large, kind) : HS_KIND_SWITCH(k_pagerank_small, kind);
   if (!k) return HS_ERR_INVALID;
-  // 3 WGs/CU (small graphs: 4), half of the registers; larger requests are served with
-  // those, up to 8 per CU
-  const int cus = hs_host::device_cus(), per = pr_large(n, m) ? 3 : 4;
+  // larger requests than the default are served with it, up to 8 per CU
+  const int cus = hs_host::device_cus(), per = hs_host::pagerank_wgs_per_cu(n, m);
   if (num_wgs > 8 * cus || num_wgs > ar->view.max_blocks) return HS_ERR_RESIDENCY;
   const int g = grid_for(k, ar, num_wgs > per * cus ? hs_host::default_grid(k, kWg, per) : num_wgs, per);
   if (g < 0 || g > 4096) return HS_ERR_RESIDENCY;

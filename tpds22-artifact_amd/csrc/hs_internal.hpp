@@ -51,6 +51,8 @@ int finish(hs_arena *arena, hipStream_t stream);
 int arena_init_words(hs_arena *arena, hipStream_t stream);
 // default persistent grid: wgs_per_cu * CUs capped by residency
 int default_grid(const void *kernel, int wg_size, int wgs_per_cu);
+// workgroups per CU of a default hs_pagerank_f32 launch
+int pagerank_wgs_per_cu(uint32_t n, uint64_t m);
 // records the current device's address of hs_scan_u32_noalloc's static scratch
 int scan_scratch_init(int device);
 // zero the barrier state a persistent launch of `kind` needs (capture-safe fills)

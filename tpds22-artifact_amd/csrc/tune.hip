@@ -12,6 +12,7 @@
 // default as measured in the same call.
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
 #include <vector>
 
 #include "hs_graph.h"
@@ -147,10 +148,15 @@ int hs_tune_scan_u32(hs_arena *a, const uint32_t *d_in, uint32_t *d_out, uint64_
   hs_scan_get_round_bytes(&round0);
   const int x = hs_host::device_xcds();
   std::vector<Cand> cands{{0, 0, HS_BAR_XCD, round0, 0}};
-  for (int per_cu : {1, 2, 4})
-    for (uint64_t mb : {32ull, 64ull, 192ull}) cands.push_back({0, per_cu * cus, HS_BAR_XCD, mb << 20, 0});
-  for (int per_cu : {1, 2, 4}) cands.push_back({0, per_cu * cus, HS_BAR_XCD, round0, 2 * x});  // fan-in
-  for (int per_cu : {2, 4, 8}) cands.push_back({1, per_cu * cus, 0, 0, 0});
+  // grids of more than one workgroup per CU are one of them, and a workgroup's round is
+  // 128 or 32 KiB, so more values of either would be the same launches again
+  for (int wgs : {cus, (cus + 1) / 2}) {
+    const uint64_t large = (uint64_t)wgs << 17, small = (uint64_t)wgs << 15;
+    for (uint64_t round : {large, small})
+      if (wgs != cus || (round == large) != (round0 >= large)) cands.push_back({0, wgs, HS_BAR_XCD, round, 0});
+    cands.push_back({0, wgs, HS_BAR_XCD, round0, 2 * x});  // fan-in
+  }
+  for (int per_cu : {1, 2}) cands.push_back({1, per_cu * cus, 0, 0, 0});
   uint64_t nscr = 0, nwork = 0;
   int rc = hs_scan_scratch_size(4 * cus, n, &nscr);
   if (rc) return rc;
@@ -188,16 +194,17 @@ int hs_tune_scan_u32(hs_arena *a, const uint32_t *d_in, uint32_t *d_out, uint64_
 
 namespace {
 
-// candidates of the persistent graph launches: the default first, then grid
-// (workgroups per CU) x barrier (XCD with one group per XCD, XCD with twice the
-// groups, two-level)
-std::vector<Cand> graph_cands() {
+// candidates of the persistent graph launches: the default first, then the grids that
+// the launch serves, in quarters of a workgroup per CU, x barrier (XCD with one group
+// per XCD, XCD with twice the groups, two-level).  `whole`: the default grid.
+std::vector<Cand> graph_cands(std::initializer_list<int> quarters, int whole) {
   const int cus = hs_host::device_cus(), x = hs_host::device_xcds();
   std::vector<Cand> c{{0, 0, HS_BAR_XCD, 0, 0}};
-  for (int per_cu : {1, 2, 4, 8}) {
-    c.push_back({0, per_cu * cus, HS_BAR_XCD, 0, 0});
-    c.push_back({0, per_cu * cus, HS_BAR_XCD, 0, 2 * x});
-    c.push_back({0, per_cu * cus, HS_BAR_TWO_LEVEL, 0, 0});
+  for (int q : quarters) {
+    const int wgs = (q * cus + 3) / 4;
+    if (q != whole) c.push_back({0, wgs, HS_BAR_XCD, 0, 0});
+    c.push_back({0, wgs, HS_BAR_XCD, 0, 2 * x});
+    c.push_back({0, wgs, HS_BAR_TWO_LEVEL, 0, 0});
   }
   return c;
 }
@@ -211,12 +218,9 @@ struct Scratch {
   bool alloc(uint64_t bytes) { return hipMalloc(&p, bytes ? bytes : 8) == hipSuccess; }
 };
 
-}  // namespace
-
-extern "C" {
-
-int hs_tune_bfs(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col, int32_t src,
-                int32_t *d_level, int reps, hs_tune_result *out, void *stream) {
+// BFS, with the in-edges or (null) without; the grid is at most one workgroup per CU
+int tune_bfs(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col, const uint32_t *d_rrow,
+             const uint32_t *d_rcol, int32_t src, int32_t *d_level, int reps, hs_tune_result *out, void *stream) {
   if (!a || !d_row || !d_col || !d_level || !out || n == 0 || reps < 1) return HS_ERR_INVALID;
   uint64_t nb = 0;
   int rc = hs_bfs_work_size(n, m, &nb);
@@ -224,9 +228,26 @@ int hs_tune_bfs(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, cons
   Scratch w;
   if (!w.alloc(nb)) return HS_ERR_NOMEM;
   hipStream_t s = (hipStream_t)stream;
-  return pick(a, graph_cands(), [&](const Cand &c) {
-    return hs_bfs(a, n, m, d_row, d_col, src, d_level, w.p, c.kind, c.num_wgs, nullptr, s);
+  return pick(a, graph_cands({1, 2, 4}, 4), [&](const Cand &c) {
+    return d_rrow ? hs_bfs_dir(a, n, m, d_row, d_col, d_rrow, d_rcol, src, d_level, w.p, c.kind, c.num_wgs, nullptr, s)
+                  : hs_bfs(a, n, m, d_row, d_col, src, d_level, w.p, c.kind, c.num_wgs, nullptr, s);
   }, reps, s, out);
+}
+
+}  // namespace
+
+extern "C" {
+
+int hs_tune_bfs(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col, int32_t src,
+                int32_t *d_level, int reps, hs_tune_result *out, void *stream) {
+  return tune_bfs(a, n, m, d_row, d_col, nullptr, nullptr, src, d_level, reps, out, stream);
+}
+
+int hs_tune_bfs_dir(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
+                    const uint32_t *d_rrow, const uint32_t *d_rcol, int32_t src, int32_t *d_level, int reps,
+                    hs_tune_result *out, void *stream) {
+  if (!d_rrow || !d_rcol) return HS_ERR_INVALID;
+  return tune_bfs(a, n, m, d_row, d_col, d_rrow, d_rcol, src, d_level, reps, out, stream);
 }
 
 int hs_tune_msbfs(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, const uint32_t *d_col,
@@ -242,7 +263,7 @@ int hs_tune_msbfs(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, co
   Scratch w;
   if (!w.alloc(nb)) return HS_ERR_NOMEM;
   hipStream_t s = (hipStream_t)stream;
-  return pick(a, graph_cands(), [&](const Cand &c) {
+  return pick(a, graph_cands({4, 8, 16}, 16), [&](const Cand &c) {
     return hs_msbfs(a, n, m, d_row, d_col, d_rrow, d_rcol, d_srcs, nsrc, d_levels, w.p, c.kind, c.num_wgs,
                     schedule, d_mlp, nullptr, nullptr, s);
   }, reps, s, out);
@@ -260,7 +281,7 @@ int hs_tune_mssp(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_row, con
   Scratch w;
   if (!w.alloc(nb)) return HS_ERR_NOMEM;
   hipStream_t s = (hipStream_t)stream;
-  return pick(a, graph_cands(), [&](const Cand &c) {
+  return pick(a, graph_cands({4, 8, 16}, 24), [&](const Cand &c) {
     return hs_mssp(a, n, m, d_row, d_col, d_w, d_srcs, nsrc, delta, d_dist, w.p, c.kind, c.num_wgs, nullptr, s);
   }, reps, s, out);
 }
@@ -275,7 +296,8 @@ int hs_tune_pagerank_f32(hs_arena *a, uint32_t n, uint64_t m, const uint32_t *d_
   Scratch w;
   if (!w.alloc(nb)) return HS_ERR_NOMEM;
   hipStream_t s = (hipStream_t)stream;
-  return pick(a, graph_cands(), [&](const Cand &c) {
+  const int whole = 4 * hs_host::pagerank_wgs_per_cu(n, m);
+  return pick(a, graph_cands({4, 8, whole}, whole), [&](const Cand &c) {
     return hs_pagerank_f32(a, n, m, d_row, d_rrow, d_rcol, alpha, tol_l1, max_iter, d_rank, w.p, c.kind,
                            c.num_wgs, nullptr, s);
   }, reps, s, out);
@@ -295,7 +317,7 @@ int hs_tune_scan_batch_u32(const uint32_t *d_in, uint32_t *d_out, const uint64_t
   hipStream_t s = (hipStream_t)stream;
   const int cus = hs_host::device_cus();
   std::vector<Cand> cands{{1, 0, 0, 0, 0}};
-  for (int per_cu : {1, 2, 4, 8}) cands.push_back({1, per_cu * cus, 0, 0, 0});
+  for (int per_cu : {1, 2}) cands.push_back({1, per_cu * cus, 0, 0, 0});  // larger grids are refused
   Timer t;
   if (!t.ok) return HS_ERR_HIP;
   float best = -1.f, def = -1.f;

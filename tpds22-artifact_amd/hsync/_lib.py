@@ -108,6 +108,7 @@ SIGNATURES = {
     "hs_tune_scan_u32": (_I, [_P, _P, _P, _U64, _I, _I, _P, _P]),
     "hs_tune_scan_batch_u32": (_I, [_P, _P, _P, _P, _U32, _I, _I, _P, _P]),
     "hs_tune_bfs": (_I, [_P, _U32, _U64, _P, _P, C.c_int32, _P, _I, _P, _P]),
+    "hs_tune_bfs_dir": (_I, [_P, _U32, _U64, _P, _P, _P, _P, C.c_int32, _P, _I, _P, _P]),
     "hs_tune_msbfs": (_I, [_P, _U32, _U64, _P, _P, _P, _P, _P, _I, _P, _I, _P, _I, _P, _P]),
     "hs_tune_mssp": (_I, [_P, _U32, _U64, _P, _P, _P, _P, _I, C.c_int32, _P, _I, _P, _P]),
     "hs_tune_pagerank_f32": (_I, [_P, _U32, _U64, _P, _P, _P, C.c_float, C.c_float, _I, _P, _I, _P, _P]),

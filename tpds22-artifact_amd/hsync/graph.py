@@ -282,8 +282,12 @@ def tune_bfs(arena: Arena, g: Graph, src: int, reps: int = 3, level=None, stream
     torch = _torch()
     level = level if level is not None else torch.empty(g.n, dtype=torch.int32, device="cuda")
     r = _tune_result()
-    L.check(L.load().hs_tune_bfs(arena.handle, g.n, g.m, _ptr(g.row), _ptr(g.col), src, _ptr(level), reps,
-                                 C.byref(r), _stream(stream)), "hs_tune_bfs")
+    if hasattr(g, "rrow"):  # the launch that bfs() makes
+        L.check(L.load().hs_tune_bfs_dir(arena.handle, g.n, g.m, _ptr(g.row), _ptr(g.col), _ptr(g.rrow), _ptr(g.rcol), src,
+                                         _ptr(level), reps, C.byref(r), _stream(stream)), "hs_tune_bfs_dir")
+    else:
+        L.check(L.load().hs_tune_bfs(arena.handle, g.n, g.m, _ptr(g.row), _ptr(g.col), src, _ptr(level), reps,
+                                     C.byref(r), _stream(stream)), "hs_tune_bfs")
     return r.as_dict()
 
 

@@ -106,12 +106,12 @@ class Tuner:
         offsets = [0, n]
         cands = [{"algo": "barrier", "num_wgs": 0, "barrier": "xcd",
                   "round_mb": api.get_scan_round_bytes() >> 20}]
-        for per_cu in (1, 2, 4):
-            for rmb in (32, 64, 192):
-                c = {"algo": "barrier", "num_wgs": per_cu * self.cus, "barrier": "xcd", "round_mb": rmb}
-                if c not in cands:
-                    cands.append(c)
-        for per_cu in (2, 4, 8):
+        # at most one workgroup per CU, 128 or 32 KiB of a round each
+        for wgs in (self.cus, -(-self.cus // 2)):
+            for rmb in (-(-wgs // 8), max(1, wgs // 32)):
+                if wgs != self.cus or (rmb * 8 >= wgs) != (cands[0]["round_mb"] * 8 >= wgs):
+                    cands.append({"algo": "barrier", "num_wgs": wgs, "barrier": "xcd", "round_mb": rmb})
+        for per_cu in (1, 2):
             cands.append({"algo": "lookback", "num_wgs": per_cu * self.cus})
         work = {}
         round0 = api.get_scan_round_bytes()
