@@ -624,8 +624,8 @@ __device__ __forceinline__ int sem_post_master(const ArenaView &, uint32_t *rec,
 // that times out leaves its tickets unserved: the launch has failed, and
 // hs_arena_sync / hs_arena_reset restore the records.
 // The count and the turn are one 64-bit word, so that an acquisition passes the turn
-// on in the same operation, and the turn's holder polls it without backoff: per
-// acquisition 3.7 us with the record's lock, 2.1 us with a lock-free count and the
+// on in the same operation, and the turn's holder polls it with one unit's sleep (64
+// clocks) after every other poll: per acquisition 3.7 us with the record's lock, 2.1 us with a lock-free count and the
 // turn passed on after it, 1.7 us so (1024 workgroups, 16 units, 1 writer in 10).
 // What is left is two round trips between the XCDs: the swap, and the next head's
 // read of it.

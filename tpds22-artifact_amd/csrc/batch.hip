@@ -326,8 +326,9 @@ __global__ void __launch_bounds__(T::kWg) __attribute__((amdgpu_waves_per_eu(4))
 // Each workgroup sums a contiguous share of the spans, its waves taking them in
 // turn.  No workgroup waits for another, so the shares are dealt, not claimed.
 // Spans of 2048 elements: 32 data registers per lane and 8 KiB of LDS per wave
-// leave 4 workgroups (128 KiB of loads in flight) on a CU.
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(8))) k_reduce_batch(BatchArgs p) {
+// leave 5 workgroups on a CU, of which the default grid has 4 (128 KiB of loads in
+// flight).
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(5))) k_reduce_batch(BatchArgs p) {
   constexpr uint32_t kSpan = span_of(kSegsReduce);
   __shared__ __align__(16) uint32_t s_pre[kWaves][kSpan];  // flat exclusive prefixes of a wave's span
   const uint32_t lane = lane_id(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
