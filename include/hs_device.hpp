@@ -625,10 +625,10 @@ __device__ __forceinline__ int sem_post_master(const ArenaView &, uint32_t *rec,
 // hs_arena_sync / hs_arena_reset restore the records.
 // The count and the turn are one 64-bit word, so that an acquisition passes the turn
 // on in the same operation, and the turn's holder polls it with one unit's sleep (64
-// clocks) after every other poll: per acquisition 3.7 us with the record's lock, 2.1 us with a lock-free count and the
-// turn passed on after it, 1.7 us so (1024 workgroups, 16 units, 1 writer in 10).
-// What is left is two round trips between the XCDs: the swap, and the next head's
-// read of it.
+// clocks) after every other poll: per acquisition 3.7 us with the record's lock, 2.1 us
+// with a lock-free count and the turn passed on after it, 1.7 us so (1024 workgroups,
+// 16 units, 1 writer in 10).  What is left is two round trips between the XCDs: the
+// swap, and the next head's read of it.
 __device__ __forceinline__ int sem_wait_queued_master(const ArenaView &a, uint32_t *rec,
                                                       uint32_t *qrec, bool writer, bool turns) {
   const uint32_t maxc = ld_relaxed(rec + kSemMax);
