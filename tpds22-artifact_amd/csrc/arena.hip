@@ -22,8 +22,8 @@ __global__ void k_fill_u32(uint32_t *p, size_t n, uint32_t v) {
     p[i] = v;
 }
 
-// the status word and the host's copy of it, both in stream order: work enqueued
-// before a reset may still fail, and sets both
+// the status word and the host's, both in stream order: work enqueued before a reset
+// may still fail, and sets both
 __global__ void k_clear_status(uint32_t *status, uint32_t *host) {
   if (threadIdx.x == 0) {
     hs::st_relaxed(status, 0u);
@@ -138,14 +138,16 @@ int default_grid(const void *kernel, int wg_size, int wgs_per_cu) {
 int finish(hs_arena *a, hipStream_t s) {
   HS_TRY_HIP(hipGetLastError());
   HS_TRY_HIP(hipStreamSynchronize(s));
-  // the first failure's code, written to host memory by the failing wait: a copy
-  // of the device word cost another round trip per synchronous call
-  const uint32_t st = __atomic_load_n(a->abort_host + hs::kHostStatus, __ATOMIC_SEQ_CST);
-  if (st != 0) {
+  // a failing wait says so in host memory: a copy of the status word cost another
+  // round trip per synchronous call
+  if (__atomic_load_n(a->abort_host + hs::kHostStatus, __ATOMIC_SEQ_CST) != 0) {
+    uint32_t st = 0;
+    HS_TRY_HIP(hipMemcpy(&st, a->view.status, sizeof(st), hipMemcpyDeviceToHost));
     // a failed wait leaves counters half-way through an episode and semaphore
     // records half-acquired: start clean (hs_arena_reset restores every
     // semaphore to its created capacity)
     if (hs_arena_reset(a, s) != HS_OK) return HS_ERR_HIP;
+    if (st == 0) return HS_OK;  // a reset covered it
     return st == hs::kErrAborted ? HS_ERR_ABORTED : HS_ERR_TIMEOUT;
   }
   return HS_OK;

@@ -227,6 +227,8 @@ __device__ __forceinline__ double block_sum_f64(double v) {
 __device__ __forceinline__ ArenaView budget_view(const ServeArgs &p) {
   ArenaView v{};
   v.status = &p.st->aborted;
+  v.abort_flag = p.st->p6;  // zero: no host flag of its own, and nobody reads kHostStatus
+  static_assert(kHostStatus < sizeof(p.st->p6) / sizeof(uint32_t), "the word that a failure sets");
   v.spin_limit = p.spin_limit;
   return v;
 }
