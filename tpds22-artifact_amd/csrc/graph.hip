@@ -2039,7 +2039,8 @@ __device__ __forceinline__ void sssp_step(const SsspArgs &p, SsState &st, const 
 }
 
 template <int KIND>
-__global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4))) k_sssp(ArenaView a, SsspArgs p) {
+__global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(KIND == HS_BAR_COOP ? 8 : 4)))  // (COOP: no team)
+k_sssp(ArenaView a, SsspArgs p) {
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;

@@ -80,7 +80,7 @@ __device__ __forceinline__ void st_word(uint64_t *p, uint64_t v) {
 // Workgroup w's tile of round r is [(r W + w) TILE, +TILE), a wave's part of it SEGS
 // segments.  words[2][W]: (round + 1) << 32 | the workgroup's sum, by round parity.
 template <int KIND, int SEGS, bool INCLUSIVE>
-__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(kWg) __attribute__((amdgpu_waves_per_eu(SEGS > 8 ? 4 : 8)))
 k_scan_u32(ArenaView a, const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *words, uint32_t ngroups, uint32_t nxcd) {
   constexpr uint32_t kPart = SEGS * kSpan, kTile = kWaves * kPart;
   __shared__ uint32_t s_wave[kWaves], s_carry[kWaves], s_before[kWaves];
