@@ -15,6 +15,18 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP kernels)")
 
 
+# Files whose tests have to come before the others of the process, whatever they are
+# called: cooperative launches of this process can make those of the command-line
+# programs, run as its children, fail; and a launch whose stream shares one of HIP's four
+# hardware queues with a running serving loop waits for the loop, so loops run while the
+# process has few streams.
+FIRST = ["test_gpu_cli.py", "test_gpu_serve.py", "test_gpu_fullsize.py"]
+
+
+def pytest_collection_modifyitems(items):
+    items.sort(key=lambda i: FIRST.index(i.path.name) if i.path.name in FIRST else len(FIRST))
+
+
 @pytest.fixture(scope="session")
 def oracle():
     import oracle_lib
