@@ -151,6 +151,12 @@ int main(int argc, char **argv) {
       bad += team_usable(size, grid, true) != (size < grid && size <= 32);
       bad += team_edges(size) != size * team_edges(32) / 32;  // a small team takes its share
     }
+  // a stretch is shorter than the limit of the others' polls, one in 1.4 us, for rounds
+  // of a team of up to 500 us, and never empty
+  for (uint64_t limit = 1; limit < 1ull << 32; limit = limit * 3 / 2 + 1) {
+    const uint32_t rounds = team_rounds((uint32_t)limit);
+    bad += rounds < 1 || rounds > 256 || (rounds > 1 && rounds * 512ull > limit + 512);
+  }
   // a mesh of mean degree 3.4, counted as 4, 1000 levels of 1000 vertices: never pulled;
   // a power-law graph's wide levels: pulled, its first and last: not
   for (uint64_t level = 0; level < 1000; ++level) bad += pull_pays(4000, 4000 * level, 3400000, 1000000);

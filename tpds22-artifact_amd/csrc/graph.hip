@@ -978,8 +978,8 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 // Correctness does not depend on the placement: everything the rounds write is
 // written and read with agent-scope operations, and every wave's stores have
 // completed before its workgroup arrives.  Nor on timing: the other workgroups wait
-// in the grid barrier meanwhile (a stretch is at most kTeamRounds rounds, so that
-// wait stays short), and what they read before it, to find out that this stretch is
+// in the grid barrier meanwhile (a stretch is at most 256 rounds, so that wait stays
+// short), and what they read before it, to find out that this stretch is
 // not theirs, is not written until it is over (team_rounds.hpp: the counters of the
 // phase and the report of the stretch before; the team counts in others).
 // Threads per workgroup of the kernels that run team rounds: with 128 registers and
@@ -992,7 +992,6 @@ __global__ void __launch_bounds__(kWg) k_msbfs(ArenaView a, MsArgs p) {
 // searches at once, spill: 392 us, 3.34 ms and 24.6 ms.
 constexpr int kTeamWg = 512;
 using hs_rounds::kTeamMax;                  // workgroups of a team
-constexpr uint32_t kTeamRounds = 256;
 constexpr uint32_t kTeamIdleSleep = 32;     // s_sleep units between the idle workgroups' polls
 constexpr uint32_t kSegCap = 2048;          // entries of a workgroup's output segment; the rest goes to the queue
 constexpr uint32_t kSegBlock = 16;          // entries a wave takes at once: 4 lanes each
@@ -1077,10 +1076,11 @@ struct Team {
   uint64_t *word;       // [2][kTeamMax] episode << 32 | segment word, zero before the first grid barrier
   uint32_t size, rank;  // rank: position in the team (workgroups outside it: any value)
   bool in, usable;
-  uint64_t most;  // edges of a round that the team runs
+  uint64_t most;    // edges of a round that the team runs
+  uint32_t rounds;  // of a stretch
   uint32_t episode;
 
-  __device__ void init(uint64_t *w, uint32_t nxcd, bool bounded) {
+  __device__ void init(const ArenaView &a, uint64_t *w, uint32_t nxcd, bool bounded) {
     const uint32_t x = nxcd < gridDim.x ? nxcd : gridDim.x;
     word = w;
     size = (gridDim.x + x - 1) / x;
@@ -1088,6 +1088,7 @@ struct Team {
     in = blockIdx.x % x == 0;
     usable = hs_rounds::team_usable(size, gridDim.x, bounded);
     most = hs_rounds::team_edges(size);
+    rounds = hs_rounds::team_rounds(a.spin_limit);
     episode = 0;
   }
   // Barrier of the team; `mine` (thread 0): this workgroup's segment word, `seg`:
@@ -1655,7 +1656,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;
-  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
+  team.init(a, reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
   __shared__ Output out;
   __shared__ WaveBuffers wb;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
@@ -1706,7 +1707,7 @@ __global__ void __launch_bounds__(kTeamWg) __attribute__((amdgpu_waves_per_eu(4)
     } else if (team.in) {
       if (threadIdx.x == 0) { out.clear(0); out.clear(1); }
       __syncthreads();
-      for (uint32_t q = 0; q < kTeamRounds; ++q) {
+      for (uint32_t q = 0; q < team.rounds; ++q) {
         const uint32_t par = r & 1;
         if (threadIdx.x == 0) out.clear(par ^ 1);
         if (t0 == 0) round.open();
@@ -2044,7 +2045,7 @@ k_sssp(ArenaView a, SsspArgs p) {
   GridBarrier gb;
   gb.init(a, KIND, p.ng, p.nx);
   Team team;
-  team.init(reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
+  team.init(a, reinterpret_cast<uint64_t *>(p.ctr + hs_rounds::kTeamWords * kCtr), p.nx, KIND != HS_BAR_COOP);
   __shared__ Output out;
   __shared__ SsLists lists;
   const uint32_t t0 = blockIdx.x * kTeamWg + threadIdx.x, nt = gridDim.x * kTeamWg;
@@ -2093,7 +2094,7 @@ k_sssp(ArenaView a, SsspArgs p) {
     } else if (team.in) {
       if (threadIdx.x == 0) { out.clear(0); out.clear(1); lists.kept.clear(); }
       __syncthreads();
-      for (uint32_t k = 0; k < kTeamRounds; ++k) {
+      for (uint32_t k = 0; k < team.rounds; ++k) {
         const uint32_t par = st.r & 1;
         sssp_step<true>(p, st, round, in, few, t0 == 0, &out, team.rank, &lists);
         ++round.i;

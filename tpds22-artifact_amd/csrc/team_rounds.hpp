@@ -74,6 +74,14 @@ HS_ROUND_FN bool pull_pays(uint64_t ahead, uint64_t behind, uint64_t m, uint64_t
   return ahead * 8 > (m > behind ? m - behind : 0) && ahead * 16 > n;
 }
 
+// Rounds of a stretch, at most: the others poll once in 1.4 us meanwhile, and as many
+// times as the arena's spin limit allows, so that small limits, under which every round
+// of the grid succeeds, get short stretches (a round of a team takes 2-6 us on meshes
+// and up to some 50).
+HS_ROUND_FN uint32_t team_rounds(uint32_t spin_limit) {
+  return spin_limit / 512 < 255 ? spin_limit / 512 + 1 : 256;
+}
+
 // the counters that round i of a side clears for the rounds after it
 template <class Clear>
 HS_ROUND_FN void open_round(Side side, uint32_t i, Clear clear) {
