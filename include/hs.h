@@ -230,7 +230,8 @@ int hs_scan_get_round_bytes(uint64_t *bytes_out);
    [offsets[s], offsets[s+1]) of d_in; offsets are given on the device (d_offsets)
    and the host (h_offsets, used to size the launch).  The segments are cut into
    tiles as one array (a tile may hold many of them), taken in order from one
-   counter (work stealing); the scan passes carries by a decoupled look-back.  d_work: hs_batch_work_size bytes.  nseg <= 65536. */
+   counter (work stealing); the scan passes carries by a decoupled look-back.
+   d_work: hs_batch_work_size bytes.  nseg <= 65536. */
 int hs_batch_work_size(const uint64_t *h_offsets, uint32_t nseg, uint64_t *bytes_out);
 int hs_scan_batch_u32(const uint32_t *d_in, uint32_t *d_out, const uint64_t *d_offsets,
                       const uint64_t *h_offsets, uint32_t nseg, int inclusive, void *d_work,

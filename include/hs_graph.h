@@ -17,6 +17,13 @@
 extern "C" {
 #endif
 
+/* Grids of the launches below: num_wgs workgroups, or (num_wgs <= 0) a default.
+   hs_bfs, hs_bfs_dir and hs_sssp run at most one workgroup per CU.  A default launch
+   of these and of hs_pagerank_f32 takes at most half of each CU, so that two of them
+   on two streams, with an arena each, are resident together; hs_msbfs and hs_mssp
+   take whole CUs.  Launches that do not fit together may wait for each other until
+   the arenas' spin limit. */
+
 /* single-source BFS: replaces gg_main + gg_main_pipe_1_gpu_gb
    (LONESTAR/apps/bfs/kernel_gsrb.cu:591-730).  d_level[v] = hops from src,
    INT32_MAX when unreached.  d_stats (device, >= 4 u32, may be NULL) receives

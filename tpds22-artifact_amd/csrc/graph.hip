@@ -1162,7 +1162,7 @@ __device__ __forceinline__ bool team_push_chunks(uint64_t *hq, uint32_t *hcnt, c
 
 // A wave's appends to one queue, staged in LDS: every atomic on a queue's counter
 // serializes for ~11 ns over the whole device, and with one per batch of 256 edges
-// those atomics were most of a large round (R-MAT 22, one source: 7.7 -> 2.9 ms).
+// those atomics were most of a large round (R-MAT 22, one source: 7.7 -> 2.9 ms then).
 // The count is the same in every lane.
 template <class T, uint32_t CAP>
 struct WaveList {
@@ -1353,8 +1353,9 @@ __device__ __forceinline__ uint32_t queue_share(uint32_t nin, uint32_t waves) {
 // "Direction-optimizing breadth-first search", 2012): the vertices not yet reached
 // look for an in-neighbour in the frontier's bitmap (512 KiB at R-MAT 22, kept in
 // L2) and stop at the first; no atomics, and the new bitmap is written a word per
-// wave.  R-MAT 22: 0.96 ms pushed only (2.0 ms with one queue atomic per 512
-// edges), 0.37 ms; a mesh of 720k vertices 15.9 -> 4.0 ms with the team.
+// wave.  R-MAT 22: 1.02 ms pushed only (1.9 ms with one queue atomic per 512
+// edges), 0.36 ms; a mesh of 720k vertices 13-16 -> 4.0-5.7 ms with the team, by the
+// card.
 struct BfsArgs1 {
   uint32_t n, m;
   const uint32_t *row, *col, *rrow, *rcol;  // rrow, rcol null: push only
