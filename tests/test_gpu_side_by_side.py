@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 
 class Work:
     """One kind of launch with its inputs and buffers: enqueue() on a stream, check()."""
+    wgs = 0  # of a search: the default grid
 
     def __init__(self, hs, name):
         import torch
@@ -42,9 +43,9 @@ class Work:
         import hsync.graph as G
         with torch.cuda.stream(stream):  # a call's own tensors belong to its stream
             if self.name == "bfs":
-                G.bfs(self.arena, self.g, self.src, level=self.out, work=self.work, sync=False)
+                G.bfs(self.arena, self.g, self.src, num_wgs=self.wgs, level=self.out, work=self.work, sync=False)
             elif self.name == "sssp":
-                G.sssp(self.arena, self.g, self.src, dist=self.out, work=self.work, sync=False)
+                G.sssp(self.arena, self.g, self.src, num_wgs=self.wgs, dist=self.out, work=self.work, sync=False)
             elif self.name == "pagerank":
                 G.pagerank(self.arena, self.g, rank=self.out, work=self.work, sync=False)
             elif self.name == "batch":
@@ -85,6 +86,26 @@ def test_on_two_streams(hs, oracle, a, b):
     jobs = [Work(hs, a), Work(hs, b)]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     try:
+        for _ in range(10):
+            for j, s in zip(jobs, streams):
+                j.enqueue(s)
+        for j, s in zip(jobs, streams):
+            j.check(s, oracle)
+    finally:
+        for s in streams:
+            s.synchronize()
+        for j in jobs:
+            j.close()
+
+
+@pytest.mark.parametrize("names", [("bfs",) * 4, ("sssp",) * 4, ("bfs", "sssp", "bfs", "sssp")])
+def test_four_searches_on_half_of_the_cus_each(hs, oracle, names):
+    import torch
+    jobs = [Work(hs, n) for n in names]
+    streams = [torch.cuda.Stream() for _ in names]
+    try:
+        for j in jobs:
+            j.wgs = hs.device_info()["num_cus"] // 2
         for _ in range(10):
             for j, s in zip(jobs, streams):
                 j.enqueue(s)
